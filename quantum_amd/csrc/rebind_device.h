@@ -76,7 +76,7 @@ struct RebindArgs {
   int tfq_fd;                // derivative matrices: TFQ's float32 central difference
 };
 
-// One thread per (row, op); kmax is the widest recipe op (1..4).
+// kmax is the widest recipe op (1..4).
 hipError_t LaunchRebind(const RebindArgs& a, int kmax, hipStream_t stream);
 
 }  // namespace tfqx

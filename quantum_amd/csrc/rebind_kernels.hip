@@ -7,7 +7,25 @@
 // BlockMatrix, ParamBlockMatrices, Embed, WriteMatrix, RebindRow), with the
 // same operations in the same order.  Contraction is off so every double
 // product and sum is rounded on its own, as in the host build.
+//
+// Sixteen lanes work on one op, four ops per wavefront.  What bounds the
+// kernel is latency, of memory and of instruction fetch: a call has few ops
+// (hundreds to some ten thousand), and each is a chain of loads, a sine and
+// cosine per gate, and a product of the gates.  So the lanes take the chain's
+// independent parts: first every gate (and every +-eps evaluation of a gradient
+// gate) is one lane's, which computes its phases; then every matrix entry is one
+// lane's; then every column of the op's product and of its derivative products
+// is one lane's, which runs the gates in order.  All gate kinds share one
+// sine/cosine site and one entry routine, so the code stays small.
+//
+// One lane per op (the former layout, with each kind unrolled: 325 KB of code
+// fetched anew by each launch) took 137 us on 64 circuits of 10 qubits and 600
+// symbols, 107 us on one 12-qubit ansatz of 144 symbols and 659 us on 2048 uneven
+// circuits; this one takes 47, 12 and 312 us.  Six gates at a time keep the working
+// set at 3.4 KB per op, so eleven wavefronts share a CU (twelve gates, seven
+// wavefronts: 59, 13 and 428 us).
 #include "rebind_device.h"
+#include "tfqx_internal.h"
 
 #pragma clang fp contract(off)
 
@@ -17,6 +35,11 @@ namespace {
 constexpr double kPi = 3.14159265358979323846;
 constexpr float kGradEps = 5e-3f;  // adj_util.cc:32
 constexpr int kRbThreads = 64;
+constexpr int kGroup = 16;                        // lanes per op
+constexpr int kGroups = kRbThreads / kGroup;      // ops per workgroup (one wavefront)
+constexpr int kChunk = 6;                         // gates evaluated at a time
+constexpr int kSlots = kChunk + 2 * kMaxDeriv;    // ... and the +-eps evaluations of two derivatives
+static_assert(kSlots <= kGroup, "a lane per evaluation");
 
 struct dc {
   double re, im;
@@ -25,459 +48,317 @@ struct dc {
 __device__ inline dc Mul(dc a, dc b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
 __device__ inline dc Scale(dc a, double s) { return {a.re * s, a.im * s}; }
 __device__ inline dc Add(dc a, dc b) { return {a.re + b.re, a.im + b.im}; }
-__device__ inline dc Expi(double y) { return {cos(y), sin(y)}; }  // e^{iy}
 __device__ inline double Mul32(float a, float b) { return double(a * b); }
 
-__device__ inline int Targets(int kind) {
-  return (kind == 0 || (kind >= 2 && kind <= 5) || kind == 13) ? 1 : 2;
-}
-
-// U(t, gs) = sum_k e^{i pi t (lam_k + gs)} P_k, or dU/dt (deriv); DIM is the
-// gate's matrix dimension (2 or 4), fixed so U stays in registers.
-template <int DIM>
-__device__ void EigenEvalT(const RbEigen& e, double t, double gs, bool deriv, dc* U) {
-#pragma unroll
-  for (int i = 0; i < DIM * DIM; ++i) U[i] = {0.0, 0.0};
-  const int count = int(e.count);
-  for (int k = 0; k < count; ++k) {
-    const double ph = kPi * t * (e.lam[k] + gs);
-    dc w = Expi(ph);
-    if (deriv) w = Mul(w, dc{0.0, kPi * (e.lam[k] + gs)});
-#pragma unroll
-    for (int i = 0; i < DIM * DIM; ++i)
-      U[i] = Add(U[i], Mul(w, dc{e.P[k][2 * i], e.P[k][2 * i + 1]}));
-  }
-}
-
-__device__ inline void EigenEval(const RbEigen* table, int kind, double t, double gs, bool deriv,
-                                 dc* U) {
-  if (Targets(kind) == 1)
-    EigenEvalT<2>(table[kind], t, gs, deriv, U);
-  else
-    EigenEvalT<4>(table[kind], t, gs, deriv, U);
-}
-
-// pidx < 0: the gate's unitary; otherwise its exact derivative wrt p[pidx].
-__device__ void UnitaryOrDeriv(const RbEigen* table, int kind, const float* p, int pidx, dc* U) {
-  const dc negI{-0.0, -1.0};
-  if (kind == 0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) U[i] = (pidx < 0 && i % 3 == 0) ? dc{1.0, 0.0} : dc{0.0, 0.0};
-    return;
-  }
-  if (kind == 1) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) U[i] = (pidx < 0 && i % 5 == 0) ? dc{1.0, 0.0} : dc{0.0, 0.0};
-    return;
-  }
-  if (kind >= 2 && kind <= 12) {
-    const double t = Mul32(p[0], p[1]);
-    EigenEval(table, kind, t, double(p[2]), pidx >= 0, U);
-    if (pidx >= 0) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) U[i] = Scale(U[i], double(p[1]));
-    }
-    return;
-  }
-  if (kind == 13) {  // PhasedX
-    const double ph = Mul32(p[0], p[1]);
-    const double t = Mul32(p[2], p[3]);
-    dc X[4];
-    EigenEval(table, 3, t, double(p[4]), pidx == 2, X);
-    const dc em = Expi(-kPi * ph), ep = Expi(kPi * ph);
-    U[0] = X[0];
-    U[1] = Mul(X[1], em);
-    U[2] = Mul(X[2], ep);
-    U[3] = X[3];
-    if (pidx == 0) {
-      U[0] = {0.0, 0.0};
-      U[3] = {0.0, 0.0};
-      U[1] = Mul(U[1], Scale(dc{0.0, -kPi}, double(p[1])));
-      U[2] = Mul(U[2], Scale(dc{0.0, kPi}, double(p[1])));
-    } else if (pidx == 2) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) U[i] = Scale(U[i], double(p[3]));
-    }
-    return;
-  }
-  if (kind == 14) {  // FSim
-    const double th = Mul32(p[0], p[1]);
-    const double phi = Mul32(p[2], p[3]);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) U[i] = {0.0, 0.0};
-    const double c = cos(th), s = sin(th);
-    if (pidx < 0) {
-      U[0] = {1.0, 0.0};
-      U[5] = {c, 0.0};
-      U[6] = Scale(negI, s);
-      U[9] = Scale(negI, s);
-      U[10] = {c, 0.0};
-      U[15] = Expi(-phi);
-    } else if (pidx == 0) {
-      const double sc = p[1];
-      U[5] = {-s * sc, 0.0};
-      U[6] = Scale(Scale(negI, c), sc);
-      U[9] = Scale(Scale(negI, c), sc);
-      U[10] = {-s * sc, 0.0};
-    } else {
-      U[15] = Scale(Mul(negI, Expi(-phi)), double(p[3]));
-    }
-    return;
-  }
-  // kind 15: PhasedISwap
-  const double ph = Mul32(p[0], p[1]);
-  const double t = Mul32(p[2], p[3]);
-  EigenEval(table, 12, t, 0.0, pidx == 2, U);
-  const dc ep = Expi(2 * kPi * ph), em = Expi(-2 * kPi * ph);
-  U[6] = Mul(U[6], ep);
-  U[9] = Mul(U[9], em);
-  if (pidx == 0) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (i != 6 && i != 9) U[i] = {0.0, 0.0};
-    U[6] = Mul(U[6], Scale(dc{0.0, 2 * kPi}, double(p[1])));
-    U[9] = Mul(U[9], Scale(dc{0.0, -2 * kPi}, double(p[1])));
-  } else if (pidx == 2) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) U[i] = Scale(U[i], double(p[3]));
-  }
-}
-
-// TFQ's gradient gates (adj_util.cc:175-302) or the exact derivative.  The
-// central difference keeps float(U(p + eps)) while U(p - eps) is evaluated
-// into dU, then combines them in float as the host does.
-__device__ void GateDerivative(const RbEigen* table, int kind, const float* params, int pidx,
-                               bool tfq_fd, dc* dU) {
-  if (!tfq_fd) {
-    UnitaryOrDeriv(table, kind, params, pidx, dU);
-    return;
-  }
-  float pp[5];
-#pragma unroll
-  for (int i = 0; i < 5; ++i) pp[i] = i == pidx ? params[i] + kGradEps : params[i];
-  UnitaryOrDeriv(table, kind, pp, -1, dU);
-  float fr[16], fi[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    fr[i] = float(dU[i].re);
-    fi[i] = float(dU[i].im);
-  }
-#pragma unroll
-  for (int i = 0; i < 5; ++i) pp[i] = i == pidx ? params[i] - kGradEps : params[i];
-  UnitaryOrDeriv(table, kind, pp, -1, dU);
-  const float scale = float(0.5 / double(kGradEps));
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const float re = fr[i] - float(dU[i].re);
-    const float im = fi[i] - float(dU[i].im);
-    dU[i] = {double(re * scale), double(im * scale)};
-  }
-}
-
-struct LGate {
-  int kind, nt;
-  int bits[2];
-  uint64_t cmask, cval;
-  float params[5];
-  int sym_pidx[2];
+// One evaluated gate of a chunk.  pidx < 0: the unitary; otherwise the exact
+// derivative with respect to argument pidx, whose scale is sc.
+struct Slot {
+  dc w[4];       // the gate's phases (see Phases)
+  double sc;
+  int kind, pidx;
+  int nt;        // targets
+  int pos;       // block position of target 0 | of target 1 << 8
+  int cm, cv;    // controls inside the block
+};
+// Per-op working set in LDS.
+struct Work {
+  Slot slot[kSlots];
+  dc U[kSlots][16];
 };
 
-// The gate's arguments with the row's symbol values substituted.
-__device__ void LoadGate(const RbGate& src, const float* v, LGate* g) {
-  g->kind = src.kind;
-  g->nt = src.nt;
-  g->bits[0] = src.bits[0];
-  g->bits[1] = src.bits[1];
-  g->cmask = src.cmask;
-  g->cval = src.cval;
-  for (int j = 0; j < 2; ++j) g->sym_pidx[j] = src.sym_pidx[j];
-  const float v0 = src.nsym > 0 ? v[src.sym_col[0]] : 0.0f;
-  const float v1 = src.nsym > 1 ? v[src.sym_col[1]] : 0.0f;
-#pragma unroll
-  for (int j = 0; j < 5; ++j)
-    g->params[j] = (src.nsym > 1 && src.sym_pidx[1] == j) ? v1
-                 : (src.nsym > 0 && src.sym_pidx[0] == j) ? v0 : src.params[j];
+// LDS traffic of one wavefront is in order; this keeps the compiler's order too.
+__device__ inline void WaveSync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// acc <- (gate U embedded over `bits`) * acc; acc is dim x dim, (re, im) interleaved.
-__device__ void ApplyLeft(int nt, const int* gbits, uint64_t cmask, uint64_t cval, const dc* U,
-                          const int* bits, int k, double* acc) {
-  const int dim = 1 << k;
-  int upos[2] = {0, 0};
-  for (int j = 0; j < nt; ++j)
-    for (int m = 0; m < k; ++m)
-      if (bits[m] == gbits[j]) upos[j] = m;
-  int cm = 0, cv = 0;
-  for (int m = 0; m < k; ++m)
-    if (cmask >> bits[m] & 1) {
+// The phases e^{iy} a gate's entries are made of, for arguments p:
+//   eigen gates   w[k] = e^{i pi t (lam_k + gs)} (times i pi (lam_k + gs): derivative)
+//   PhasedX       those of X, w[2] = e^{-i pi phase}
+//   FSim          w[0] = e^{i theta}, w[1] = e^{-i phi}
+//   PhasedISwap   those of ISwap, w[3] = e^{2 i pi phase}
+__device__ void Phases(const RbEigen* table, int kind, const float* p, int pidx, Slot* s) {
+  const bool phased = kind == 13 || kind == 15;
+  const double a = Mul32(p[0], p[1]), b = Mul32(p[2], p[3]);
+  const double t = phased ? b : a;
+  const double gs = kind == 13 ? double(p[4]) : kind == 15 ? 0.0 : double(p[2]);
+  const bool deriv = phased ? pidx == 2 : pidx >= 0;
+  const RbEigen& e = table[kind == 13 ? 3 : kind == 15 ? 12 : kind == 14 ? 0 : kind];
+  const int count = kind == 14 ? 2 : kind < 2 ? 0 : int(e.count);
+#pragma unroll 1
+  for (int k = 0; k < 4; ++k) {
+    double y;
+    if (kind == 14) y = k == 0 ? a : -b;
+    else if (k < count) y = kPi * t * (e.lam[k] + gs);
+    else if (kind == 13 && k == 2) y = -kPi * a;
+    else if (kind == 15 && k == 3) y = 2 * kPi * a;
+    else continue;
+    if (kind == 14 && k >= count) continue;
+    dc w;
+    sincos(y, &w.im, &w.re);
+    if (deriv && kind != 14 && k < count) w = Mul(w, dc{0.0, kPi * (e.lam[k] + gs)});
+    s->w[k] = w;
+  }
+  s->sc = double((phased || kind == 14) && pidx == 2 ? p[3] : p[1]);
+}
+
+// Entry i (row-major) of the slot's matrix.
+__device__ dc Entry(const RbEigen* table, const Slot& s, int i) {
+  const dc zero{0.0, 0.0}, negI{-0.0, -1.0};
+  const int kind = s.kind, pidx = s.pidx;
+  if (kind < 2) return pidx < 0 && i % (kind == 0 ? 3 : 5) == 0 ? dc{1.0, 0.0} : zero;
+  if (kind == 14) {
+    const double c = s.w[0].re, sn = s.w[0].im;
+    const bool diag = i == 5 || i == 10, off = i == 6 || i == 9;
+    if (pidx < 0)
+      return i == 0 ? dc{1.0, 0.0} : diag ? dc{c, 0.0} : off ? Scale(negI, sn) : i == 15 ? s.w[1] : zero;
+    if (pidx == 0)
+      return diag ? dc{-sn * s.sc, 0.0} : off ? Scale(Scale(negI, c), s.sc) : zero;
+    return i == 15 ? Scale(Mul(negI, s.w[1]), s.sc) : zero;
+  }
+  const RbEigen& e = table[kind == 13 ? 3 : kind == 15 ? 12 : kind];
+  dc u = zero;
+  const int count = int(e.count);
+  dc P[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) P[k] = dc{e.P[k][2 * i], e.P[k][2 * i + 1]};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const dc x = Add(u, Mul(s.w[k], P[k]));
+    if (k < count) u = x;
+  }
+  if (kind <= 12) return pidx >= 0 ? Scale(u, s.sc) : u;
+  // PhasedX / PhasedISwap: the off-diagonal pair gains opposite phases.
+  const int lo = kind == 13 ? 1 : 6, hi = kind == 13 ? 2 : 9;
+  if (i == lo || i == hi) {
+    // PhasedX: e^{-i pi phase} above the diagonal; PhasedISwap: e^{2 i pi phase}.
+    dc ph = s.w[kind == 13 ? 2 : 3];
+    if (i == hi) ph.im = -ph.im;
+    u = Mul(u, ph);
+    if (pidx == 0) {
+      const double f = kind == 13 ? (i == lo ? -kPi : kPi) : (i == lo ? 2 * kPi : -2 * kPi);
+      u = Mul(u, Scale(dc{0.0, f}, s.sc));
+    }
+  } else if (pidx == 0) {
+    u = zero;
+  }
+  return pidx == 2 ? Scale(u, s.sc) : u;
+}
+
+// Evaluate gate `src` for the row's values v into slot s: its unitary (delta =
+// 0, pidx < 0), the unitary with argument pidx shifted by delta, or (delta = 0)
+// the exact derivative.  bits: the op's K qubits.
+__device__ void EvalGate(const RebindArgs& a, const RbGate& src, const float* v, int pidx,
+                         float delta, const int* bits, int k, bool controls, Slot* s) {
+  const int nsym = src.nsym;
+  const float v0 = nsym > 0 ? v[src.sym_col[0]] : 0.0f;
+  const float v1 = nsym > 1 ? v[src.sym_col[1]] : 0.0f;
+  float p[5];
+#pragma unroll
+  for (int j = 0; j < 5; ++j) {
+    p[j] = (nsym > 1 && src.sym_pidx[1] == j) ? v1
+         : (nsym > 0 && src.sym_pidx[0] == j) ? v0 : src.params[j];
+    if (delta != 0.0f && j == pidx) p[j] += delta;
+  }
+  s->kind = src.kind;
+  s->pidx = delta != 0.0f ? -1 : pidx;
+  s->nt = src.nt;
+  int pos = 0, cm = 0, cv = 0;
+  for (int m = 0; m < k; ++m) {
+    if (bits[m] == src.bits[0]) pos |= m;
+    if (src.nt > 1 && bits[m] == src.bits[1]) pos |= m << 8;
+    if (controls && (src.cmask >> bits[m] & 1)) {
       cm |= 1 << m;
-      if (cval >> bits[m] & 1) cv |= 1 << m;
+      if (src.cval >> bits[m] & 1) cv |= 1 << m;
     }
-  const int udim = 1 << nt;
-  int gmask = 0;
-  for (int j = 0; j < nt; ++j) gmask |= 1 << upos[j];
-  int rows[4];
-  for (int r0 = 0; r0 < dim; ++r0) {
-    if (r0 & gmask) continue;
-    if ((r0 & cm) != cv) continue;
-    for (int sidx = 0; sidx < udim; ++sidx) {
-      int r = r0;
-      for (int j = 0; j < nt; ++j)
-        if (sidx >> (nt - 1 - j) & 1) r |= 1 << upos[j];
-      rows[sidx] = r;
-    }
-    for (int c = 0; c < dim; ++c) {
-      double vr[4], vi[4];
-      for (int sidx = 0; sidx < udim; ++sidx) {
-        vr[sidx] = acc[2 * (rows[sidx] * dim + c)];
-        vi[sidx] = acc[2 * (rows[sidx] * dim + c) + 1];
-      }
-      for (int e = 0; e < udim; ++e) {
-        double sr = 0, si = 0;
-        for (int b = 0; b < udim; ++b) {
-          const double xr = U[e * udim + b].re, xi = U[e * udim + b].im;
-          sr += xr * vr[b] - xi * vi[b];
-          si += xr * vi[b] + xi * vr[b];
+  }
+  s->pos = pos;
+  s->cm = cm;
+  s->cv = cv;
+  Phases(a.eigen, src.kind, p, s->pidx, s);
+}
+
+// TFQ's gradient gate (adj_util.cc:175-302) from the two shifted unitaries: the
+// float32 central difference, as the host combines them.
+__device__ inline dc FdEntry(dc up, dc um) {
+  const float scale = float(0.5 / double(kGradEps));
+  const float re = float(up.re) - float(um.re), im = float(up.im) - float(um.im);
+  return {double(re * scale), double(im * scale)};
+}
+
+// One column of the block product: v <- (gate embedded in the block) v.  The
+// column's 2^K entries are in registers for K <= 2.  D: the derivative's slots
+// instead of the gate's unitary (fd: two shifted unitaries to combine).
+__device__ inline dc MatEntry(const Work& wk, int t, int d, bool fd, int i) {
+  if (d < 0) return wk.U[t][i];
+  const dc up = wk.U[kChunk + 2 * d][i];
+  return fd ? FdEntry(up, wk.U[kChunk + 2 * d + 1][i]) : up;
+}
+
+template <int DIM>
+__device__ void ApplyColumn(const Work& wk, int t, int d, bool fd, dc* v) {
+  const Slot& s = wk.slot[t];
+  const int p0 = s.pos & 255, p1 = s.pos >> 8, cm = s.cm, cv = s.cv;
+  if (s.nt == 1) {
+    dc u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = MatEntry(wk, t, d, fd, i);
+    if constexpr (DIM <= 4) {
+#pragma unroll
+      for (int b = 0; b < (DIM > 2 ? 2 : 1); ++b) {
+        if (b != p0) continue;
+#pragma unroll
+        for (int r0 = 0; r0 < DIM; ++r0) {
+          if (r0 & (1 << b)) continue;
+          if ((r0 & cm) != cv) continue;
+          const dc x = v[r0], y = v[r0 | (1 << b)];
+          v[r0] = Add(Add(dc{0.0, 0.0}, Mul(u[0], x)), Mul(u[1], y));
+          v[r0 | (1 << b)] = Add(Add(dc{0.0, 0.0}, Mul(u[2], x)), Mul(u[3], y));
         }
-        acc[2 * (rows[e] * dim + c)] = sr;
-        acc[2 * (rows[e] * dim + c) + 1] = si;
       }
-    }
-  }
-}
-
-__device__ void Identity(double* acc, int dim) {
-  for (int i = 0; i < 2 * dim * dim; ++i) acc[i] = 0;
-  for (int i = 0; i < dim; ++i) acc[2 * (i * dim + i)] = 1.0;
-}
-
-__device__ void Write(float2* dst, const double* acc, bool diag_only, int dim) {
-  if (diag_only) {
-    for (int i = 0; i < dim; ++i)
-      dst[i] = make_float2(float(acc[2 * (i * dim + i)]), float(acc[2 * (i * dim + i) + 1]));
-  } else {
-    for (int i = 0; i < dim * dim; ++i) dst[i] = make_float2(float(acc[2 * i]), float(acc[2 * i + 1]));
-  }
-}
-
-// Single gate over the op's qubits (no controls inside): out = 0 + U placed.
-__device__ void Embed(const dc* U, const int* ubits, int uk, const int* obits, int ok, double* out) {
-  const int dim = 1 << ok;
-  for (int i = 0; i < 2 * dim * dim; ++i) out[i] = 0;
-  int upos[2] = {0, 0};
-  for (int j = 0; j < uk; ++j)
-    for (int m = 0; m < ok; ++m)
-      if (obits[m] == ubits[j]) upos[j] = m;
-  const int udim = 1 << uk;
-  for (int c = 0; c < dim; ++c) {
-    int sub = 0;
-    for (int j = 0; j < uk; ++j) sub |= ((c >> upos[j]) & 1) << (uk - 1 - j);
-    for (int r = 0; r < udim; ++r) {
-      int row = c;
-      for (int j = 0; j < uk; ++j) {
-        const int bit = (r >> (uk - 1 - j)) & 1;
-        row = (row & ~(1 << upos[j])) | (bit << upos[j]);
+    } else {
+      for (int r0 = 0; r0 < DIM; ++r0) {
+        if ((r0 >> p0) & 1 || (r0 & cm) != cv) continue;
+        const dc x = v[r0], y = v[r0 | (1 << p0)];
+        v[r0] = Add(Add(dc{0.0, 0.0}, Mul(u[0], x)), Mul(u[1], y));
+        v[r0 | (1 << p0)] = Add(Add(dc{0.0, 0.0}, Mul(u[2], x)), Mul(u[3], y));
       }
-      out[2 * (row * dim + c)] += U[r * udim + sub].re;
-      out[2 * (row * dim + c) + 1] += U[r * udim + sub].im;
-    }
-  }
-}
-
-// ---------------------------------------------------------------- ops of <= 2 qubits
-// The same recipes with every index fixed at compile time, so the block
-// matrix and the gate's matrix stay in registers.
-
-// ApplyLeft for a K-qubit block and an NT-qubit gate whose target j sits at
-// block position Pj (P0 holds the gate's matrix MSB); controls inside the
-// block (cm, cv) are runtime predicates.
-template <int K, int NT, int P0, int P1>
-__device__ void ApplyLeftT(const dc* U, int cm, int cv, double* acc) {
-  constexpr int dim = 1 << K, udim = 1 << NT;
-  constexpr int gmask = (1 << P0) | (NT == 2 ? (1 << P1) : 0);
-#pragma unroll
-  for (int r0 = 0; r0 < dim; ++r0) {
-    if (r0 & gmask) continue;
-    if ((r0 & cm) != cv) continue;
-    int rows[udim];
-#pragma unroll
-    for (int sidx = 0; sidx < udim; ++sidx) {
-      int r = r0;
-      if ((sidx >> (NT - 1)) & 1) r |= 1 << P0;
-      if (NT == 2 && (sidx & 1)) r |= 1 << P1;
-      rows[sidx] = r;
-    }
-#pragma unroll
-    for (int c = 0; c < dim; ++c) {
-      double vr[udim], vi[udim];
-#pragma unroll
-      for (int sidx = 0; sidx < udim; ++sidx) {
-        vr[sidx] = acc[2 * (rows[sidx] * dim + c)];
-        vi[sidx] = acc[2 * (rows[sidx] * dim + c) + 1];
-      }
-#pragma unroll
-      for (int e = 0; e < udim; ++e) {
-        double sr = 0, si = 0;
-#pragma unroll
-        for (int b = 0; b < udim; ++b) {
-          const double xr = U[e * udim + b].re, xi = U[e * udim + b].im;
-          sr += xr * vr[b] - xi * vi[b];
-          si += xr * vi[b] + xi * vr[b];
-        }
-        acc[2 * (rows[e] * dim + c)] = sr;
-        acc[2 * (rows[e] * dim + c) + 1] = si;
-      }
-    }
-  }
-}
-
-template <int K>
-__device__ void ApplyLeftK(const LGate& g, const dc* U, const int* bits, double* acc) {
-  int upos[2] = {0, 0};
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int m = 0; m < K; ++m)
-      if (j < g.nt && bits[m] == g.bits[j]) upos[j] = m;
-  int cm = 0, cv = 0;
-#pragma unroll
-  for (int m = 0; m < K; ++m)
-    if (g.cmask >> bits[m] & 1) {
-      cm |= 1 << m;
-      if (g.cval >> bits[m] & 1) cv |= 1 << m;
-    }
-  if (K == 1) {
-    ApplyLeftT<1, 1, 0, 0>(U, cm, cv, acc);
-  } else if (g.nt == 1) {
-    if (upos[0] == 0)
-      ApplyLeftT<K, 1, 0, 0>(U, cm, cv, acc);
-    else
-      ApplyLeftT<K, 1, (K > 1 ? 1 : 0), 0>(U, cm, cv, acc);
-  } else {
-    if (upos[0] == 0)
-      ApplyLeftT<K, 2, 0, (K > 1 ? 1 : 0)>(U, cm, cv, acc);
-    else
-      ApplyLeftT<K, 2, (K > 1 ? 1 : 0), 0>(U, cm, cv, acc);
-  }
-}
-
-template <int K>
-__device__ void IdentityK(double* acc) {
-  constexpr int dim = 1 << K;
-#pragma unroll
-  for (int i = 0; i < 2 * dim * dim; ++i) acc[i] = 0;
-#pragma unroll
-  for (int i = 0; i < dim; ++i) acc[2 * (i * dim + i)] = 1.0;
-}
-
-template <int K>
-__device__ void WriteK(float2* dst, const double* acc, bool diag_only) {
-  constexpr int dim = 1 << K;
-  if (diag_only) {
-#pragma unroll
-    for (int i = 0; i < dim; ++i)
-      dst[i] = make_float2(float(acc[2 * (i * dim + i)]), float(acc[2 * (i * dim + i) + 1]));
-  } else {
-#pragma unroll
-    for (int i = 0; i < dim * dim; ++i) dst[i] = make_float2(float(acc[2 * i]), float(acc[2 * i + 1]));
-  }
-}
-
-// One symbolic op of <= 2 qubits.  Kind 3's derivative products recompute the
-// running prefix up to their gate (the same operations the host's single
-// sweep performs before copying it), so each needs one accumulator only.
-// Kinds 1 and 2 place the gate by applying it to the identity: the entries
-// equal the host's Embed (x - 0*y and 0 + x are x).
-template <int K>
-__device__ void EvalOpK(const RebindArgs& a, const RbOp& op, const RbRow& row, const float* v,
-                        float2* mats) {
-  const int32_t* gl = a.gidx + row.gidx_base + op.gate_begin;
-  const int ng = op.gate_end - op.gate_begin;
-  double acc[2 * (1 << K) * (1 << K)];
-  dc U[16];
-  LGate g;
-  if (op.kind == 0 || op.kind == 3) {
-    // Pass 0 builds the block's matrix; pass s + 1 its derivative product s.
-    for (int pass = 0; pass <= (op.kind == 3 ? op.nderiv : 0); ++pass) {
-      const int dg = pass == 0 ? -1 : op.dgate[pass - 1];
-      IdentityK<K>(acc);
-      for (int t = 0; t < ng; ++t) {
-        LoadGate(a.gates[row.gate_base + gl[t]], v, &g);
-        if (t == dg)
-          GateDerivative(a.eigen, g.kind, g.params, g.sym_pidx[op.dsym[pass - 1]], a.tfq_fd != 0, U);
-        else
-          UnitaryOrDeriv(a.eigen, g.kind, g.params, -1, U);
-        ApplyLeftK<K>(g, U, op.bits, acc);
-      }
-      WriteK<K>(mats + (pass == 0 ? op.mat : op.dmat[pass - 1]), acc,
-                pass == 0 && op.kind == 0 && op.diag != 0);
     }
     return;
   }
-  LoadGate(a.gates[row.gate_base + gl[0]], v, &g);
-  g.cmask = g.cval = 0;  // recipes of kinds 1 and 2 keep controls outside the matrix
-  for (int pass = 0; pass <= op.nderiv; ++pass) {
-    if (pass == 0)
-      UnitaryOrDeriv(a.eigen, g.kind, g.params, -1, U);
-    else
-      GateDerivative(a.eigen, g.kind, g.params, g.sym_pidx[pass - 1], a.tfq_fd != 0, U);
-    IdentityK<K>(acc);
-    ApplyLeftK<K>(g, U, op.bits, acc);
-    WriteK<K>(mats + (pass == 0 ? op.mat : op.dmat[pass - 1]), acc, pass == 0 && op.diag != 0);
-  }
-}
-
-// ---------------------------------------------------------------- ops of 3-4 qubits
-template <int DIM>
-__device__ void EvalOpWide(const RebindArgs& a, const RbOp& op, const RbRow& row, const float* v,
-                           float2* mats) {
-  double acc[2 * DIM * DIM];
-  const int dim = 1 << op.k;
-  const int32_t* gl = a.gidx + row.gidx_base + op.gate_begin;
-  const int ng = op.gate_end - op.gate_begin;
-  LGate g;
-  dc U[16];
-  if (op.kind == 0) {
-    Identity(acc, dim);
-    for (int t = 0; t < ng; ++t) {
-      LoadGate(a.gates[row.gate_base + gl[t]], v, &g);
-      UnitaryOrDeriv(a.eigen, g.kind, g.params, -1, U);
-      ApplyLeft(g.nt, g.bits, g.cmask, g.cval, U, op.bits, op.k, acc);
+  if constexpr (DIM <= 4) {
+    // Both block qubits are targets (no room for a control).  Block index r is
+    // the gate's index with its two bits swapped when target 0 (the matrix's
+    // most significant bit) sits at position 0.
+    if constexpr (DIM == 4) {
+      const bool swap = p0 == 0;
+      dc x[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = v[r];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int e = swap ? ((r & 1) << 1 | r >> 1) : r;
+        // Summed in the gate's index order, as the host does.
+        dc sum{0.0, 0.0};
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int c = (b & 1) << 1 | b >> 1;
+          const dc xb = swap ? x[c] : x[b];
+          sum = Add(sum, Mul(MatEntry(wk, t, d, fd, e * 4 + b), xb));
+        }
+        v[r] = sum;
+      }
     }
-    Write(mats + op.mat, acc, op.diag != 0, dim);
-    return;
-  }
-  // Kinds 1 and 2 (kind 3 blocks have at most two qubits).
-  LoadGate(a.gates[row.gate_base + gl[0]], v, &g);
-  UnitaryOrDeriv(a.eigen, g.kind, g.params, -1, U);
-  Embed(U, g.bits, g.nt, op.bits, op.k, acc);
-  Write(mats + op.mat, acc, op.diag != 0, dim);
-  for (int d = 0; d < op.nderiv; ++d) {
-    dc dU[16];
-    GateDerivative(a.eigen, g.kind, g.params, g.sym_pidx[d], a.tfq_fd != 0, dU);
-    Embed(dU, g.bits, g.nt, op.bits, op.k, acc);
-    Write(mats + op.dmat[d], acc, false, dim);
+  } else {
+    const int gm = (1 << p0) | (1 << p1);
+    for (int r0 = 0; r0 < DIM; ++r0) {
+      if ((r0 & gm) || (r0 & cm) != cv) continue;
+      dc x[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) x[b] = v[r0 | ((b >> 1) << p0) | ((b & 1) << p1)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        dc sum{0.0, 0.0};
+#pragma unroll
+        for (int b = 0; b < 4; ++b) sum = Add(sum, Mul(MatEntry(wk, t, d, fd, e * 4 + b), x[b]));
+        v[r0 | ((e >> 1) << p0) | ((e & 1) << p1)] = sum;
+      }
+    }
   }
 }
 
-// One thread per (row, op): per-row tables list every row's ops (op.row
-// names the row); shared tables hold one program's ops for every row.
+// One op per kGroup lanes: per-row tables list every row's ops (op.row names the
+// row); shared tables hold one program's ops for every row.  DIM: 4 when every
+// op has at most two qubits (columns in registers), else 16 (columns in LDS;
+// such ops are fused blocks without derivatives, one column per lane).
 template <int DIM>
-__global__ __launch_bounds__(kRbThreads, 2) void rebind_kernel(RebindArgs a) {
-  const long long i = (long long)blockIdx.x * kRbThreads + threadIdx.x;
+__global__ __launch_bounds__(kRbThreads) void rebind_kernel(RebindArgs a) {
+  __shared__ Work work[kGroups];
+  __shared__ dc cols[DIM > 4 ? kRbThreads * DIM : 1];
+  const int g = int(threadIdx.x) / kGroup, lane = int(threadIdx.x) % kGroup;
+  const long long i = (long long)blockIdx.x * kGroups + g;
   const long long items = a.shared ? (long long)a.num_ops * a.num_rows : a.num_ops;
   if (i >= items) return;
-  const int oi = a.shared ? int(i % a.num_ops) : int(i);
-  const RbOp op = a.ops[oi];
-  const RbRow row = a.rows[a.shared ? int(i / a.num_ops) : op.row];
-  const float* v = a.values + size_t(row.vrow) * a.num_symbols;
+  Work& wk = work[g];
+  const RbOp& op = a.ops[a.shared ? int(i % a.num_ops) : int(i)];
+  const RbRow& row = a.rows[a.shared ? int(i / a.num_ops) : op.row];
+  const float* vals = a.values + size_t(row.vrow) * a.num_symbols;
   float2* mats = a.mats + row.mat_base;
-  if (op.k == 1)
-    EvalOpK<1>(a, op, row, v, mats);
-  else if (op.k == 2)
-    EvalOpK<2>(a, op, row, v, mats);
-  else if (DIM > 4)
-    EvalOpWide<DIM>(a, op, row, v, mats);
+  const int k = op.k, kind = op.kind, nd = op.nderiv, ng = op.gate_end - op.gate_begin;
+  const bool block = kind == 0 || kind == 3;  // else one gate, controls outside the matrix
+  const int npass = kind == 0 ? 1 : 1 + nd, ngates = block ? ng : 1;
+  const bool fd = a.tfq_fd != 0;
+  int bits[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) bits[m] = op.bits[m];
+  const int dim = 1 << k;
+  // This lane's column: of derivative product `pass - 1`, or of the op's matrix.
+  const int pass = DIM > 4 && dim > 4 ? 0 : lane >> 2;
+  const int col = DIM > 4 && dim > 4 ? lane : lane & 3;
+  const bool mine = pass < npass && col < dim;
+  const int dgate = pass > 0 && mine ? (block ? op.dgate[pass - 1] : 0) : -1;
+  dc reg[4];
+  dc* v = reg;
+  if constexpr (DIM > 4) v = cols + threadIdx.x * DIM;
+#pragma unroll
+  for (int r = 0; r < (DIM > 4 ? 16 : 4); ++r) v[r] = {r == col ? 1.0 : 0.0, 0.0};
+#pragma unroll 1
+  for (int t0 = 0; t0 < ngates; t0 += kChunk) {
+    const int nt = min(kChunk, ngates - t0);
+    // Phases: lane t a gate of the chunk, the last lanes the gradient gates in it.
+    int gate = -1, pidx = -1;
+    float delta = 0.0f;
+    if (lane < kChunk) {
+      if (lane < nt) gate = t0 + lane;
+    } else if (lane < kSlots) {
+      const int s = (lane - kChunk) >> 1, minus = (lane - kChunk) & 1;
+      if (s < npass - 1 && (fd || !minus)) {
+        const int dg = block ? op.dgate[s] : 0;
+        if (dg >= t0 && dg < t0 + nt) {
+          gate = dg;
+          delta = !fd ? 0.0f : minus ? -kGradEps : kGradEps;
+        }
+      }
+    }
+    if (gate >= 0) {
+      const RbGate& src = a.gates[row.gate_base + a.gidx[row.gidx_base + op.gate_begin + gate]];
+      if (lane >= kChunk) {
+        const int s = (lane - kChunk) >> 1;
+        pidx = src.sym_pidx[block ? op.dsym[s] : s];
+      }
+      EvalGate(a, src, vals, pidx, delta, bits, k, block, &wk.slot[lane]);
+    }
+    // Which slots hold a gate, for every lane of the group.
+    const unsigned long long live = __ballot(gate >= 0) >> (g * kGroup);
+    WaveSync();
+    // Four slots at a time, four entries of each (a two-qubit gate's 16 in four steps).
+#pragma unroll 1
+    for (int t4 = 0; t4 < kSlots; t4 += 4) {
+      const int t = t4 + (lane >> 2);
+      if (t >= kSlots || !((live >> t) & 1)) continue;
+      const int ne = wk.slot[t].nt == 1 ? 4 : 16;
+#pragma unroll 1
+      for (int e = lane & 3; e < ne; e += 4) wk.U[t][e] = Entry(a.eigen, wk.slot[t], e);
+    }
+    WaveSync();
+    if (mine)
+#pragma unroll 1
+      for (int t = 0; t < nt; ++t)
+        ApplyColumn<DIM>(wk, t, t0 + t == dgate ? pass - 1 : -1, fd, v);
+    WaveSync();
+  }
+  if (!mine) return;
+  float2* dst = mats + (pass == 0 ? op.mat : op.dmat[pass - 1]);
+  if (pass == 0 && kind != 3 && op.diag != 0) {
+#pragma unroll
+    for (int r = 0; r < DIM; ++r)
+      if (r == col) dst[r] = make_float2(float(v[r].re), float(v[r].im));
+  } else {
+#pragma unroll
+    for (int r = 0; r < DIM; ++r)
+      if (r < dim) dst[r * dim + col] = make_float2(float(v[r].re), float(v[r].im));
+  }
 }
 
 }  // namespace
@@ -485,11 +366,9 @@ __global__ __launch_bounds__(kRbThreads, 2) void rebind_kernel(RebindArgs a) {
 hipError_t LaunchRebind(const RebindArgs& a, int kmax, hipStream_t stream) {
   const long long items = a.shared ? (long long)a.num_ops * a.num_rows : a.num_ops;
   if (items <= 0) return hipSuccess;
-  const dim3 grid(unsigned((items + kRbThreads - 1) / kRbThreads)), block(kRbThreads);
+  const dim3 grid(unsigned((items + kGroups - 1) / kGroups)), block(kRbThreads);
   if (kmax <= 2)
     hipLaunchKernelGGL(rebind_kernel<4>, grid, block, 0, stream, a);
-  else if (kmax == 3)
-    hipLaunchKernelGGL(rebind_kernel<8>, grid, block, 0, stream, a);
   else
     hipLaunchKernelGGL(rebind_kernel<16>, grid, block, 0, stream, a);
   return hipGetLastError();

@@ -282,3 +282,32 @@ def test_op_calls_without_symbols_and_with_empty_rows():
         np.testing.assert_allclose(e2.cpu().numpy(), eo2, atol=TOL)
         np.testing.assert_allclose(gr.cpu().numpy(), go2, atol=TOL * max(1, np.abs(go2).max()))
     plan_cache.clear()
+
+
+@pytest.mark.parametrize("mode", ["tfq", "analytic"])
+@pytest.mark.parametrize("gates,at", [(1, (0,)), (6, (0, 5)), (7, (5, 6)), (7, (6,)), (12, (0, 11)),
+                                      (13, (0, 12)), (30, (3, 27))])
+def test_device_values_of_long_blocks(mode, gates, at):
+    """One two-qubit block of ``gates`` gates with symbolic ones at ``at``:
+    rebind_kernel evaluates six gates at a time, so symbols (and the gradient
+    gates) sit first, last and on both sides of a boundary.  The host evaluates
+    the same recipe, so the outputs agree as in the tests above."""
+    rng = np.random.default_rng(gates * 10 + len(at))
+    q = C.LineQubit.range(2)
+    names = ["a", "b"]
+    ops = []
+    for i in range(gates):
+        two = i % 3 == 2 or gates == 1
+        sym = C.Symbol(names[at.index(i)]) if i in at else float(rng.uniform(-1, 1))
+        ops.append(C.ISwapPowGate(exponent=sym).on(q[1], q[0]) if two else
+                   C.YPowGate(exponent=sym).on(q[i % 2]))
+    progs = S.convert_to_tensor([C.Circuit(ops + [C.I(x) for x in q])] * 3)
+    ps = S.convert_to_tensor([[W.random_pauli_sum(rng, q, 3), W.random_pauli_sum(rng, q, 2)]] * 3)
+    v1, v2 = _values(rng, 3, 2), _values(rng, 3, 2)
+    g = rng.uniform(-1, 1, size=(3, 2)).astype(np.float32)
+    host, shape = _adjoint_plan(progs, names, v1, ps, g, mode)
+    dev, _ = _adjoint_plan(progs, names, v1, ps, g, mode)
+    host.rebind(v2)
+    dev.stage_values(v2)
+    _say(f"long block, {gates} gates, mode={mode}")
+    np.testing.assert_allclose(_launch(dev, shape), _launch(host, shape), atol=MATCH)

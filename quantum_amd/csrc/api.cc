@@ -110,7 +110,7 @@ struct tfqx_plan {
   bool rb_tables_dirty = false, values_staged = false;
   bool device_mats = false;  // the device holds matrices newer than staging's
   int lds_log2 = 0;
-  int kmax = 2;
+  int variant = kVariantAny;
   int grid = 0;
   bool with_expectation = false;  // adjoint plan also writes expectations
   bool tfq_fd = true;
@@ -310,6 +310,29 @@ void Layout(tfqx_plan* p) {
   put(p->off_passes, g.passes.data(), g.passes.size() * sizeof(DevPass));
 }
 
+// The kernel variant of a batch program (batch_kernels.h): the engine of an op
+// list shows in its first op, a remap for the register engine.  The LDS variant
+// keeps gradient partials in LDS beside two states of up to 12 qubits (a wider
+// circuit without the register engine, which tuning can ask for, runs in the
+// general one).
+int ChooseVariant(const BatchProgram& g, int mode) {
+  for (const auto& o : g.ops)
+    if (o.k > 2) return kVariantWide;
+  bool lds = false, engine = false;
+  auto list = [&](int b, int e) {
+    if (b < e) (g.ops[size_t(b)].type == kOpRemap ? engine : lds) = true;
+  };
+  for (const auto& c : g.circuits) {
+    if (c.flags & (kFlagTiled | kFlagWave)) return kVariantAny;
+    list(c.fwd_begin, c.fwd_end);
+    list(c.rev_begin, c.rev_end);
+    for (int k = c.other_begin; k < c.other_end; ++k)
+      list(g.others[size_t(k)].op_begin, g.others[size_t(k)].op_end);
+  }
+  if (lds && (engine || (BatchBuffers(mode) == 2 && g.max_n > 12))) return kVariantAny;
+  return engine ? kVariantEngine : kVariantLds;
+}
+
 std::atomic<int> g_wave_min{kWaveMinCircuits};
 std::atomic<int> g_stream_min{kTiledMaxQubits + 1};
 
@@ -394,8 +417,7 @@ int BuildPlan(int mode, Inputs& in, int64_t B, int64_t S, int64_t O, int64_t K,
   // Wave mode carves the full LDS allocation into one pair of 2^kWaveMaxQubits
   // buffers per wavefront.
   if (p->prog.num_block < int(p->prog.circuits.size())) p->lds_log2 = resident;
-  p->kmax = 2;
-  for (const auto& o : p->prog.ops) p->kmax = std::max<int>(p->kmax, o.k);
+  p->variant = ChooseVariant(p->prog, mode);
   Layout(p.get());
   *out = p.release();
   return TFQX_OK;
@@ -554,7 +576,7 @@ BatchArgs MakeArgs(tfqx_plan* p, void* ws, void* output) {
   uint8_t* base = static_cast<uint8_t*>(ws);
   BatchArgs a{};
   a.mode = p->mode;
-  a.kmax = p->kmax;
+  a.variant = p->variant;
   a.circuits = reinterpret_cast<const DevCircuit*>(base + p->off_circuits);
   a.ncirc = int(p->prog.circuits.size());
   a.nblock = p->prog.num_block;
@@ -1169,7 +1191,7 @@ int tfqx_plan_launch(tfqx_plan* p, void* ws, void* output, void* stream, char* e
   if (p->noisy) return NoisyLaunch(p->noisy_plan.get(), ws, output, AsStream(stream), err, len);
   if (p->prog.circuits.empty()) return TFQX_OK;
   if (p->grid == 0) {
-    int maxg = BatchMaxGrid(p->lds_log2, p->mode, p->kmax);
+    int maxg = BatchMaxGrid(p->lds_log2, p->mode, p->variant);
     if (p->prog.any_tiled) maxg = std::min(maxg, kTiledGridCap);
     p->grid = std::max(1, std::min<int>(maxg, int(p->prog.circuits.size())));
   }
@@ -1200,7 +1222,7 @@ int tfqx_graph_capture(tfqx_plan* p, void* ws, void* output, void* stream, tfqx_
   hipStream_t s = AsStream(stream);
   // Resolve occupancy and kernel attributes before capture.
   if (!p->large && p->grid == 0 && !p->prog.circuits.empty()) {
-    int maxg = BatchMaxGrid(p->lds_log2, p->mode, p->kmax);
+    int maxg = BatchMaxGrid(p->lds_log2, p->mode, p->variant);
     if (p->prog.any_tiled) maxg = std::min(maxg, kTiledGridCap);
     p->grid = std::max(1, std::min<int>(maxg, int(p->prog.circuits.size())));
   }

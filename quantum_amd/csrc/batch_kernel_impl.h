@@ -24,6 +24,7 @@
 
 #include "batch_kernels.h"
 #include "lds_ops.h"
+#include "lds_engine.h"
 #include "reg_engine.h"
 
 namespace tfqx {
@@ -55,17 +56,29 @@ __device__ __forceinline__ void for_ops_cached(const DevOp* ops, int b, int e, M
 }
 
 // Forward ops [b, e) on an LDS tile of n qubits (register engine when planned).
-template <int KMAX>
-__device__ __forceinline__ void run_ops(float2* s, int n, const DevOp* ops, int b, int e, MatCache& mc) {
-  if (reg_run_any<false>(s, s, n, ops, b, e, mc, NoAcc())) return;
-  for_ops_cached(ops, b, e, mc,
-                 [&](const DevOp& op, const float2* M) { apply_op<false, KMAX>(s, n, op, M); });
+template <int VAR>
+__device__ __forceinline__ void run_ops(float2* s, int n, const DevOp* ops, int b, int e,
+                                        MatCache& mc, uint32_t* win) {
+  constexpr int KMAX = VariantKmax(VAR);
+  if constexpr (VAR != kVariantLds)
+    if (reg_run_any<false>(s, s, n, ops, b, e, mc, NoAcc())) return;
+  if constexpr (VAR != kVariantEngine) {
+    if (n >= 2) {
+      lds_run<false, KMAX, false>(s, s, n, ops, b, e, mc, win,
+                                  static_cast<PartRing<false>*>(nullptr),
+                                  [](int, double, double) {});
+      return;
+    }
+    for_ops_cached(ops, b, e, mc,
+                   [&](const DevOp& op, const float2* M) { apply_op<false, KMAX>(s, n, op, M); });
+  }
 }
 
 // Adjoint sweep of ops [b, e) on psi (A) and lambda (B), gradients into gacc.
-template <int KMAX, bool CPLX = false>
+template <int VAR, bool CPLX = false>
 __device__ __forceinline__ void run_reverse(float2* A, float2* B, int n, const DevOp* ops, int b, int e,
-                                            double* gacc, MatCache& mc);
+                                            double* gacc, MatCache& mc, uint32_t* win,
+                                            PartRing<CPLX>* rings);
 
 __device__ __forceinline__ void set_zero_state(float2* s, uint32_t N) {
   for (uint32_t x = threadIdx.x; x < N; x += kThreads) s[x] = make_float2(x == 0 ? 1.f : 0.f, 0.f);
@@ -102,23 +115,42 @@ __device__ __forceinline__ uint32_t cdf_search(const double* cdf, uint32_t N, do
   return lo;
 }
 
+// Pauli terms through the descriptor window in LDS (terms and op descriptors are
+// never needed together): read from memory one by one, each costs its latency.
+constexpr int kTermWindow = kDescWindow * int(sizeof(DevOp)) / int(sizeof(DevTerm));
+__device__ __forceinline__ void load_terms(const DevTerm* terms, int t, int te, uint32_t* win) {
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(terms + t);
+  const int words = min(te - t, kTermWindow) * int(sizeof(DevTerm) / 4);
+  __syncthreads();
+  for (int i = threadIdx.x; i < words; i += kThreads) win[i] = src[i];
+  __syncthreads();
+}
+
 // Pauli expectations of state S (LDS or global) for all slots of a circuit.
 __device__ __forceinline__ void expectations(const float2* __restrict__ S, uint32_t N,
                                              const BatchArgs& a, const DevCircuit& c, int row,
-                                             double* red) {
+                                             double* red, uint32_t* win) {
   const int tid = threadIdx.x;
-  int t = uniform(c.term_begin);
-  const int te = uniform(c.term_end);
+  const DevTerm* W = reinterpret_cast<const DevTerm*>(win);
+  const int tb = uniform(c.term_begin), te = uniform(c.term_end);
+  int t = tb, lo = tb;  // the window holds terms [lo, lo + kTermWindow)
+  if (t < te) load_terms(a.terms, t, te, win);
   for (int j = 0; j < a.nslots; ++j) {
     double acc = 0.0;
     bool any = false;
-    while (t < te && a.terms[t].slot == j) {
-      const DevTerm T = a.terms[t];
+    while (t < te) {
+      if (t - lo == kTermWindow) {
+        load_terms(a.terms, t, te, win);
+        lo = t;
+      }
+      const DevTerm T = W[t - lo];
+      if (uniform(T.slot) != j) break;
+      const uint32_t fmask = uint32_t(uniform(int(T.fmask))), zmask = uint32_t(uniform(int(T.zmask)));
       float part = 0.f;
       for (uint32_t x = tid; x < N; x += kThreads) {
-        const float2 pr = cmul_conj_a(S[x ^ T.fmask], S[x]);
+        const float2 pr = cmul_conj_a(S[x ^ fmask], S[x]);
         const float v = T.re * pr.x - T.im * pr.y;
-        part += (__popc(x & T.zmask) & 1) ? -v : v;
+        part += (__popc(x & zmask) & 1) ? -v : v;
       }
       acc += double(part);
       ++t;
@@ -132,18 +164,26 @@ __device__ __forceinline__ void expectations(const float2* __restrict__ S, uint3
 
 // lambda = sum_t w_t P_t psi.
 __device__ __forceinline__ void build_lambda(const float2* __restrict__ S, float2* __restrict__ Lm,
-                                             uint32_t N, const BatchArgs& a, int lb, int le) {
-  for (uint32_t y = threadIdx.x; y < N; y += kThreads) {
-    float2 l = make_float2(0.f, 0.f);
-    for (int t = lb; t < le; ++t) {
-      const DevTerm T = a.terms[t];
-      const uint32_t x = y ^ T.fmask;
-      float2 w = cmul(make_float2(T.re, T.im), S[x]);
-      if (__popc(x & T.zmask) & 1) w = make_float2(-w.x, -w.y);
-      l = cadd(l, w);
+                                             uint32_t N, const BatchArgs& a, int lb, int le,
+                                             uint32_t* win) {
+  const DevTerm* W = reinterpret_cast<const DevTerm*>(win);
+  int lo = lb;
+  do {  // at least once: no terms leave lambda zero
+    const int cnt = min(le - lo, kTermWindow);
+    load_terms(a.terms, lo, le, win);
+    for (uint32_t y = threadIdx.x; y < N; y += kThreads) {
+      float2 l = lo == lb ? make_float2(0.f, 0.f) : Lm[y];
+      for (int t = 0; t < cnt; ++t) {
+        const DevTerm T = W[t];
+        const uint32_t x = y ^ T.fmask;
+        float2 w = cmul(make_float2(T.re, T.im), S[x]);
+        if (__popc(x & T.zmask) & 1) w = make_float2(-w.x, -w.y);
+        l = cadd(l, w);
+      }
+      Lm[y] = l;
     }
-    Lm[y] = l;
-  }
+    lo += kTermWindow;
+  } while (lo < le);
   __syncthreads();
 }
 
@@ -155,10 +195,7 @@ template <bool CPLX>
 __device__ __forceinline__ void param_step(float2* A, float2* B, int n, const DevOp& op,
                                            const float2* M, double* gacc) {
   double acc[2 * kMaxDeriv] = {0.0, 0.0, 0.0, 0.0};
-  switch (op.k) {
-    case 1: apply_param<1>(A, B, n, op, M, acc); break;
-    default: apply_param<2>(A, B, n, op, M, acc); break;
-  }
+  apply_param<1>(A, B, n, op, M, acc);
   const bool lead = (threadIdx.x & 63) == 0;
 #pragma unroll
   for (int d = 0; d < kMaxDeriv; ++d) {
@@ -176,9 +213,11 @@ __device__ __forceinline__ void param_step(float2* A, float2* B, int n, const De
   }
 }
 
-template <int KMAX, bool CPLX>
+template <int VAR, bool CPLX>
 __device__ __forceinline__ void run_reverse(float2* A, float2* B, int n, const DevOp* ops, int b, int e,
-                                            double* gacc, MatCache& mc) {
+                                            double* gacc, MatCache& mc, uint32_t* win,
+                                            PartRing<CPLX>* rings) {
+  constexpr int KMAX = VariantKmax(VAR);
   auto acc = [gacc](int, int col, double w, double v) {
     if (CPLX) {
       atomicAdd(&gacc[2 * col], w);
@@ -187,15 +226,23 @@ __device__ __forceinline__ void run_reverse(float2* A, float2* B, int n, const D
       atomicAdd(&gacc[col], 2.0 * w);
     }
   };
-  if (reg_run_any<true>(A, B, n, ops, b, e, mc, acc)) return;
-  for_ops_cached(ops, b, e, mc, [&](const DevOp& op, const float2* M) {
-    if (op.type == kOpParam) {
-      param_step<CPLX>(A, B, n, op, M, gacc);
-    } else {
-      apply_op<true, KMAX>(A, n, op, M);
-      apply_op<true, KMAX>(B, n, op, M);
+  if constexpr (VAR != kVariantLds)
+    if (reg_run_any<true>(A, B, n, ops, b, e, mc, acc)) return;
+  if constexpr (VAR != kVariantEngine) {
+    if (n >= 2) {
+      lds_run<true, KMAX, CPLX>(A, B, n, ops, b, e, mc, win, rings,
+                                [&](int col, double w, double v) { acc(0, col, w, v); });
+      return;
     }
-  });
+    for_ops_cached(ops, b, e, mc, [&](const DevOp& op, const float2* M) {
+      if (op.type == kOpParam) {
+        param_step<CPLX>(A, B, n, op, M, gacc);
+      } else {
+        apply_op<true, KMAX>(A, n, op, M);
+        apply_op<true, KMAX>(B, n, op, M);
+      }
+    });
+  }
 }
 
 // ------------------------------------------------------------------ wave mode
@@ -288,9 +335,9 @@ __device__ __forceinline__ void wave_circuit(const BatchArgs& a, int ci, float2*
 
 // Tiled forward: the state lives in global memory G; each pass streams its
 // tiles through LDS buffer A.  The first pass starts from |0>.
-template <int KMAX, int RMAX = 4>
+template <int VAR, int RMAX = 4>
 __device__ __forceinline__ void tiled_forward(float2* G, int n, const BatchArgs& a, int pb, int pe, float2* A,
-                              uint64_t* tab, MatCache& mc) {
+                              uint64_t* tab, MatCache& mc, uint32_t* win) {
   const int tid = threadIdx.x;
   bool first = true;
   for (int p = pb; p < pe; ++p) {
@@ -325,7 +372,7 @@ __device__ __forceinline__ void tiled_forward(float2* G, int n, const BatchArgs&
         tile_gather(A, G, T, gidx);
       }
       __syncthreads();
-      run_ops<KMAX>(A, ps.L, a.ops, ps.op_begin, ps.op_end, mc);
+      run_ops<VAR>(A, ps.L, a.ops, ps.op_begin, ps.op_end, mc, win);
       tile_scatter(G, A, T, gidx);
       __syncthreads();
     }
@@ -341,10 +388,10 @@ __device__ __forceinline__ void tiled_forward(float2* G, int n, const BatchArgs&
 }
 
 // Tiled adjoint sweep on psi (G) and lambda (Lg) with LDS tiles A and B.
-template <int KMAX>
+template <int VAR>
 __device__ __forceinline__ void tiled_reverse(float2* G, float2* Lg, int n, const BatchArgs& a, int pb, int pe,
                               float2* A, float2* B, double* gacc, uint64_t* tab,
-                              MatCache& mc) {
+                              MatCache& mc, uint32_t* win) {
   const int tid = threadIdx.x;
   for (int p = pb; p < pe; ++p) {
     const DevPass ps = a.passes[p];
@@ -373,7 +420,8 @@ __device__ __forceinline__ void tiled_reverse(float2* G, float2* Lg, int n, cons
       if (reg_run_any<true>(A, B, ps.L, a.ops, ps.op_begin, ps.op_end, mc, acc, io)) continue;
       tile_gather2(A, B, G, Lg, T, gidx);
       __syncthreads();
-      run_reverse<KMAX>(A, B, ps.L, a.ops, ps.op_begin, ps.op_end, gacc, mc);
+      run_reverse<VAR>(A, B, ps.L, a.ops, ps.op_begin, ps.op_end, gacc, mc, win,
+                       static_cast<PartRing<false>*>(nullptr));
       tile_scatter(G, A, T, gidx);
       tile_scatter(Lg, B, T, gidx);
       __syncthreads();
@@ -386,16 +434,28 @@ __device__ __forceinline__ void tiled_reverse(float2* G, float2* Lg, int n, cons
 // VGPRs at 128 so two workgroups share a CU (four wavefronts per SIMD): on
 // 11-13-qubit expectation batches that runs 1.4-1.5x faster than 190 VGPRs
 // at one workgroup per CU, the spills it costs included.
-constexpr int BatchMinWaves(int mode) {
-  return (mode == kModeExpectation || mode == kModeState || mode == kModeSamples) ? 4 : 1;
+// The LDS engine needs few registers in every mode.
+constexpr int BatchMinWaves(int mode, int var) {
+  return (var == kVariantLds || mode == kModeExpectation || mode == kModeState ||
+          mode == kModeSamples)
+             ? 4
+             : 1;
 }
 
-template <int MODE, int KMAX>
-__global__ __launch_bounds__(kThreads, BatchMinWaves(MODE)) void batch_kernel(BatchArgs a) {
+template <int MODE, int VAR>
+__global__ __launch_bounds__(kThreads, BatchMinWaves(MODE, VAR)) void batch_kernel(BatchArgs a) {
   extern __shared__ float2 lds[];
   __shared__ double red[kWaves];
   __shared__ int s_ci;
-  __shared__ uint64_t tab[kTileTable];
+  constexpr bool kGeneral = VAR == kVariantAny || VAR == kVariantWide;
+  __shared__ uint64_t tab[kGeneral ? kTileTable : 1];
+  __shared__ uint32_t win[kDescWindow * kDescWords];
+  // The general kernels have no LDS left for partials (two 13-qubit tiles).
+  constexpr bool kGradMode = MODE == kModeAdjoint || MODE == kModeInnerProductGrad;
+  constexpr bool kRings = VAR == kVariantLds && kGradMode;
+  using Ring = PartRing<MODE == kModeInnerProductGrad>;
+  __shared__ std::conditional_t<kRings, Ring, char> ring_mem[kRings ? kWaves : 1];
+  Ring* rings = kRings ? reinterpret_cast<Ring*>(ring_mem) : nullptr;
   constexpr int kWindow = MODE == kModeAdjoint ? kMatCacheWide : kMatCache;
   __shared__ float2 mcache[kWindow];
   MatCache mc = mat_cache(mcache, a.mats, kWindow);
@@ -421,7 +481,7 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE)) void batch_kernel(Ba
     const int row = uniform(c.row);
     const uint32_t N = 1u << n;
     const bool empty = (c.flags & kFlagEmpty) != 0;
-    const bool tiled = (c.flags & kFlagTiled) != 0;
+    const bool tiled = kGeneral && (c.flags & kFlagTiled) != 0;
 
     if (empty) {
       if (MODE == kModeExpectation || MODE == kModeSampledExpectation ||
@@ -452,7 +512,7 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE)) void batch_kernel(Ba
       for (int o = uniform(c.other_begin); o < c.other_end; ++o) {
         const DevOther ot = a.others[o];
         set_zero_state(psi, N);
-        run_ops<KMAX>(psi, n, a.ops, uniform(ot.op_begin), uniform(ot.op_end), mc);
+        run_ops<VAR>(psi, n, a.ops, uniform(ot.op_begin), uniform(ot.op_end), mc, win);
         const float w = ot.weight;
         for (uint32_t x = tid; x < N; x += kThreads) {
           const float2 p = psi[x];
@@ -461,35 +521,36 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE)) void batch_kernel(Ba
         __syncthreads();
       }
     }
-    if (tiled) {
+    if (!tiled) {
+      set_zero_state(psi, N);
+      run_ops<VAR>(psi, n, a.ops, uniform(c.fwd_begin), uniform(c.fwd_end), mc, win);
+    } else if constexpr (kGeneral) {
       // The adjoint's forward carries one state: its passes may use 14-qubit
       // tiles (the LDS of the two 13-qubit reverse tiles) and five register
       // qubits.
-      tiled_forward<KMAX, MODE == kModeAdjoint ? 5 : 4>(gpsi, n, a, uniform(c.fwd_pass_begin),
-                                                        uniform(c.fwd_pass_end), psi, tab, mc);
-    } else {
-      set_zero_state(psi, N);
-      run_ops<KMAX>(psi, n, a.ops, uniform(c.fwd_begin), uniform(c.fwd_end), mc);
+      tiled_forward<VAR, MODE == kModeAdjoint ? 5 : 4>(gpsi, n, a, uniform(c.fwd_pass_begin),
+                                                       uniform(c.fwd_pass_end), psi, tab, mc, win);
     }
 
     if (MODE == kModeExpectation || (MODE == kModeAdjoint && a.exp_out)) {
-      if (tiled) expectations(gpsi, N, a, c, row, red);
-      else expectations(psi, N, a, c, row, red);
+      if (tiled) expectations(gpsi, N, a, c, row, red, win);
+      else expectations(psi, N, a, c, row, red, win);
     }
 
-    if (MODE == kModeAdjoint) {
+    if constexpr (MODE == kModeAdjoint) {
       double* gacc = a.grad_acc + size_t(row) * a.nsym;
       for (int j = tid; j < a.nsym; j += kThreads) gacc[j] = 0.0;
       __threadfence();  // the zeros reach L2 before any wavefront's atomics
       const int lb = uniform(c.lam_begin), le = uniform(c.lam_end);
-      if (tiled) {
-        build_lambda(gpsi, glam, N, a, lb, le);
-        tiled_reverse<KMAX>(gpsi, glam, n, a, uniform(c.rev_pass_begin), uniform(c.rev_pass_end), psi,
-                      buf2, gacc, tab, mc);
-      } else {
+      if (!tiled) {
         float2* lam = buf2;
-        build_lambda(psi, lam, N, a, lb, le);
-        run_reverse<KMAX>(psi, lam, n, a.ops, uniform(c.rev_begin), uniform(c.rev_end), gacc, mc);
+        build_lambda(psi, lam, N, a, lb, le, win);
+        run_reverse<VAR>(psi, lam, n, a.ops, uniform(c.rev_begin), uniform(c.rev_end), gacc, mc, win,
+                         rings);
+      } else if constexpr (kGeneral) {
+        build_lambda(gpsi, glam, N, a, lb, le, win);
+        tiled_reverse<VAR>(gpsi, glam, n, a, uniform(c.rev_pass_begin), uniform(c.rev_pass_end), psi,
+                           buf2, gacc, tab, mc, win);
       }
       // Gradients arrive by atomics; read them back from L2.
       __threadfence();
@@ -499,14 +560,14 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE)) void batch_kernel(Ba
             float(__hip_atomic_load(&gacc[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     }
 
-    if (MODE == kModeInnerProductGrad) {
+    if constexpr (MODE == kModeInnerProductGrad) {
       // Adjoint sweep with complex accumulation (tfq_inner_product_grad.cc:259-314).
       double* gacc = a.grad_acc + size_t(row) * a.nsym * 2;
       for (int j = tid; j < 2 * a.nsym; j += kThreads) gacc[j] = 0.0;
       __threadfence();  // the zeros reach L2 before any wavefront's atomics
       __syncthreads();
-      run_reverse<KMAX, true>(psi, buf2, n, a.ops, uniform(c.rev_begin), uniform(c.rev_end), gacc,
-                              mc);
+      run_reverse<VAR, true>(psi, buf2, n, a.ops, uniform(c.rev_begin), uniform(c.rev_end), gacc,
+                             mc, win, rings);
       __threadfence();
       __syncthreads();
       for (int j = tid; j < a.nsym; j += kThreads)
@@ -580,7 +641,7 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE)) void batch_kernel(Ba
       for (int o = uniform(c.other_begin); o < c.other_end; ++o) {
         const DevOther ot = a.others[o];
         set_zero_state(phi, N);
-        run_ops<KMAX>(phi, n, a.ops, uniform(ot.op_begin), uniform(ot.op_end), mc);
+        run_ops<VAR>(phi, n, a.ops, uniform(ot.op_begin), uniform(ot.op_end), mc, win);
         double re = 0.0, im = 0.0;
         for (uint32_t x = tid; x < N; x += kThreads) {
           const float2 p = cmul_conj_a(psi[x], phi[x]);
@@ -597,7 +658,7 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE)) void batch_kernel(Ba
   }
 
   // Wave mode: each wavefront pulls small circuits of its own.
-  if constexpr (MODE == kModeExpectation || MODE == kModeAdjoint) {
+  if constexpr (kGeneral && (MODE == kModeExpectation || MODE == kModeAdjoint)) {
     if (a.nblock < a.ncirc) {
       const int nwave = a.ncirc - a.nblock;
       float2* P = lds + size_t(tid >> 6) * (2u << kWaveMaxQubits);

@@ -7,9 +7,21 @@
 
 namespace tfqx {
 
+// Kernel variants of a mode, chosen by what a plan's circuits need.  One kernel
+// with every engine spills registers in each engine's loop (a scratch reload per
+// op costs as much as a 10-qubit op), so plans that need one engine only get a
+// kernel with that one.
+enum BatchVariant : int {
+  kVariantAny = 0,     // ops of at most two qubits, any circuits
+  kVariantWide = 1,    // ops of three or four qubits
+  kVariantLds = 2,     // every op list runs on the LDS engine; none tiled, none in wave mode
+  kVariantEngine = 3,  // every op list runs on the register engine; likewise
+};
+constexpr int VariantKmax(int variant) { return variant == kVariantWide ? 4 : 2; }
+
 struct BatchArgs {
   int mode;            // BatchMode
-  int kmax;            // widest fused op in the program (selects the kernel variant)
+  int variant;         // BatchVariant
   const DevCircuit* circuits;
   int ncirc;
   int nblock;          // circuits [0, nblock) run per workgroup, the rest per wavefront
@@ -57,6 +69,6 @@ constexpr int kTiledGridCap = 512;
 int BatchBuffers(int mode);
 size_t BatchLdsBytes(int lds_log2, int mode);
 hipError_t LaunchBatch(const BatchArgs& args, int grid, hipStream_t stream);
-int BatchMaxGrid(int lds_log2, int mode, int kmax);
+int BatchMaxGrid(int lds_log2, int mode, int variant);
 
 }  // namespace tfqx

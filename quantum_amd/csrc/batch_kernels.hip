@@ -7,19 +7,19 @@
 
 namespace tfqx {
 
-const void* BatchKernelExpectation(int mode, int kmax);
-const void* BatchKernelAdjoint(int mode, int kmax);
-const void* BatchKernelInnerProductGrad(int mode, int kmax);
-const void* BatchKernelOther(int mode, int kmax);
+const void* BatchKernelExpectation(int mode, int variant);
+const void* BatchKernelAdjoint(int mode, int variant);
+const void* BatchKernelInnerProductGrad(int mode, int variant);
+const void* BatchKernelOther(int mode, int variant);
 
 namespace {
 
-const void* KernelFor(int mode, int kmax) {
+const void* KernelFor(int mode, int variant) {
   switch (mode) {
-    case kModeExpectation: return BatchKernelExpectation(mode, kmax);
-    case kModeAdjoint: return BatchKernelAdjoint(mode, kmax);
-    case kModeInnerProductGrad: return BatchKernelInnerProductGrad(mode, kmax);
-    default: return BatchKernelOther(mode, kmax);
+    case kModeExpectation: return BatchKernelExpectation(mode, variant);
+    case kModeAdjoint: return BatchKernelAdjoint(mode, variant);
+    case kModeInnerProductGrad: return BatchKernelInnerProductGrad(mode, variant);
+    default: return BatchKernelOther(mode, variant);
   }
 }
 
@@ -41,16 +41,16 @@ hipError_t LaunchBatch(const BatchArgs& args, int grid, hipStream_t stream) {
   // attribute (and setting one above 64 KiB is rejected by the runtime).
   const size_t lds = BatchLdsBytes(args.lds_log2, args.mode);
   void* params[] = {const_cast<BatchArgs*>(&args)};
-  return hipLaunchKernel(KernelFor(args.mode, args.kmax), dim3(grid), dim3(kThreads), params, lds,
+  return hipLaunchKernel(KernelFor(args.mode, args.variant), dim3(grid), dim3(kThreads), params, lds,
                          stream);
 }
 
-int BatchMaxGrid(int lds_log2, int mode, int kmax) {
+int BatchMaxGrid(int lds_log2, int mode, int variant) {
   int dev = 0, cus = 0, per_cu = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   const size_t lds = BatchLdsBytes(lds_log2, mode);
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, KernelFor(mode, kmax), kThreads, lds);
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, KernelFor(mode, variant), kThreads, lds);
   if (per_cu < 1) per_cu = 1;
   if (cus < 1) cus = 1;
   return cus * per_cu;

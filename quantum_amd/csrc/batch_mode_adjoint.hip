@@ -5,16 +5,20 @@ namespace tfqx {
 namespace {
 
 template <int MODE>
-const void* KernelPtr(int kmax) {
-  return kmax <= 2 ? reinterpret_cast<const void*>(&batch_kernel<MODE, 2>)
-                   : reinterpret_cast<const void*>(&batch_kernel<MODE, 4>);
+const void* KernelPtr(int variant) {
+  switch (variant) {
+    case kVariantWide: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantWide>);
+    case kVariantLds: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantLds>);
+    case kVariantEngine: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantEngine>);
+    default: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantAny>);
+  }
 }
 
 }  // namespace
 
-const void* BatchKernelAdjoint(int mode, int kmax) {
+const void* BatchKernelAdjoint(int mode, int variant) {
   switch (mode) {
-    default: return KernelPtr<kModeAdjoint>(kmax);
+    default: return KernelPtr<kModeAdjoint>(variant);
   }
 }
 

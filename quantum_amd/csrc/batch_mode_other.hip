@@ -5,19 +5,23 @@ namespace tfqx {
 namespace {
 
 template <int MODE>
-const void* KernelPtr(int kmax) {
-  return kmax <= 2 ? reinterpret_cast<const void*>(&batch_kernel<MODE, 2>)
-                   : reinterpret_cast<const void*>(&batch_kernel<MODE, 4>);
+const void* KernelPtr(int variant) {
+  switch (variant) {
+    case kVariantWide: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantWide>);
+    case kVariantLds: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantLds>);
+    case kVariantEngine: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantEngine>);
+    default: return reinterpret_cast<const void*>(&batch_kernel<MODE, kVariantAny>);
+  }
 }
 
 }  // namespace
 
-const void* BatchKernelOther(int mode, int kmax) {
+const void* BatchKernelOther(int mode, int variant) {
   switch (mode) {
-    case kModeState: return KernelPtr<kModeState>(kmax);
-    case kModeSamples: return KernelPtr<kModeSamples>(kmax);
-    case kModeSampledExpectation: return KernelPtr<kModeSampledExpectation>(kmax);
-    default: return KernelPtr<kModeInnerProduct>(kmax);
+    case kModeState: return KernelPtr<kModeState>(variant);
+    case kModeSamples: return KernelPtr<kModeSamples>(variant);
+    case kModeSampledExpectation: return KernelPtr<kModeSampledExpectation>(variant);
+    default: return KernelPtr<kModeInnerProduct>(variant);
   }
 }
 

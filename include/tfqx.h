@@ -231,6 +231,11 @@ int tfqx_plan_rebind_downstream(tfqx_plan* plan, const float* downstream_grads, 
 int tfqx_plan_stage_values(tfqx_plan* plan, const float* symbol_values, char* err,
                            int64_t err_len);
 
+/* New random seed for the sampling and noisy plans (no upload needed; other
+ * plans ignore it).  The reference draws a fresh seed per call
+ * (tfq_simulate_samples_op.cc:131-140). */
+int tfqx_plan_set_seed(tfqx_plan* plan, uint64_t seed, char* err, int64_t err_len);
+
 /* Fusion decisions of the planner for one program (host only): the fused ops
  * of the forward program at the given width (1..4).  ops_out[i][8] = {k,
  * bit0..bit3 (global bit positions, ascending, -1 unused), 1 if the op keeps

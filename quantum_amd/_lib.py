@@ -80,6 +80,8 @@ def _declare(lib):
     lib.tfqx_plan_rebind_downstream.restype = c.c_int
     lib.tfqx_plan_stage_values.argtypes = [P, P, c.c_char_p, i64]
     lib.tfqx_plan_stage_values.restype = c.c_int
+    lib.tfqx_plan_set_seed.argtypes = [P, c.c_uint64, c.c_char_p, i64]
+    lib.tfqx_plan_set_seed.restype = c.c_int
     lib.tfqx_plan_upload_changed.argtypes = [P, P, P, c.c_char_p, i64]
     lib.tfqx_plan_upload_changed.restype = c.c_int
     lib.tfqx_plan_stats.argtypes = [P, P, i64]
@@ -151,7 +153,8 @@ EXPORTED_SYMBOLS = (
     "tfqx_strings_data", "tfqx_strings_offsets", "tfqx_strings_dim", "tfqx_strings_destroy",
     "tfqx_plan_inner_product",
     "tfqx_plan_inner_product_grad", "tfqx_plan_adjoint_gradient", "tfqx_plan_expectation_and_gradient", "tfqx_plan_rebind",
-    "tfqx_plan_rebind_downstream", "tfqx_plan_stage_values", "tfqx_plan_upload_changed",
+    "tfqx_plan_rebind_downstream", "tfqx_plan_stage_values", "tfqx_plan_set_seed",
+    "tfqx_plan_upload_changed",
     "tfqx_debug_fuse", "tfqx_debug_philox_uniform",
     "tfqx_plan_stats",
     "tfqx_plan_max_num_qubits", "tfqx_plan_workspace_bytes",
@@ -245,6 +248,11 @@ class Plan:
         err = ctypes.create_string_buffer(4096)
         check(self._lib.tfqx_plan_stage_values(self.handle, v.ctypes.data if v.size else None,
                                                err, 4096), err)
+
+    def set_seed(self, seed):
+        """New random seed for a sampling or noisy plan."""
+        err = ctypes.create_string_buffer(4096)
+        check(self._lib.tfqx_plan_set_seed(self.handle, seed, err, 4096), err)
 
     def rebind_downstream(self, grads):
         """New downstream gradients (float32 [batch, n_ops]) for an adjoint plan of

@@ -17,6 +17,7 @@
 #include "circuit.h"
 #include "large.h"
 #include "noisy.h"
+#include "parallel.h"
 #include "plan.h"
 #include "wire.h"
 
@@ -36,31 +37,6 @@ void SetErr(char* err, int64_t len, const std::string& msg) {
 int Fail(char* err, int64_t len, int code, const std::string& msg) {
   SetErr(err, len, msg);
   return code;
-}
-
-int HostThreads() {
-  unsigned n = std::thread::hardware_concurrency();
-  return int(std::max(1u, std::min(n, 16u)));  // one GPU's share of host cores
-}
-
-template <typename F>
-void ParallelFor(int n, F f) {
-  const int T = std::min(HostThreads(), n);
-  if (T <= 1) {
-    for (int i = 0; i < n; ++i) f(i);
-    return;
-  }
-  std::atomic<int> next(0);
-  std::vector<std::thread> pool;
-  for (int t = 0; t < T; ++t)
-    pool.emplace_back([&]() {
-      while (true) {
-        int i = next.fetch_add(1);
-        if (i >= n) break;
-        f(i);
-      }
-    });
-  for (auto& th : pool) th.join();
 }
 
 struct FirstError {
@@ -184,8 +160,8 @@ Status Prepare(const uint8_t* programs, const int64_t* poff, int64_t B, const ui
   if (B < 0 || S < 0 || O < 0 || K < 0) return Status::Invalid("negative dimension");
   in->values = values;
   // Byte-identical programs (a circuit tiled over a batch of parameter sets)
-  // are parsed and resolved once.
-  bool same = B >= 1 && !other && !noisy;
+  // are parsed and resolved once (a noisy program's channels have no symbols).
+  bool same = B >= 1 && !other;
   for (int64_t i = 1; same && i < B; ++i) same = SameBytes(programs, poff, i, 0);
   Status s = ParsePrograms(programs, poff, same ? 1 : B, &in->programs);
   if (!s.ok()) return s;
@@ -210,7 +186,8 @@ Status Prepare(const uint8_t* programs, const int64_t* poff, int64_t B, const ui
     SymbolMap sm;
     sm.columns = &in->columns;
     sm.values = values;
-    s = BuildCircuit(in->programs[0], sm, &tmpl);
+    s = noisy ? BuildNoisyCircuit(in->programs[0], sm, &tmpl)
+              : BuildCircuit(in->programs[0], sm, &tmpl);
     if (!s.ok()) return s;
     in->shared = tmpl.num_qubits <= shared_max_n;
   }
@@ -975,6 +952,14 @@ int tfqx_plan_stage_values(tfqx_plan* p, const float* values, char* err, int64_t
   if (p->B * p->S > 0)
     memcpy(p->rb_image.data(), values, size_t(p->B) * size_t(p->S) * sizeof(float));
   p->values_staged = true;
+  return TFQX_OK;
+}
+
+int tfqx_plan_set_seed(tfqx_plan* p, uint64_t seed, char* err, int64_t len) {
+  if (!p) return Fail(err, len, TFQX_INVALID_ARGUMENT, "null argument");
+  p->seed = seed;
+  if (p->large) p->large_plan->seed = seed;
+  if (p->noisy) p->noisy_plan->seed = seed;
   return TFQX_OK;
 }
 

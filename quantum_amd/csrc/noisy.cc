@@ -1,6 +1,8 @@
 // Host planner of the noisy trajectory kernel (see noisy.h).
 #include "noisy.h"
 
+#include "parallel.h"
+
 #include <string.h>
 
 #include <algorithm>
@@ -64,11 +66,24 @@ Status BuildNoisyPlan(int mode, const std::vector<Circuit>& circuits,
   p->row_empty.assign(size_t(B), 0);
   FuseOptions fo;
   fo.max_fuse = 2;  // the register engine applies one- and two-qubit blocks
-  std::vector<DevChunk> wg_chunks, wave_chunks;
-  std::vector<double> cost;
+  // Each row's program, offsets relative to its own arrays; rows in parallel.
+  struct Piece {
+    DevCircuit dc{};
+    std::vector<DevOp> ops;
+    std::vector<cfloat> mats;
+    std::vector<DevTerm> terms;
+  };
   for (int64_t i = 0; i < B; ++i) {
     const Circuit& c = circuits[size_t(i)];
     p->max_nq = std::max(p->max_nq, c.num_qubits);
+    if (c.num_qubits > kNoisyMaxQubits && !(c.gates.empty() && c.channels.empty()))
+      return Status{12, "Noisy circuits of at most " + std::to_string(kNoisyMaxQubits) +
+                            " qubits are supported, got " + std::to_string(c.num_qubits) + "."};
+  }
+  std::vector<Piece> pieces(static_cast<size_t>(B));
+  ParallelFor(int(B), [&](int i) {
+    const Circuit& c = circuits[size_t(i)];
+    Piece& pc = pieces[size_t(i)];
     // Identity terms (and rows of empty programs) are finished on the host side.
     if (!sums.empty() && !sums[size_t(i)].empty())
       for (int64_t j = 0; j < O; ++j)
@@ -77,18 +92,14 @@ Status BuildNoisyPlan(int mode, const std::vector<Circuit>& circuits,
     // (#679) programs without operations give -2 (tfq_noisy_expectation.cc:190-196).
     if (c.gates.empty() && c.channels.empty()) {
       p->row_empty[size_t(i)] = 1;
-      continue;
+      return;
     }
     const int n = c.num_qubits;
-    if (n > kNoisyMaxQubits)
-      return Status{12, "Noisy circuits of at most " + std::to_string(kNoisyMaxQubits) +
-                            " qubits are supported, got " + std::to_string(n) + "."};
     const bool wave = n <= kWaveMaxQubits;
-    DevCircuit dc{};
+    DevCircuit& dc = pc.dc;
     dc.n = wave ? std::max(n, kWaveRegBits) : n;
     dc.row = int(i);
     dc.flags = wave ? kFlagWave : 0;
-    dc.fwd_begin = int(p->ops.size());
     // Fused gate segments between channels, each channel an op of its own.
     int g0 = 0;
     for (size_t k = 0; k <= c.channels.size(); ++k) {
@@ -96,31 +107,50 @@ Status BuildNoisyPlan(int mode, const std::vector<Circuit>& circuits,
       if (g1 > g0) {
         std::vector<FusedOp> fused;
         FuseGates(c, g0, g1, fo, &fused);
-        for (const auto& f : fused) p->ops.push_back(FusedToDevOp(f, &p->mats));
+        for (const auto& f : fused) pc.ops.push_back(FusedToDevOp(f, &pc.mats));
       }
-      if (k < c.channels.size()) p->ops.push_back(ChannelOp(c.channels[k], int(k), &p->mats));
+      if (k < c.channels.size()) pc.ops.push_back(ChannelOp(c.channels[k], int(k), &pc.mats));
       g0 = g1;
     }
-    if (wave) InsertRemapsR(&p->ops, size_t(dc.fwd_begin), dc.n, kWaveRegBits);
-    dc.fwd_end = int(p->ops.size());
+    if (wave) InsertRemapsR(&pc.ops, 0, dc.n, kWaveRegBits);
+    dc.fwd_end = int(pc.ops.size());
     // Non-identity terms, slot by slot.  Sampled expectation: unit weight
     // (times i^#Y) with the coefficient's float bits in `pad`.
-    dc.term_begin = int(p->terms.size());
     if (mode != kModeNoisySamples) {
       for (int64_t j = 0; j < O; ++j) {
         for (const auto& t : sums[size_t(i)][size_t(j)]) {
           if (t.ops.empty()) continue;
           if (mode == kModeNoisyExpectation) {
-            p->terms.push_back(PauliToTerm(t, t.coef, int(j)));
+            pc.terms.push_back(PauliToTerm(t, t.coef, int(j)));
           } else {
             DevTerm d = PauliToTerm(t, 1.0f, int(j));
             memcpy(&d.pad, &t.coef, sizeof(float));
-            p->terms.push_back(d);
+            pc.terms.push_back(d);
           }
         }
       }
     }
-    dc.term_end = int(p->terms.size());
+    dc.term_end = int(pc.terms.size());
+  });
+  std::vector<DevChunk> wg_chunks, wave_chunks;
+  std::vector<double> cost;
+  for (int64_t i = 0; i < B; ++i) {
+    if (p->row_empty[size_t(i)]) continue;
+    Piece& pc = pieces[size_t(i)];
+    DevCircuit dc = pc.dc;
+    const int op_base = int(p->ops.size()), term_base = int(p->terms.size());
+    const uint32_t mat_base = uint32_t(p->mats.size());
+    dc.fwd_begin += op_base;
+    dc.fwd_end += op_base;
+    dc.term_begin += term_base;
+    dc.term_end += term_base;
+    for (DevOp o : pc.ops) {
+      o.mat += mat_base;
+      for (int d = 0; d < o.nderiv; ++d) o.dmat[d] += mat_base;
+      p->ops.push_back(o);
+    }
+    p->mats.insert(p->mats.end(), pc.mats.begin(), pc.mats.end());
+    p->terms.insert(p->terms.end(), pc.terms.begin(), pc.terms.end());
     const int ci = int(p->circuits.size());
     p->circuits.push_back(dc);
     int T = 0;
@@ -132,7 +162,8 @@ Status BuildNoisyPlan(int mode, const std::vector<Circuit>& circuits,
     p->trajectories += T;
     const double amps = std::ldexp(1.0, dc.n);
     cost.push_back(amps * double(dc.fwd_end - dc.fwd_begin + 1));
-    if (wave) {
+    const int n = circuits[size_t(i)].num_qubits;
+    if (dc.flags & kFlagWave) {
       const int G = 1 << (kWaveMaxQubits - dc.n);
       for (int t = 0; t < T; t += G) wave_chunks.push_back(DevChunk{ci, t, std::min(T, t + G), n});
     } else {

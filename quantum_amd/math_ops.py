@@ -22,7 +22,8 @@ import numpy as np
 
 from . import _lib
 from ._lib import InvalidArgumentError, Plan, StringTensor
-from .tfq_simulate_ops import _common, _plan_args, _run, _torch, as_string_tensor, as_values
+from .tfq_simulate_ops import (_common, _plan_args, _run, _run_cached, _torch, as_string_tensor,
+                               as_values)
 
 _MODES = {"tfq": 0, "analytic": 1}
 
@@ -37,10 +38,13 @@ def _checked_others(programs, other_programs):
 
 
 def _inner_product_raw(programs, names, values, other):
-    P, N, args = _plan_args(programs, names, values)
-    Ot = StringTensor(other)
-    plan = Plan(_lib.lib().tfqx_plan_inner_product, *args, Ot.ptr, Ot.off, other.shape[1])
-    return _run(plan, other.shape, _torch().complex64)
+    def build():
+        P, N, args = _plan_args(programs, names, values)
+        Ot = StringTensor(other)
+        return Plan(_lib.lib().tfqx_plan_inner_product, *args, Ot.ptr, Ot.off, other.shape[1])
+
+    return _run_cached("inner_product", (programs, other), names, values, build,
+                       lambda plan: _run(plan, other.shape, _torch().complex64))
 
 
 def _grad_raw(programs, names, values, other, prev_grad, derivative):

@@ -2,8 +2,8 @@
 
 The reference parses, resolves and fuses every program on every call
 (``core/ops/parse_context.cc:60-92``).  Here an op call whose programs, symbol
-names and Pauli sums are byte-identical to a recent call's reuses that call's
-plan: only the symbolic gate matrices are re-evaluated for the new symbol
+names and Pauli sums (or paired programs) are byte-identical to a recent call's
+reuses that call's plan, and a sampling op's new seed is set in it: only the symbolic gate matrices are re-evaluated for the new symbol
 values (on the device, ``tfqx_plan_stage_values``), and for the adjoint the
 lambda weights for the new downstream gradients
 (``tfqx_plan_rebind_downstream``); the upload then carries only what changed

@@ -119,6 +119,25 @@ def _run(plan, out_shape, dtype):
     return out
 
 
+def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None):
+    """``launch(plan)`` with the plan of a recent call of ``op`` whose string
+    tensors, names and ``extra`` arguments were the same, rebound to ``values``
+    and ``seed``, or with ``build()``'s (see ``plan_cache``)."""
+    from . import plan_cache
+    if not _torch().cuda.is_available():
+        return launch(build())  # the inputs' own errors before the missing device
+    dev, stream = _device_and_stream()
+    key = (op, plan_cache.digest(*strings), tuple(names), tuple(x.shape for x in strings),
+           dev.index, stream, *extra)
+
+    def rebind(plan):
+        plan.stage_values(values)
+        if seed is not None:
+            plan.set_seed(seed)
+
+    return plan_cache.run(key, build, rebind, launch)
+
+
 def _plan_args(programs, names, values):
     P = StringTensor(programs)
     N = StringTensor(names)
@@ -145,27 +164,25 @@ def tfq_simulate_expectation(programs, symbol_names, symbol_values, pauli_sums):
     A call with the same programs, names and Pauli sums as a recent one reuses
     its plan (``plan_cache``): the new symbol values are uploaded and evaluated
     into the plan's matrices on the device."""
-    from . import plan_cache
     programs, names, values = _common(programs, symbol_names, symbol_values)
     pauli_sums = as_string_tensor(pauli_sums, 2, "pauli_sums")
-    _, stream = _device_and_stream()
-    key = ("expectation", plan_cache.digest(programs, pauli_sums), tuple(names),
-           programs.shape, pauli_sums.shape, stream)
     shape = (programs.shape[0], pauli_sums.shape[1])
-
-    def build():
-        return plan_expectation(programs, names, values, pauli_sums)[0]
-
-    return plan_cache.run(key, build, lambda plan: plan.stage_values(values),
-                          lambda plan: _run(plan, shape, _torch().float32))
+    return _run_cached("expectation", (programs, pauli_sums), names, values,
+                       lambda: plan_expectation(programs, names, values, pauli_sums)[0],
+                       lambda plan: _run(plan, shape, _torch().float32))
 
 
 def tfq_simulate_state(programs, symbol_names, symbol_values):
     """Final states ``[batch, 2**max_nq]`` (complex64), padded with -2."""
     programs, names, values = _common(programs, symbol_names, symbol_values)
-    P, N, args = _plan_args(programs, names, values)
-    plan = Plan(_lib.lib().tfqx_plan_simulate_state, *args)
-    return _run(plan, (programs.shape[0], 2 ** plan.max_num_qubits), _torch().complex64)
+
+    def build():
+        P, N, args = _plan_args(programs, names, values)
+        return Plan(_lib.lib().tfqx_plan_simulate_state, *args)
+
+    return _run_cached("state", (programs,), names, values, build,
+                       lambda plan: _run(plan, (programs.shape[0], 2 ** plan.max_num_qubits),
+                                         _torch().complex64))
 
 
 def _num_samples_scalar(num_samples):
@@ -190,9 +207,15 @@ def tfq_simulate_samples(programs, symbol_names, symbol_values, num_samples, see
     ``seed`` fixes the Philox stream (the reference draws a fresh seed per call)."""
     programs, names, values = _common(programs, symbol_names, symbol_values)
     n = _num_samples_scalar(num_samples)
-    P, N, args = _plan_args(programs, names, values)
-    plan = Plan(_lib.lib().tfqx_plan_simulate_samples, *args, n, _seed(seed))
-    return _run(plan, (programs.shape[0], n, plan.max_num_qubits), _torch().int8)
+    seed = _seed(seed)
+
+    def build():
+        P, N, args = _plan_args(programs, names, values)
+        return Plan(_lib.lib().tfqx_plan_simulate_samples, *args, n, seed)
+
+    return _run_cached("samples", (programs,), names, values, build,
+                       lambda plan: _run(plan, (programs.shape[0], n, plan.max_num_qubits),
+                                         _torch().int8), extra=(n,), seed=seed)
 
 
 def tfq_simulate_sampled_expectation(programs, symbol_names, symbol_values, pauli_sums,
@@ -210,11 +233,17 @@ def tfq_simulate_sampled_expectation(programs, symbol_names, symbol_values, paul
         raise InvalidArgumentError(
             f"num_samples and pauli_sums do not match. Got {list(ns.shape)} and "
             f"{list(pauli_sums.shape)}.")
-    P, N, args = _plan_args(programs, names, values)
-    S = StringTensor(pauli_sums)
-    plan = Plan(_lib.lib().tfqx_plan_simulate_sampled_expectation, *args, S.ptr, S.off,
-                pauli_sums.shape[1], np_ptr(ns), _seed(seed))
-    return _run(plan, pauli_sums.shape, _torch().float32)
+    seed = _seed(seed)
+
+    def build():
+        P, N, args = _plan_args(programs, names, values)
+        S = StringTensor(pauli_sums)
+        return Plan(_lib.lib().tfqx_plan_simulate_sampled_expectation, *args, S.ptr, S.off,
+                    pauli_sums.shape[1], np_ptr(ns), seed)
+
+    return _run_cached("sampled_expectation", (programs, pauli_sums), names, values, build,
+                       lambda plan: _run(plan, pauli_sums.shape, _torch().float32),
+                       extra=(ns.tobytes(),), seed=seed)
 
 
 def padded_to_ragged(masked_state):

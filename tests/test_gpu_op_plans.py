@@ -1,0 +1,80 @@
+"""Ops that reuse their plans across calls (state, samples, sampled expectation,
+inner product): a call with new values, and a new seed, equals the same call
+with the cache off.  The matrices of a reused plan are evaluated on the device
+(last-bit sine and cosine), so states agree to 1e-6 and draws may move only where
+a uniform lies that close to a prefix sum: at most 1 bit in 1000."""
+
+import numpy as np
+import pytest
+
+from quantum_amd import circuits as C
+from quantum_amd import plan_cache
+from quantum_amd import serialize as S
+from quantum_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _need_gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    plan_cache.clear()
+    yield
+    plan_cache.set_capacity(8)
+
+
+def _ops(progs, names, sums, other):
+    from quantum_amd import math_ops, tfq_simulate_ops as sim
+    B = len(progs)
+    counts = np.arange(1, 2 * B + 1, dtype=np.int32).reshape(B, 2) * 50
+    return {
+        "state": (lambda v, seed: sim.tfq_simulate_state(progs, names, v), 1e-6),
+        "samples": (lambda v, seed: sim.tfq_simulate_samples(progs, names, v, [300], seed=seed), 0),
+        "sampled": (lambda v, seed: sim.tfq_simulate_sampled_expectation(
+            progs, names, v, sums, counts, seed=seed), 0),
+        "inner": (lambda v, seed: math_ops.inner_product(progs, names, v, other), 1e-6),
+    }
+
+
+@pytest.mark.parametrize("op", ["state", "samples", "sampled", "inner"])
+@pytest.mark.parametrize("widths", [(4, 4, 4), (3, 9, 12), (13, 5, 2)])
+def test_reused_plan_equals_a_fresh_one(op, widths):
+    rng = np.random.default_rng(sum(widths))
+    names = ["a", "b"]
+    circuits, sums, other = [], [], []
+    for n in widths:
+        q = C.LineQubit.range(n)
+        make = lambda sym: W.random_circuit(  # noqa: E731
+            rng, q, 3 * n, symbols=sym, p_symbol=0.6) + C.Circuit([C.I(x) for x in q])
+        circuits.append(make(names))
+        sums.append([W.random_pauli_sum(rng, q, 3) for _ in range(2)])
+        other.append([make(()), make(())])
+    progs, psums, others = map(S.convert_to_tensor, (circuits, sums, other))
+    fn, tol = _ops(progs, names, psums, others)[op]
+    print(f"[gpu-case] reused plan, {op}, widths {widths}", flush=True)
+    values = [rng.uniform(-2, 2, (3, 2)).astype(np.float32) for _ in range(3)]
+    got = [fn(v, seed).cpu().numpy() for seed, v in enumerate(values)]
+    assert len(plan_cache._CACHE) == 1
+    plan_cache.set_capacity(0)
+    for seed, (v, g) in enumerate(zip(values, got)):
+        want = fn(v, seed).cpu().numpy()
+        if tol:
+            np.testing.assert_allclose(g, want, atol=tol)
+        elif op == "samples":
+            assert np.mean(g != want) <= 1e-3
+        else:  # one moved shot of the fewest (50) changes a value by 2 |coefficient| / 50
+            assert np.mean(np.abs(g - want) > 1e-6) <= 0.2
+            np.testing.assert_allclose(g, want, atol=0.2)
+
+
+def test_other_counts_and_shapes_are_other_plans():
+    from quantum_amd import tfq_simulate_ops as sim
+    q = C.LineQubit.range(3)
+    progs = S.convert_to_tensor([C.Circuit(C.H(q[0]), C.CNOT(q[0], q[1]), C.I(q[2]))])
+    a = sim.tfq_simulate_samples(progs, [], np.zeros((1, 0), np.float32), [10], seed=1)
+    b = sim.tfq_simulate_samples(progs, [], np.zeros((1, 0), np.float32), [20], seed=1)
+    assert a.shape == (1, 10, 3) and b.shape == (1, 20, 3)
+    np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy()[:, :10])
+    assert len(plan_cache._CACHE) == 2

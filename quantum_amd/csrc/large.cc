@@ -185,6 +185,80 @@ void SchedulePasses(const std::vector<FusedOp>& ops, int n, int L, std::vector<D
 
 namespace {
 
+// Split `terms` of an n-qubit state into sweeps (TermGroup), appended to `out`.
+// Terms that flip no qubit outside the lowest kTermTile (Z terms flip none) share
+// the first, contiguous tile; the others are taken in order, each tile growing by
+// the qubits of the next terms that still fit.  Terms that flip more than
+// kTermHigh qubits above the low ones, states smaller than a tile and whatever
+// is left after kMaxTermGroups tiles go one by one through memory (direct).
+// lambda: fold (-1)^{popc(f & z)} into the coefficient, since lambda's sign is
+// taken at the target index.
+constexpr int kMaxTermGroups = 16;
+std::vector<TermGroup> GroupTerms(const std::vector<DevTermWide>& terms, int n, bool lambda,
+                                  std::vector<DevTermTile>* out) {
+  std::vector<TermGroup> groups;
+  const uint64_t low = (uint64_t(1) << kTermLow) - 1;
+  std::vector<char> done(terms.size(), 0);
+  size_t left = terms.size();
+  auto emit = [&](size_t i, const DevTermMap& m) {
+    const DevTermWide& T = terms[i];
+    DevTermTile t{};
+    t.fmask = T.fmask;
+    t.zmask = T.zmask;
+    t.floc = uint32_t(T.fmask & low);
+    t.zloc = uint32_t(T.zmask & low);
+    for (int h = 0; h < kTermHigh; ++h) {
+      if (T.fmask >> m.hbit[h] & 1) t.floc |= 1u << (kTermLow + h);
+      if (T.zmask >> m.hbit[h] & 1) t.zloc |= 1u << (kTermLow + h);
+    }
+    const bool minus = lambda && (Popc(T.fmask & T.zmask) & 1);
+    t.re = minus ? -T.re : T.re;
+    t.im = minus ? -T.im : T.im;
+    out->push_back(t);
+    done[i] = 1;
+    --left;
+  };
+  while (left > 0 && n >= kTermTile && int(groups.size()) < kMaxTermGroups) {
+    // High qubits of this tile.
+    uint64_t high = 0;
+    if (groups.empty()) {
+      for (int b = kTermLow; b < kTermTile; ++b) high |= uint64_t(1) << b;
+    } else {
+      for (size_t i = 0; i < terms.size(); ++i) {
+        const uint64_t h = high | (terms[i].fmask & ~low);
+        if (!done[i] && Popc(h) <= kTermHigh) high = h;
+      }
+    }
+    if (Popc(high) == 0) break;  // only terms too wide for any tile are left
+    for (int b = kTermLow; b < n && Popc(high) < kTermHigh; ++b) high |= uint64_t(1) << b;
+    TermGroup g;
+    g.begin = int(out->size());
+    g.map.tilemask = low | high;
+    int h = 0;
+    for (int b = kTermLow; b < n; ++b)
+      if (high >> b & 1) g.map.hbit[h++] = uint8_t(b);
+    for (size_t i = 0; i < terms.size(); ++i)
+      if (!done[i] && (terms[i].fmask & ~(low | high)) == 0) emit(i, g.map);
+    g.end = int(out->size());
+    if (g.end > g.begin) groups.push_back(g);
+    else if (!groups.empty()) break;
+    else groups.push_back(g);  // no term in the contiguous tile: an empty first group
+  }
+  if (left > 0) {
+    TermGroup g;
+    g.direct = true;
+    g.begin = int(out->size());
+    DevTermMap none{};
+    for (int h = 0; h < kTermHigh; ++h) none.hbit[h] = uint8_t(kTermLow + h);
+    for (size_t i = 0; i < terms.size(); ++i)
+      if (!done[i]) emit(i, none);
+    g.end = int(out->size());
+    groups.push_back(g);
+  }
+  if (!groups.empty() && groups[0].begin == groups[0].end) groups.erase(groups.begin());
+  return groups;
+}
+
 int TileQubits(int mode, bool two_buffers) {
   (void)mode;
   const Tuning t = GetTuning();
@@ -319,14 +393,18 @@ Status BuildLargePlan(int mode, const std::vector<Circuit>& circuits,
     if (mode == kModeExpectation || sampled || mode == kModeAdjoint) {
       for (int64_t j = 0; j < O; ++j) {
         int idx = 0;
+        std::vector<DevTermWide> slot;
         for (const auto& p : sums[i][j]) {
           if (p.ops.empty()) {
             lc.ident[j] += p.coef;
+          } else if (sampled) {
+            lp->terms.push_back(WideTerm(p, p.coef, int(j), false, idx));
           } else if (mode != kModeAdjoint || with_expectation) {
-            lp->terms.push_back(WideTerm(p, p.coef, int(j), !sampled, idx));
+            slot.push_back(WideTerm(p, p.coef, int(j), true, idx));
           }
           ++idx;
         }
+        lc.exp_groups.push_back(GroupTerms(slot, lc.n, false, &lp->tile_terms));
       }
     }
     if (sampled) {
@@ -341,16 +419,16 @@ Status BuildLargePlan(int mode, const std::vector<Circuit>& circuits,
     }
     lc.term_end = int(lp->terms.size());
     if (mode == kModeAdjoint) {
-      lc.lam_begin = int(lp->terms.size());
+      std::vector<DevTermWide> lam;
       for (int64_t j = 0; j < O; ++j) {
         const float gj = downstream[i * O + j];
         for (const auto& p : sums[i][j]) {
           const float w = gj * p.coef;
           if (std::fabs(w) < 1e-5f) continue;
-          lp->terms.push_back(WideTerm(p, w, 0, true, 0));
+          lam.push_back(WideTerm(p, w, 0, true, 0));
         }
       }
-      lc.lam_end = int(lp->terms.size());
+      lc.lam_groups = GroupTerms(lam, lc.n, true, &lp->tile_terms);
     }
     if (grad) {
       // Reverse program (as the batch planner), param ops numbered by partial slot.

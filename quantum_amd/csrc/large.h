@@ -25,6 +25,14 @@ struct PassPlan {
   int first_param = 0;   // index of this program's first kOpParam in the param table
 };
 
+// Pauli terms [begin, end) of LargePlan::tile_terms reduced in one sweep of the
+// state: those whose flipped qubits lie in one tile, or (direct) the rest.
+struct TermGroup {
+  int begin = 0, end = 0;
+  bool direct = false;
+  DevTermMap map{};
+};
+
 struct LargeCircuit {
   int n = 0;
   int row = 0;
@@ -35,7 +43,8 @@ struct LargeCircuit {
   std::vector<PassPlan> others;       // inner product paired programs
   std::vector<float> other_weights;   // inner-product gradient: g[row, k] of each paired program
   int term_begin = 0, term_end = 0;   // DevTermWide ranges in the plan's term table
-  int lam_begin = 0, lam_end = 0;
+  std::vector<std::vector<TermGroup>> exp_groups;  // expectation: per slot
+  std::vector<TermGroup> lam_groups;               // adjoint: lambda
   std::vector<int> rot_groups;        // sampled expectation: term ranges per rotation pattern
   std::vector<float> ident;           // O identity constants
 };
@@ -62,10 +71,11 @@ struct LargePlan {
   std::vector<cfloat> mats;
   std::vector<DevPass> passes;
   std::vector<DevTermWide> terms;
+  std::vector<DevTermTile> tile_terms;
   std::vector<int32_t> param_cols;    // symbol column of every (param op, derivative)
   std::vector<DenseOp> dense;         // dense passes (DevPass::dense - 1 indexes this)
   // Workspace layout.
-  size_t off_ops = 0, off_mats = 0, off_passes = 0, off_terms = 0, off_partials = 0,
+  size_t off_ops = 0, off_mats = 0, off_passes = 0, off_terms = 0, off_tile_terms = 0, off_partials = 0,
          off_gacc = 0, off_psi = 0, off_buf2 = 0, off_cdf = 0, off_blocks = 0,
          workspace_bytes = 0;
   size_t image_bytes = 0;

@@ -7,8 +7,8 @@
 //                    The two-buffer variant runs the adjoint reverse sweep on
 //                    psi and lambda together and accumulates FP64 gradient
 //                    partials per workgroup.
-//   expect_kernel    XOR-mask Pauli reduction over the state, FP64 partials.
-//   lambda_kernel    lambda = sum_t w_t P_t psi (one streaming pass).
+//   terms_kernel     Pauli expectations (FP64 partials), or lambda = sum_t w_t P_t
+//                    psi, from tiles of the state in LDS.
 //   ip_kernel        <psi|phi> with FP64 partials.
 //   prob_blocks / shots_*  sampling without a full CDF: one coalesced read of
 //                    the state gives, per 4096-amplitude block, the FP64
@@ -338,9 +338,105 @@ __global__ __launch_bounds__(kThreads, K == 5 ? 4 : 2) void dense_kernel(DenseAr
   }
 }
 
+// ------------------------------------------------------------------ Pauli terms
+// Terms [0, count) of one group over the state: LAMBDA = false, this workgroup's
+// FP64 share of sum_t <psi|P_t|psi> in partials[blockIdx.x]; LAMBDA = true,
+// lam (first: =, else +=) sum_t w_t P_t psi.
+//
+// HBM-bound when the terms are few: a term that flips qubits pairs every
+// amplitude with another one, and read from memory each such term is a sweep
+// of its own (the direct kernels below: 502 us for the 23 ZZ and 24 X terms of a
+// 24-qubit Ising sum, and 524 us for its lambda).  Here a workgroup holds a
+// tile of 2^12 amplitudes in LDS, so all terms that flip only the tile's qubits
+// cost one read of the state: three sweeps of 72 us for that sum, three of 98 us
+// for its lambda (a copy's rate would be 28 and 84).  Each thread has eight amplitudes in
+// registers, j = tid + 512 i, and reads the partners from LDS; signs are
+// parities of the tile base (uniform), the thread and i.  Z terms add up to one
+// weight per amplitude.
+template <bool LAMBDA>
+__global__ __launch_bounds__(kThreads) void terms_kernel(const float2* __restrict__ psi,
+                                                         float2* __restrict__ lam, int n,
+                                                         DevTermMap map,
+                                                         const DevTermTile* __restrict__ terms,
+                                                         int count, int first, double* partials) {
+  constexpr int PER = (1 << kTermTile) / kThreads;
+  __shared__ float2 tile[1 << kTermTile];
+  __shared__ double red[kWaves];
+  const uint32_t tid = threadIdx.x;
+  uint64_t toff = tid & ((1u << kTermLow) - 1u);
+#pragma unroll
+  for (int h = 0; h < 3; ++h) toff |= uint64_t((tid >> (kTermLow + h)) & 1u) << map.hbit[h];
+  uint64_t ioff[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    ioff[i] = (uint64_t(i & 1) << map.hbit[3]) | (uint64_t((i >> 1) & 1) << map.hbit[4]) |
+              (uint64_t((i >> 2) & 1) << map.hbit[5]);
+  static_assert(PER == 8 && kTermLow + 3 == 9 && kTermHigh == 6, "512 threads, eight amplitudes each");
+  const uint64_t ntiles = uint64_t(1) << (n - kTermTile);
+  double total = 0.0;
+  for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const uint64_t base = tile_base(t, map.tilemask, n);
+    float2 a[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) a[i] = psi[base | toff | ioff[i]];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) tile[tid + uint32_t(kThreads * i)] = a[i];
+    __syncthreads();
+    float zw[PER];          // summed weights of the Z terms
+    float ax[PER], ay[PER];  // the others: the value (ax), or lambda's parts
+#pragma unroll
+    for (int i = 0; i < PER; ++i) zw[i] = ax[i] = ay[i] = 0.f;
+    for (int k = 0; k < count; ++k) {
+      kconst<DevTermTile>* T = as_const(terms + k);
+      const uint32_t floc = T->floc, zloc = T->zloc;
+      const float re = T->re, im = T->im;
+      const uint32_t st = (uint32_t(__popcll(base & T->zmask)) + uint32_t(__popc(tid & zloc))) & 1u;
+      if (floc == 0) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          const uint32_t s = st ^ (uint32_t(__popc(uint32_t(kThreads * i) & zloc)) & 1u);
+          zw[i] += __uint_as_float(__float_as_uint(re) ^ (s << 31));
+        }
+        continue;
+      }
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const uint32_t s = st ^ (uint32_t(__popc(uint32_t(kThreads * i) & zloc)) & 1u);
+        const float2 p = tile[(tid + uint32_t(kThreads * i)) ^ floc];
+        const float wr = __uint_as_float(__float_as_uint(re) ^ (s << 31));
+        const float wi = __uint_as_float(__float_as_uint(im) ^ (s << 31));
+        if (LAMBDA) {
+          ax[i] += wr * p.x - wi * p.y;
+          ay[i] += wr * p.y + wi * p.x;
+        } else {
+          const float2 pr = cmul_conj_a(p, a[i]);
+          ax[i] += wr * pr.x - wi * pr.y;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (LAMBDA) {
+        const uint64_t g = base | toff | ioff[i];
+        float2 l = make_float2(ax[i] + zw[i] * a[i].x, ay[i] + zw[i] * a[i].y);
+        if (!first) l = cadd(l, lam[g]);
+        lam[g] = l;
+      } else {
+        total += double(ax[i] + zw[i] * (a[i].x * a[i].x + a[i].y * a[i].y));
+      }
+    }
+    __syncthreads();  // the tile is read before the next one overwrites it
+  }
+  if (!LAMBDA) {
+    const double tot = block_sum(total, red);
+    if (tid == 0) partials[blockIdx.x] = tot;
+  }
+}
+
+// Terms that no tile holds (and states smaller than a tile), straight from memory.
 __global__ __launch_bounds__(kThreads) void expect_kernel(const float2* __restrict__ psi, int n,
-                                                          const DevTermWide* __restrict__ terms,
-                                                          int tb, int te, double* partials) {
+                                                          const DevTermTile* __restrict__ terms,
+                                                          int count, double* partials) {
   __shared__ double red[kWaves];
   const uint64_t N = uint64_t(1) << n;
   double acc = 0.0;
@@ -348,8 +444,8 @@ __global__ __launch_bounds__(kThreads) void expect_kernel(const float2* __restri
        x += uint64_t(gridDim.x) * kThreads) {
     const float2 va = psi[x];
     float part = 0.f;
-    for (int t = tb; t < te; ++t) {
-      const DevTermWide T = terms[t];
+    for (int t = 0; t < count; ++t) {
+      const DevTermTile T = terms[t];
       const float2 pr = cmul_conj_a(psi[x ^ T.fmask], va);
       const float v = T.re * pr.x - T.im * pr.y;
       part += (__popcll(x & T.zmask) & 1) ? -v : v;
@@ -362,17 +458,16 @@ __global__ __launch_bounds__(kThreads) void expect_kernel(const float2* __restri
 
 __global__ __launch_bounds__(kThreads) void lambda_kernel(const float2* __restrict__ psi,
                                                           float2* __restrict__ lam, int n,
-                                                          const DevTermWide* __restrict__ terms,
-                                                          int tb, int te) {
+                                                          const DevTermTile* __restrict__ terms,
+                                                          int count, int first) {
   const uint64_t N = uint64_t(1) << n;
   for (uint64_t y = uint64_t(blockIdx.x) * kThreads + threadIdx.x; y < N;
        y += uint64_t(gridDim.x) * kThreads) {
-    float2 l = make_float2(0.f, 0.f);
-    for (int t = tb; t < te; ++t) {
-      const DevTermWide T = terms[t];
-      const uint64_t x = y ^ T.fmask;
-      float2 w = cmul(make_float2(T.re, T.im), psi[x]);
-      if (__popcll(x & T.zmask) & 1) w = make_float2(-w.x, -w.y);
+    float2 l = first ? make_float2(0.f, 0.f) : lam[y];
+    for (int t = 0; t < count; ++t) {
+      const DevTermTile T = terms[t];
+      float2 w = cmul(make_float2(T.re, T.im), psi[y ^ T.fmask]);
+      if (__popcll(y & T.zmask) & 1) w = make_float2(-w.x, -w.y);
       l = cadd(l, w);
     }
     lam[y] = l;
@@ -411,10 +506,17 @@ __global__ __launch_bounds__(kThreads) void reduce_kernel(const double* __restri
   if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
-// Serial finishing steps (one thread): avoids host round trips between kernels.
-__global__ void finish_expect(const double* sums, float ident, float* out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *out = float(sums[0] + double(ident));
+// One slot's expectation: the groups' partials and the identity terms.
+__global__ __launch_bounds__(kThreads) void finish_expect(const double* __restrict__ partials,
+                                                          int count, float ident, float* out) {
+  __shared__ double red[kWaves];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < count; i += kThreads) s += partials[i];
+  s = block_sum(s, red);
+  if (threadIdx.x == 0) *out = float(s + double(ident));
 }
+
+// Serial finishing steps (one thread): avoids host round trips between kernels.
 
 __global__ void finish_sampled(const double* sums, int count, const float* coefs,
                                const int* shots, float ident, float* out) {
@@ -663,6 +765,7 @@ static void LargeLayout(LargePlan* p, size_t* off_pcols, size_t* off_ident, size
   p->off_ops = off; off = AlignUp(off + p->ops.size() * sizeof(DevOp));
   p->off_mats = off; off = AlignUp(off + (p->mats.size() + kMatCache) * sizeof(cfloat));
   p->off_terms = off; off = AlignUp(off + p->terms.size() * sizeof(DevTermWide));
+  p->off_tile_terms = off; off = AlignUp(off + p->tile_terms.size() * sizeof(DevTermTile));
   *off_pcols = off; off = AlignUp(off + p->param_cols.size() * sizeof(int32_t));
   const size_t nslots = size_t(p->mode == kModeInnerProduct ? p->K : p->O);
   *off_ident = off; off = AlignUp(off + size_t(p->B) * nslots * sizeof(float));
@@ -719,6 +822,7 @@ int LargeUpload(LargePlan* p, void* ws, hipStream_t stream, char* err, int64_t l
   put(p->off_ops, p->ops.data(), p->ops.size() * sizeof(DevOp));
   put(p->off_mats, p->mats.data(), p->mats.size() * sizeof(cfloat));
   put(p->off_terms, p->terms.data(), p->terms.size() * sizeof(DevTermWide));
+  put(p->off_tile_terms, p->tile_terms.data(), p->tile_terms.size() * sizeof(DevTermTile));
   put(o.pcols, p->param_cols.data(), p->param_cols.size() * sizeof(int32_t));
   const size_t nslots = size_t(p->mode == kModeInnerProduct ? p->K : p->O);
   std::vector<float> ident(size_t(p->B) * nslots, 0.0f), coefs(p->terms.size(), 0.0f);
@@ -751,7 +855,7 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
   uint8_t* base = static_cast<uint8_t*>(ws);
   const DevOp* ops = reinterpret_cast<const DevOp*>(base + p->off_ops);
   const float2* mats = reinterpret_cast<const float2*>(base + p->off_mats);
-  const DevTermWide* terms = reinterpret_cast<const DevTermWide*>(base + p->off_terms);
+  const DevTermTile* tile_terms = reinterpret_cast<const DevTermTile*>(base + p->off_tile_terms);
   const int* pcols = reinterpret_cast<const int*>(base + o.pcols);
   const float* coefs = reinterpret_cast<const float*>(base + o.coefs);
   const int* shots = reinterpret_cast<const int*>(base + o.shots);
@@ -868,6 +972,8 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
       continue;
     }
     const int sgrid = int(std::min<uint64_t>(uint64_t(grid), ((uint64_t(1) << n) + 255) / 256));
+    // Term tiles: four workgroups of 32 KiB share a CU.
+    const int tgrid = int(std::min<uint64_t>(1024, uint64_t(1) << std::max(0, n - kTermTile)));
     if (p->mode == kModeInnerProductGrad) {
       // lambda = sum_j g_j |phi_j> in buf2 (AccumulateFusedCircuits,
       // util_qsim.h:421-442), each phi_j simulated in psi's buffer first.
@@ -886,19 +992,27 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
     const float* ident = reinterpret_cast<const float*>(base + o.ident) + size_t(row) * nslots;
     if (p->mode == kModeExpectation || (p->mode == kModeAdjoint && p->with_expectation)) {
       float* exp_base = static_cast<float*>(output);
-      int t = lc.term_begin;
       for (int64_t j = 0; j < nslots; ++j) {
-        const int tb = t;
-        while (t < lc.term_end && p->terms[t].slot == j) ++t;
         float* out = exp_base + size_t(row) * nslots + j;
-        if (t == tb) {
-          hipLaunchKernelGGL(fill_row_f32, dim3(1), dim3(64), 0, stream, out, 1, lc.ident[j]);
-          continue;
+        int count = 0;
+        for (const TermGroup& g : lc.exp_groups[size_t(j)]) {
+          const int cnt = g.end - g.begin;
+          if (g.direct) {
+            hipLaunchKernelGGL(expect_kernel, dim3(sgrid), dim3(kThreads), 0, stream, psi, n,
+                               tile_terms + g.begin, cnt, partials + count);
+            count += sgrid;
+          } else {
+            hipLaunchKernelGGL(terms_kernel<false>, dim3(tgrid), dim3(kThreads), 0, stream, psi,
+                               static_cast<float2*>(nullptr), n, g.map, tile_terms + g.begin, cnt, 0,
+                               partials + count);
+            count += tgrid;
+          }
         }
-        hipLaunchKernelGGL(expect_kernel, dim3(sgrid), dim3(kThreads), 0, stream, psi, n, terms, tb,
-                           t, partials);
-        hipLaunchKernelGGL(reduce_kernel, dim3(1), dim3(kThreads), 0, stream, partials, sgrid, 1, 0, redbuf);
-        hipLaunchKernelGGL(finish_expect, dim3(1), dim3(64), 0, stream, redbuf, lc.ident[j], out);
+        if (count == 0)
+          hipLaunchKernelGGL(fill_row_f32, dim3(1), dim3(64), 0, stream, out, 1, lc.ident[j]);
+        else
+          hipLaunchKernelGGL(finish_expect, dim3(1), dim3(kThreads), 0, stream, partials, count,
+                             lc.ident[j], out);
       }
     }
     if (p->mode == kModeAdjoint || p->mode == kModeInnerProductGrad) {
@@ -909,9 +1023,23 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
       const int width = cplx ? 2 : 1;
       float* grad_base = static_cast<float*>(output) +
                          (p->with_expectation ? size_t(p->B) * size_t(p->O) : 0);
-      if (!cplx)
-        hipLaunchKernelGGL(lambda_kernel, dim3(sgrid), dim3(kThreads), 0, stream, psi, buf2, n, terms,
-                           lc.lam_begin, lc.lam_end);
+      if (!cplx) {
+        int first = 1;
+        for (const TermGroup& g : lc.lam_groups) {
+          const int cnt = g.end - g.begin;
+          if (g.direct)
+            hipLaunchKernelGGL(lambda_kernel, dim3(sgrid), dim3(kThreads), 0, stream, psi, buf2, n,
+                               tile_terms + g.begin, cnt, first);
+          else
+            hipLaunchKernelGGL(terms_kernel<true>, dim3(tgrid), dim3(kThreads), 0, stream, psi, buf2,
+                               n, g.map, tile_terms + g.begin, cnt, first,
+                               static_cast<double*>(nullptr));
+          first = 0;
+        }
+        if (first)  // no terms: lambda = 0
+          hipLaunchKernelGGL(lambda_kernel, dim3(sgrid), dim3(kThreads), 0, stream, psi, buf2, n,
+                             tile_terms, 0, 1);
+      }
       hipLaunchKernelGGL(fill_f64, dim3(1), dim3(256), 0, stream, gacc, int64_t(p->S) * width, 0.0);
       for (const DevPass& ps : lc.rev.passes) {
         PassArgs a{};

@@ -104,6 +104,26 @@ struct alignas(8) DevTermWide {
   int32_t pad;
 };
 
+// A term of the streaming reductions (terms_kernel): its masks, its masks over
+// the bits of a tile, and the coefficient (times i^{nY}).
+struct alignas(8) DevTermTile {
+  uint64_t fmask;
+  uint64_t zmask;
+  uint32_t floc;
+  uint32_t zloc;
+  float re;
+  float im;
+};
+// Tiles of the term reductions: 2^kTermTile amplitudes, the lowest kTermLow
+// qubits (512 contiguous bytes) and kTermHigh others.
+constexpr int kTermTile = 12;
+constexpr int kTermLow = 6;
+constexpr int kTermHigh = kTermTile - kTermLow;
+struct DevTermMap {
+  uint64_t tilemask;
+  uint8_t hbit[kTermHigh + 2];  // the others, ascending
+};
+
 // One pass over a multi-tile state: tile-local bit j <-> global bit tbit[j].
 constexpr int kMaxTile = 14;
 struct alignas(8) DevPass {

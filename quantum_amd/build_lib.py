@@ -40,8 +40,11 @@ def _hipcc():
 
 # Device code: keep SimplifyCFG from sinking the stores of the register
 # engine's per-qubit-position variants into one store through a PHI of
-# addresses, which would demote the register arrays to scratch memory.
-HIP_ONLY = ["-mllvm", "-simplifycfg-sink-common=false"]
+# addresses, which would demote the register arrays to scratch memory, and keep
+# the engine's result tuples whole through PHIs (split into scalars they are
+# copied register by register at every op and spilled).
+HIP_ONLY = ["-mllvm", "-simplifycfg-sink-common=false",
+            "-mllvm", "-amdgpu-codegenprepare-break-large-phis=false"]
 
 
 def _compile(src):

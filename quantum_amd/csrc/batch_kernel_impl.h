@@ -304,8 +304,16 @@ __device__ __forceinline__ void wave_circuit(const BatchArgs& a, int ci, float2*
   const uint32_t N = 1u << n;
   const uint32_t lane = threadIdx.x & 63u;
   // Forward from |0>, final state to P in the natural layout.
-  auto fio = tile_io([](uint32_t x, cf& va, cf&) { va = cf{x == 0 ? 1.f : 0.f, 0.f}; },
-                     [P](uint32_t x, const cf& va, const cf&) { P[x] = make_float2(va.x, va.y); });
+  auto fio = tile_io(
+      [](uint64_t t, const auto& g, auto&& set) {
+        each_reg(g, [&](int r) { set(r, cf{(t | g[r]) == 0 ? 1.f : 0.f, 0.f}, cf{}); });
+      },
+      [P](uint64_t t, const auto& g, auto&& get_a, auto&&) {
+        each_reg(g, [&](int r) {
+          const cf va = get_a(r);
+          P[uint32_t(t | g[r])] = make_float2(va.x, va.y);
+        });
+      });
   reg_run_wave<false>(P, P, n, a.ops, uniform(c.fwd_begin), uniform(c.fwd_end), a.mats, NoAcc(),
                       fio);
   esync<true>();
@@ -317,12 +325,14 @@ __device__ __forceinline__ void wave_circuit(const BatchArgs& a, int ci, float2*
     __threadfence();
     wave_lambda(P, Q, N, a, uniform(c.lam_begin), uniform(c.lam_end));
     auto rio = tile_io(
-        [P, Q](uint32_t x, cf& va, cf& vb) {
-          const float2 u = P[x], v = Q[x];
-          va = cf{u.x, u.y};
-          vb = cf{v.x, v.y};
+        [P, Q](uint64_t t, const auto& g, auto&& set) {
+          each_reg(g, [&](int r) {
+            const uint32_t x = uint32_t(t | g[r]);
+            const float2 u = P[x], v = Q[x];
+            set(r, cf{u.x, u.y}, cf{v.x, v.y});
+          });
         },
-        [](uint32_t, const cf&, const cf&) {});
+        [](uint64_t, const auto&, auto&&, auto&&) {});
     auto acc = [gacc](int, int col, double w, double) { atomicAdd(&gacc[col], 2.0 * w); };
     reg_run_wave<true>(P, Q, n, a.ops, uniform(c.rev_begin), uniform(c.rev_end), a.mats, acc, rio);
     __threadfence();
@@ -348,22 +358,33 @@ __device__ __forceinline__ void tiled_forward(float2* G, int n, const BatchArgs&
     const uint32_t T = 1u << ps.L;
     const uint32_t ntiles = 1u << (n - ps.L);
     for (uint32_t t = 0; t < ntiles; ++t) {
-      const uint64_t base = tile_base(t, ps.tilemask, n);
+      const uint64_t base = tile_base_of(t, ps);
       auto gidx = [&](uint32_t j) -> uint64_t {
         return use_tab ? tile_index_tab(base, j, ps.nlow, tab) : tile_index(base, j, ps);
       };
       // Register engine: the tile goes straight between G and the registers.
       auto io = tile_io_indexed(
-          gidx,
-          [&](uint64_t g, cf& va, cf&) {
+          [&](uint32_t j) -> uint64_t {
+            return use_tab ? tile_index_tab(0, j, ps.nlow, tab) : tile_index(0, j, ps);
+          },
+          [&](uint64_t th, const auto& g, auto&& set) {
+            const uint64_t x = base | th;
             if (first) {
-              va = cf{g == 0 ? 1.f : 0.f, 0.f};
+              each_reg(g, [&](int r) { set(r, cf{(x | g[r]) == 0 ? 1.f : 0.f, 0.f}, cf{}); });
             } else {
-              const float2 v = G[g];
-              va = cf{v.x, v.y};
+              each_reg(g, [&](int r) {
+                const float2 v = G[x + g[r]];
+                set(r, cf{v.x, v.y}, cf{});
+              });
             }
           },
-          [&](uint64_t g, const cf& va, const cf&) { G[g] = make_float2(va.x, va.y); });
+          [&](uint64_t th, const auto& g, auto&& get_a, auto&&) {
+            const uint64_t x = base | th;
+            each_reg(g, [&](int r) {
+              const cf va = get_a(r);
+              G[x + g[r]] = make_float2(va.x, va.y);
+            });
+          });
       if (reg_run_any<false, RMAX>(A, A, ps.L, a.ops, ps.op_begin, ps.op_end, mc, NoAcc(), io))
         continue;
       if (first) {
@@ -401,20 +422,28 @@ __device__ __forceinline__ void tiled_reverse(float2* G, float2* Lg, int n, cons
     const uint32_t T = 1u << ps.L;
     const uint32_t ntiles = 1u << (n - ps.L);
     for (uint32_t t = 0; t < ntiles; ++t) {
-      const uint64_t base = tile_base(t, ps.tilemask, n);
+      const uint64_t base = tile_base_of(t, ps);
       auto gidx = [&](uint32_t j) -> uint64_t {
         return use_tab ? tile_index_tab(base, j, ps.nlow, tab) : tile_index(base, j, ps);
       };
       auto io = tile_io_indexed(
-          gidx,
-          [&](uint64_t g, cf& va, cf& vb) {
-            const float2 u = G[g], v = Lg[g];
-            va = cf{u.x, u.y};
-            vb = cf{v.x, v.y};
+          [&](uint32_t j) -> uint64_t {
+            return use_tab ? tile_index_tab(0, j, ps.nlow, tab) : tile_index(0, j, ps);
           },
-          [&](uint64_t g, const cf& va, const cf& vb) {
-            G[g] = make_float2(va.x, va.y);
-            Lg[g] = make_float2(vb.x, vb.y);
+          [&](uint64_t th, const auto& g, auto&& set) {
+            const uint64_t x = base | th;
+            each_reg(g, [&](int r) {
+              const float2 u = G[x + g[r]], v = Lg[x + g[r]];
+              set(r, cf{u.x, u.y}, cf{v.x, v.y});
+            });
+          },
+          [&](uint64_t th, const auto& g, auto&& get_a, auto&& get_b) {
+            const uint64_t x = base | th;
+            each_reg(g, [&](int r) {
+              const cf va = get_a(r), vb = get_b(r);
+              G[x + g[r]] = make_float2(va.x, va.y);
+              Lg[x + g[r]] = make_float2(vb.x, vb.y);
+            });
           });
       auto acc = [gacc](int, int col, double w, double) { atomicAdd(&gacc[col], 2.0 * w); };
       if (reg_run_any<true>(A, B, ps.L, a.ops, ps.op_begin, ps.op_end, mc, acc, io)) continue;

@@ -64,11 +64,12 @@ struct PassArgs {
 // CPLX (two-buffer passes only): each derivative also accumulates the
 // imaginary part of <dG psi|lambda>, written to the partial slot after the
 // real part's.
-// WIDE: one-state passes on 14-qubit tiles (128 KiB of LDS, one workgroup
-// per CU) with the five-register-qubit engine and the VGPR budget of two
-// waves per SIMD.
-template <bool TWO, bool CPLX = false, bool WIDE = false>
-__global__ __launch_bounds__(kThreads, (TWO || WIDE) ? 2 : 4) void pass_kernel(PassArgs a) {
+// ENG: register qubits of the engine that runs the pass, 0 for the LDS path; one
+// kernel each, so that no engine is held to another's registers.  5: one-state passes
+// on 14-qubit tiles (128 KiB of LDS, one workgroup per CU) with the VGPR budget of
+// two waves per SIMD.
+template <bool TWO, bool CPLX, int ENG>
+__global__ __launch_bounds__(kThreads, (TWO || ENG == 5) ? 2 : 4) void pass_kernel(PassArgs a) {
   constexpr int kPacc = TWO ? (CPLX ? 2 : 1) * kMaxPassDerivs : 1;
   extern __shared__ float2 lds[];
   __shared__ double red[kWaves];
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(kThreads, (TWO || WIDE) ? 2 : 4) void pass_kernel(P
     for (int k = tid; k < kPacc; k += kThreads) pacc[k] = 0.0;
   __syncthreads();
   for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const uint64_t base = tile_base(t, ps.tilemask, a.n);
+    const uint64_t base = tile_base_of(t, ps);
     auto gidx = [&](uint32_t j) -> uint64_t {
       return use_tab ? tile_index_tab(base, j, nlow, tab) : tile_index(base, j, ps);
     };
@@ -100,31 +101,42 @@ __global__ __launch_bounds__(kThreads, (TWO || WIDE) ? 2 : 4) void pass_kernel(P
       atomicAdd(&pacc[slot], w);
       if (CPLX) atomicAdd(&pacc[kMaxPassDerivs + slot], v);
     };
-    // Register engine: the tile goes straight between memory and registers.
-    auto io = tile_io_indexed(
-        gidx,
-        [&](uint64_t g, cf& va, cf& vb) {
-          if (TWO) {
-            const float2 u = a.psi[g], v = a.lam[g];
-            va = cf{u.x, u.y};
-            vb = cf{v.x, v.y};
-          } else if (a.init) {
-            va = cf{g == 0 ? 1.f : 0.f, 0.f};
-          } else {
-            const float2 u = a.src[g];
-            va = cf{u.x, u.y};
-          }
-        },
-        [&](uint64_t g, const cf& va, const cf& vb) {
-          if (TWO) {
-            a.psi[g] = make_float2(va.x, va.y);
-            a.lam[g] = make_float2(vb.x, vb.y);
-          } else {
-            a.dst[g] = make_float2(va.x, va.y);
-          }
-        });
-    if (reg_run_any<TWO, WIDE ? 5 : 4>(A, Bf, L, a.ops, ps.op_begin, ps.op_end, mc, acc, io))
+    if constexpr (ENG > 0) {
+      // The tile goes straight between memory and registers.
+      auto io = tile_io_indexed(
+          [&](uint32_t j) -> uint64_t {
+            return use_tab ? tile_index_tab(0, j, nlow, tab) : tile_index(0, j, ps);
+          },
+          [&](uint64_t th, const auto& g, auto&& set) {
+            const uint64_t x = base | th;
+            if (TWO) {
+              each_reg(g, [&](int r) {
+                const float2 u = a.psi[x + g[r]], v = a.lam[x + g[r]];
+                set(r, cf{u.x, u.y}, cf{v.x, v.y});
+              });
+            } else if (a.init) {
+              each_reg(g, [&](int r) { set(r, cf{(x | g[r]) == 0 ? 1.f : 0.f, 0.f}, cf{}); });
+            } else {
+              each_reg(g, [&](int r) {
+                const float2 u = a.src[x + g[r]];
+                set(r, cf{u.x, u.y}, cf{});
+              });
+            }
+          },
+          [&](uint64_t th, const auto& g, auto&& get_a, auto&& get_b) {
+            const uint64_t x = base | th;
+            each_reg(g, [&](int r) {
+              const cf va = get_a(r);
+              (TWO ? a.psi : a.dst)[x + g[r]] = make_float2(va.x, va.y);
+              if (TWO) {
+                const cf vb = get_b(r);
+                a.lam[x + g[r]] = make_float2(vb.x, vb.y);
+              }
+            });
+          });
+      reg_run<ENG, TWO, false>(A, Bf, L, a.ops, ps.op_begin, ps.op_end, mc, acc, io);
       continue;
+    }
     if (TWO) {
       tile_gather2(A, Bf, a.psi, a.lam, T, gidx);
     } else if (a.init) {
@@ -180,6 +192,25 @@ __global__ __launch_bounds__(kThreads, (TWO || WIDE) ? 2 : 4) void pass_kernel(P
       }
       pl += op.nderiv;
     }
+  }
+}
+
+// The engine a pass was planned for (its op list starts with a remap, or not).
+int pass_engine(const LargePlan& p, const DevPass& ps) {
+  if (ps.op_begin >= ps.op_end || p.ops[ps.op_begin].type != kOpRemap) return 0;
+  return RegBitsForTile(ps.L, 5);
+}
+template <bool TWO, bool CPLX>
+void launch_pass(const PassArgs& a, int eng, int grid, size_t lds, hipStream_t stream) {
+  if (eng == 5) {
+    if constexpr (!TWO)
+      hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 5>), dim3(grid), dim3(kThreads), lds, stream, a);
+  } else if (eng == 4) {
+    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 4>), dim3(grid), dim3(kThreads), lds, stream, a);
+  } else if (eng == 3) {
+    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 3>), dim3(grid), dim3(kThreads), lds, stream, a);
+  } else {
+    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 0>), dim3(grid), dim3(kThreads), lds, stream, a);
   }
 }
 
@@ -907,8 +938,7 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
       const uint64_t ntiles = uint64_t(1) << (n - ps.L);
       const int g = int(std::min<uint64_t>(ntiles, uint64_t(grid)));
       const size_t lds = (size_t(1) << ps.L) * sizeof(float2);
-      if (ps.L > 13) hipLaunchKernelGGL((pass_kernel<false, false, true>), dim3(g), dim3(kThreads), lds, stream, a);
-      else hipLaunchKernelGGL(pass_kernel<false>, dim3(g), dim3(kThreads), lds, stream, a);
+      launch_pass<false, false>(a, pass_engine(*p, ps), g, lds, stream);
       first = false;
     }
     if (first) {  // no ops at all: still need |0>
@@ -1053,8 +1083,8 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
         const uint64_t ntiles = uint64_t(1) << (n - ps.L);
         const int g = int(std::min<uint64_t>(ntiles, uint64_t(grid)));
         const size_t lds = 2 * (size_t(1) << ps.L) * sizeof(float2);
-        if (cplx) hipLaunchKernelGGL((pass_kernel<true, true>), dim3(g), dim3(kThreads), lds, stream, a);
-        else hipLaunchKernelGGL((pass_kernel<true, false>), dim3(g), dim3(kThreads), lds, stream, a);
+        if (cplx) launch_pass<true, true>(a, pass_engine(*p, ps), g, lds, stream);
+        else launch_pass<true, false>(a, pass_engine(*p, ps), g, lds, stream);
         // Partial slots of a pass are contiguous [s0, s0 + nd) (numbered at planning).
         int s0 = -1, nd = 0;
         for (int i = ps.op_begin; i < ps.op_end; ++i) {

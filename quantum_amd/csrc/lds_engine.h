@@ -49,7 +49,7 @@ __device__ __forceinline__ DevOp desc_unpack(uint32_t word) {
   o.type = uint8_t(w[0]);
   o.k = uint8_t(w[0] >> 8);
   o.nderiv = uint8_t(w[0] >> 16);
-  o.pad0 = 0;
+  o.code = uint8_t(w[0] >> 24);
   o.q[0] = uint8_t(w[1]);
   o.q[1] = uint8_t(w[1] >> 8);
   o.q[2] = uint8_t(w[1] >> 16);

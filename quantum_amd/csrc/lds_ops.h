@@ -63,7 +63,7 @@ __device__ __forceinline__ DevOp load_op(const DevOp* p) {
   o.type = uint8_t(w[0]);
   o.k = uint8_t(w[0] >> 8);
   o.nderiv = uint8_t(w[0] >> 16);
-  o.pad0 = 0;
+  o.code = uint8_t(w[0] >> 24);
   o.q[0] = uint8_t(w[1]);
   o.q[1] = uint8_t(w[1] >> 8);
   o.q[2] = uint8_t(w[1] >> 16);
@@ -362,6 +362,19 @@ __device__ __forceinline__ uint64_t tile_base(uint64_t t, uint64_t tm, int n) {
       t >>= 1;
     }
   }
+  return base;
+}
+
+// The same for a pass's tile, whose low bits are the nlow lowest: t shifted past
+// them, with a zero inserted at each of the few other tile bits.
+__device__ __forceinline__ uint64_t tile_base_of(uint64_t t, const DevPass& p) {
+  uint64_t base = t << p.nlow;
+#pragma unroll
+  for (int h = 0; h < kMaxTile; ++h)
+    if (h >= p.nlow && h < p.L) {
+      const uint64_t low = (uint64_t(1) << p.tbit[h]) - 1u;
+      base = ((base & ~low) << 1) | (base & low);
+    }
   return base;
 }
 

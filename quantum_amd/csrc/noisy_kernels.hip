@@ -268,8 +268,17 @@ __device__ __forceinline__ void wave_chunk(const NoisyArgs& a, const DevChunk& c
   const int fb = uniform(c.fwd_begin), fe = uniform(c.fwd_end);
   if (fb < fe) {
     auto fio = tile_io(
-        [N](uint32_t x, cf& va, cf&) { va = cf{(x & (N - 1u)) == 0u ? 1.f : 0.f, 0.f}; },
-        [P](uint32_t x, const cf& va, const cf&) { P[x] = make_float2(va.x, va.y); });
+        [N](uint64_t t, const auto& g, auto&& set) {
+          each_reg(g, [&](int r) {
+            set(r, cf{(uint32_t(t | g[r]) & (N - 1u)) == 0u ? 1.f : 0.f, 0.f}, cf{});
+          });
+        },
+        [P](uint64_t t, const auto& g, auto&& get_a, auto&&) {
+          each_reg(g, [&](int r) {
+            const cf va = get_a(r);
+            P[uint32_t(t | g[r])] = make_float2(va.x, va.y);
+          });
+        });
     GlobalMats gm{a.mats};
     reg_run<kWaveRegBits, false, true>(P, P, kWaveMaxQubits, a.ops, fb, fe, gm, nd, fio);
   } else {

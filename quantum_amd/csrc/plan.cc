@@ -321,6 +321,74 @@ void InsertRemapsR(std::vector<DevOp>* ops, size_t begin, int L, int R) {
     }
     while (first < n && done[first]) ++first;
   }
+  AnnotateEngine(ops, begin, L, R);
+}
+
+void AnnotateEngine(std::vector<DevOp>* ops, size_t begin, int L, int R) {
+  std::vector<int> slots;
+  uint32_t mask = 0;
+  auto pack = [&]() {
+    uint32_t p = 0;
+    for (int j = 0; j < R; ++j) p |= uint32_t(slots[size_t(j)]) << (4 * j);
+    return p;
+  };
+  auto slot_of = [&](int q) {
+    for (int j = 0; j < R; ++j)
+      if (slots[size_t(j)] == q) return j;
+    return R;
+  };
+  // Tile positions of the wavefront-index bits: the non-register positions
+  // after the six lowest (the lane bits).
+  auto wave_positions = [L](uint32_t m) {
+    uint32_t rest = ((1u << L) - 1u) & ~m;
+    for (int k = 0; k < 6; ++k) rest &= rest - 1u;
+    return rest;
+  };
+  for (size_t i = begin; i < ops->size(); ++i) {
+    DevOp& o = (*ops)[i];
+    if (o.type == kOpRemap) {
+      if (i > begin) {
+        o.cval = pack();
+        if (wave_positions(mask) == wave_positions(o.cmask)) o.code = kCodeLocal;
+      }
+      mask = o.cmask;
+      slots.clear();
+      for (int b = 0; b < L; ++b)
+        if (mask >> b & 1) slots.push_back(b);
+      o.dmat[0] = pack();
+      continue;
+    }
+    o.q[2] = o.q[3] = 0;
+    for (int j = 0; j < R; ++j) {
+      if (o.cmask >> slots[size_t(j)] & 1) o.q[2] |= uint8_t(1 << j);
+      if (o.cval >> slots[size_t(j)] & 1) o.q[3] |= uint8_t(1 << j);
+    }
+    if (o.type == kOpDiag) {
+      o.code = uint8_t(slot_of(o.q[0]) | (o.k > 1 ? slot_of(o.q[1]) : R) << 3);
+      continue;
+    }
+    int a = slot_of(o.q[0]);
+    if (o.type == kOpChannel) {
+      o.code = uint8_t(a);
+      continue;
+    }
+    int b;
+    bool swap;
+    if (o.k > 1) {
+      b = slot_of(o.q[1]);
+      swap = a > b;
+    } else {
+      swap = a != 0;
+      b = a == 0 ? 1 : 0;
+    }
+    const int lo = std::min(a, b), hi = std::max(a, b);
+    o.code = uint8_t((lo * (2 * R - lo - 1) / 2 + (hi - lo - 1)) | (swap ? kCodeSwap : 0));
+    std::vector<int> next{slots[size_t(lo)], slots[size_t(hi)]};
+    for (int j = 0; j < R; ++j)
+      if (j != lo && j != hi) next.push_back(slots[size_t(j)]);
+    slots.swap(next);
+  }
+  (*ops)[begin].dmat[1] = pack();
 }
 
 bool KindDiagonal(GateKind kind) {

@@ -112,6 +112,18 @@ int GetReverseFusion();
 void InsertRemaps(std::vector<DevOp>* ops, size_t begin, int L, int max_r = 4);
 // The same with an explicit register-qubit count R (wave mode).
 void InsertRemapsR(std::vector<DevOp>* ops, size_t begin, int L, int R);
+// Follow the register slots through the list (InsertRemapsR calls it last) and
+// store what each op meets:
+//   remap     dmat[0]: the new slots' tile bits (4 bits each, ascending); cval: the
+//             old slots' (not the first); code kCodeLocal: no qubit of the
+//             wavefront index moves.  The first remap's dmat[1]: the slots at the end.
+//   others    q[2], q[3]: controls among the slots and their values
+//   diagonal  code: slot of q[0] | slot of q[1] << 3 (R: a thread bit, or no target)
+//   channel   code: slot of q[0]
+//   dense,    code: number of the slot pair, in order, and kCodeSwap.  A one-qubit
+//   param     op takes slot 0, or slots 0 and its own, along.
+// A dense or parameterised op leaves its pair in slots 0 and 1, the others after it.
+void AnnotateEngine(std::vector<DevOp>* ops, size_t begin, int L, int R);
 
 // Planner tuning (process-wide; 0 = default): register engine on/off and the
 // streaming path's tile qubits for one- and two-state passes.

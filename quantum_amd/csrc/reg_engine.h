@@ -1,22 +1,36 @@
 // Register-resident gate engine for a 2^L-amplitude state tile held in LDS.
 //
 // A workgroup of 512 threads keeps the tile in VGPRs: each thread holds 2^R
-// amplitudes (R = L - 9, 3..4) whose indices differ only in R "register
+// amplitudes (R = L - 9, 3..5) whose indices differ only in R "register
 // qubits"; the thread index fills the other L - R bits.  Ops whose targets
 // are register qubits (and diagonal ops on any qubits, with controls on any
 // qubits) are applied in registers with no LDS traffic and no barrier.  The
 // host planner splits the op list into segments whose non-diagonal targets
-// fit R qubits and starts each with a kOpRemap op carrying the segment's
-// register-qubit mask; a remap writes the registers back to LDS and reloads
-// them in the new layout (two barriers).  Between remaps LDS holds the tile in
-// a swizzled layout (x ^ ((x >> 4) & 15)) so that the strided register loads
-// and stores of a wavefront are spread over the LDS banks; on entry and exit
-// the layout is the natural one.
+// fit R qubits and starts each with a kOpRemap op; a remap writes the registers
+// to LDS and reloads them in the new layout (two barriers).  Between remaps LDS
+// holds the tile in a swizzled layout (x ^ ((x >> 4) & 15)) so that the strided
+// register loads and stores of a wavefront are spread over the LDS banks; on
+// entry and exit the layout is the natural one.
+//
+// The amplitudes of a thread are kept as MFMA result tuples (Regs): register
+// index i is element i & 3 of tuple i >> 2, and each index bit ("slot") stands
+// for one register qubit.  A two-qubit op reads its operands from any two slots
+// and writes whole result tuples, whose two in-tuple slots are its targets: it
+// permutes the slots instead of moving registers, and goes from one set of
+// registers to another, so the op loop has two halves, one per set.  (In place,
+// with fixed slots, every op ended in 64 register moves beside its 64 MFMAs.)
+// The planner knows the slots at every op and stores in each descriptor which
+// code path it takes (AnnotateEngine), so the device decodes nothing.
+//
+// Bound by instruction issue: per tile of a 28-qubit pass (13 qubits, 8.4 two-qubit
+// ops and 2.8 remaps) a wavefront issues 1226 VALU instructions, 535 of them MFMA,
+// and 939 SALU (in place, and with slots and layouts decoded on the device: 2062 and
+// 1954), and the pass takes 1.41 ms (1.83 ms); copying the state takes 0.89 ms.
 //
 // Op matrices are read from an LDS window over the plan's matrix array,
-// refilled when an op's matrices fall outside it.  Parameterised ops (reverse sweep) accumulate their FP64
-// gradient partials per thread, reduce them across the wavefront and hand the
-// sum to the caller's accumulator.
+// refilled when an op's matrices fall outside it.  Parameterised ops (reverse
+// sweep) accumulate their FP64 gradient partials per thread, reduce them across
+// the wavefront and hand the sum to the caller's accumulator.
 #pragma once
 
 #include <type_traits>
@@ -108,62 +122,47 @@ __host__ __device__ constexpr int ins0(int g, int j) {
   return ((g >> j) << (j + 1)) | (g & ((1 << j) - 1));
 }
 
+// ------------------------------------------------------------------ registers
 template <int R>
-struct RegMap {
-  uint32_t rpos[R];  // register qubit positions, ascending (wave-uniform)
-  uint32_t mask;     // wave-uniform
-  uint32_t tbase;    // this thread's bits on the non-register positions
+struct Regs {
+  mf4 re[1 << (R - 2)], im[1 << (R - 2)];
+  __device__ __forceinline__ cf get(int i) const { return cf{re[i >> 2][i & 3], im[i >> 2][i & 3]}; }
+  __device__ __forceinline__ void set(int i, cf v) {
+    re[i >> 2][i & 3] = v.x;
+    im[i >> 2][i & 3] = v.y;
+  }
 };
 
-// Tile index of register i (compile-time i) relative to tbase.
-template <int R>
-__device__ __forceinline__ uint32_t rdep(const RegMap<R>& m, int i) {
-  uint32_t o = 0;
-#pragma unroll
-  for (int j = 0; j < R; ++j)
-    if ((i >> j) & 1) o |= 1u << m.rpos[j];
-  return o;
+// Tile bit of slot j in a packed slot map (kOpRemap; 4 bits per slot).
+__device__ __forceinline__ uint32_t slot_bit(uint32_t slots, int j) {
+  return 1u << ((slots >> (4 * j)) & 15u);
 }
 
-template <int R, bool WAVE = false>
-__device__ __forceinline__ void make_map(RegMap<R>& m, uint32_t mask, int L) {
-  mask = uint32_t(uniform(int(mask)));
-  m.mask = mask;
-  uint32_t mm = mask;
+// This thread's bits on the non-register positions of an L-qubit tile: its
+// index with zeros inserted at the register positions (slots of a fresh map
+// ascend).  Wave mode: the lane; lanes past 2^(L - R) replicate a lane below.
+template <int R, bool WAVE>
+__device__ __forceinline__ uint32_t thread_base(uint32_t slots, int L) {
+  uint32_t x = (WAVE ? (threadIdx.x & 63u) : threadIdx.x) & ((1u << (L - R)) - 1u);
+  asm volatile("" : "+v"(x));  // not kept in registers from remap to remap
 #pragma unroll
-  for (int j = 0; j < R; ++j) {
-    m.rpos[j] = mm ? uint32_t(__builtin_ctz(mm)) : 0u;  // the planner always sets R bits
-    mm &= mm - 1;
-  }
-  // Wave mode: the lane id supplies the L - R <= 6 thread bits; lanes whose
-  // higher bits are set replicate a lane below them.
-  const uint32_t tid = WAVE ? (threadIdx.x & 63u) : threadIdx.x;
-  uint32_t tb = 0;
-  int k = 0;
-  for (int p = 0; p < L; ++p) {
-    if (!((mask >> p) & 1u)) {
-      tb |= ((tid >> k) & 1u) << p;
-      ++k;
-    }
-  }
-  m.tbase = tb;
+  for (int j = 0; j < R; ++j) x = insert_zero(x, (slots >> (4 * j)) & 15u);
+  return x;
 }
 
-// Byte offsets in LDS of the 2^R registers of this thread.  Register i's
-// index is tbase | rdep(i) = tbase ^ (XOR of bit(rpos[j]) over the set bits j
-// of i), and the swizzle is XOR-linear (swz(a ^ b) = swz(a) ^ swz(b)), so
-// offset(i) = offset(i without its highest bit h) ^ sb[h]: one XOR per
-// register after R per-map terms.
+// Byte offsets in LDS of the 2^R registers: register i's index is tbase XOR
+// the bits of its set slots, and the swizzle is XOR-linear, so each offset is
+// one XOR from the one without its highest bit.
 template <int R>
-__device__ __forceinline__ void reg_offsets(const RegMap<R>& m, bool swizzled,
+__device__ __forceinline__ void reg_offsets(uint32_t tbase, uint32_t slots, bool swizzled,
                                             uint32_t (&off)[1 << R]) {
   uint32_t sb[R];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const uint32_t b = 1u << m.rpos[j];
+    const uint32_t b = slot_bit(slots, j);
     sb[j] = (swizzled ? swz(b) : b) << 3;
   }
-  off[0] = (swizzled ? swz(m.tbase) : m.tbase) << 3;
+  off[0] = (swizzled ? swz(tbase) : tbase) << 3;
 #pragma unroll
   for (int i = 1; i < (1 << R); ++i) {
     const int h = 31 - __builtin_clz(uint32_t(i));
@@ -172,462 +171,243 @@ __device__ __forceinline__ void reg_offsets(const RegMap<R>& m, bool swizzled,
 }
 
 template <int R>
-__device__ __forceinline__ void reg_load(cf (&a)[1 << R], const float2* __restrict__ S,
-                                         const RegMap<R>& m, bool swizzled) {
-  uint32_t off[1 << R];
-  reg_offsets<R>(m, swizzled, off);
+__device__ __forceinline__ void reg_load(Regs<R>& a, const float2* __restrict__ S,
+                                         const uint32_t (&off)[1 << R]) {
   const char* base = reinterpret_cast<const char*>(S);
 #pragma unroll
   for (int i = 0; i < (1 << R); ++i) {
     const float2 v = *reinterpret_cast<const float2*>(base + off[i]);
-    a[i] = cf{v.x, v.y};
+    a.set(i, cf{v.x, v.y});
   }
 }
-
 template <int R>
-__device__ __forceinline__ void reg_store(const cf (&a)[1 << R], float2* __restrict__ S,
-                                          const RegMap<R>& m, bool swizzled) {
-  uint32_t off[1 << R];
-  reg_offsets<R>(m, swizzled, off);
+__device__ __forceinline__ void reg_store(const Regs<R>& a, float2* __restrict__ S,
+                                          const uint32_t (&off)[1 << R]) {
   char* base = reinterpret_cast<char*>(S);
 #pragma unroll
-  for (int i = 0; i < (1 << R); ++i)
-    *reinterpret_cast<float2*>(base + off[i]) = make_float2(a[i].x, a[i].y);
+  for (int i = 0; i < (1 << R); ++i) {
+    const cf v = a.get(i);
+    *reinterpret_cast<float2*>(base + off[i]) = make_float2(v.x, v.y);
+  }
 }
 
 // ------------------------------------------------------------------ dense ops
-template <int R, int J, bool DAG, bool BOTH, bool CTRL>
-__device__ __forceinline__ void reg_dense1_c(cf (&a)[1 << R], cf (&b)[1 << R],
-                                             const float2* __restrict__ M, const RegMap<R>& m,
-                                             uint32_t cmask, uint32_t cval) {
-  cf u00 = ldm(M, 0), u01 = ldm(M, 1), u10 = ldm(M, 2), u11 = ldm(M, 3);
-  if (DAG) {
-    const cf t = u01;
-    u00 = cconj(u00);
-    u01 = cconj(u10);
-    u10 = cconj(t);
-    u11 = cconj(u11);
-  }
+// A operands of an op's matrix.  sw: the group index has the op's two index
+// bits exchanged (the planner gives targets to slots in either order).  A
+// one-qubit matrix acts on group bit t, the identity on the other.
+template <bool DAG>
+__device__ __forceinline__ void engine_rows(const float2* __restrict__ M, const DevOp& op,
+                                            MfmaRows& r) {
+  const uint32_t code = op.code;
+  uint32_t l = threadIdx.x & 3u;
+  asm volatile("" : "+v"(l));  // not kept in registers from op to op
+  if (op.k == 1) {
+    const int t = (code & kCodeSwap) ? 1 : 0;
+    const int row = int(l);
+    const int rt = (row >> t) & 1, ro = (row >> (1 - t)) & 1;
+    cf m[2];
 #pragma unroll
-  for (int g = 0; g < (1 << (R - 1)); ++g) {
-    constexpr int one = 1 << J;
-    const int i0 = ins0(g, J);
-    if (CTRL && (((m.tbase | rdep(m, i0)) & cmask) != cval)) continue;
-    const cf v0 = a[i0], v1 = a[i0 | one];
-    a[i0] = cmac(cmulr(u00, v0), u01, v1);
-    a[i0 | one] = cmac(cmulr(u10, v0), u11, v1);
-    if (BOTH) {
-      const cf w0 = b[i0], w1 = b[i0 | one];
-      b[i0] = cmac(cmulr(u00, w0), u01, w1);
-      b[i0 | one] = cmac(cmulr(u10, w0), u11, w1);
+    for (int c = 0; c < 2; ++c) {
+      m[c] = ldm(M, DAG ? c * 2 + rt : rt * 2 + c);
+      if (DAG) m[c].y = -m[c].y;
     }
-  }
-}
-
-template <int R, int J0, int J1>
-__device__ __forceinline__ void group_idx(int g, int (&idx)[4]) {
-  const int i0 = ins0(ins0(g, J0), J1);
 #pragma unroll
-  for (int s = 0; s < 4; ++s) idx[s] = i0 | ((s & 1) << J0) | ((s >> 1) << J1);
-}
-
-template <int R, int J0, int J1, bool DAG, bool BOTH, bool CTRL>
-__device__ __forceinline__ void reg_dense2_c(cf (&a)[1 << R], cf (&b)[1 << R],
-                                             const float2* __restrict__ M, const RegMap<R>& m,
-                                             uint32_t cmask, uint32_t cval) {
-  if constexpr (!CTRL) {
-    MfmaRows rows;
-    mfma_rows<DAG>(M, rows);
-#pragma unroll
-    for (int g = 0; g < (1 << (R - 2)); ++g) {
-      int idx[4];
-      group_idx<R, J0, J1>(g, idx);
-      mf4 dr, di;
-      mfma_apply(a, idx, rows, dr, di);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) a[idx[r]] = cf{dr[r], di[r]};
-      if (BOTH) {
-        mfma_apply(b, idx, rows, dr, di);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) b[idx[r]] = cf{dr[r], di[r]};
-      }
+    for (int k = 0; k < 4; ++k) {
+      const bool same = ((k >> (1 - t)) & 1) == ro;
+      const cf v = ((k >> t) & 1) ? m[1] : m[0];
+      r.gr[k] = same ? v.x : 0.f;
+      r.gi[k] = same ? v.y : 0.f;
+      r.ngi[k] = -r.gi[k];
     }
     return;
   }
-  cf u[16];
+  const bool sw = (code & kCodeSwap) != 0;
+  const uint32_t row = sw ? ((l & 1u) << 1 | l >> 1) : l;
+  const int k1 = sw ? 2 : 1;
+  const float2* base = M + (DAG ? row : row * 4u);
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int k = 0; k < 4; ++k) {
+    const int c = k == 1 ? k1 : k == 2 ? 3 - k1 : k;
+    // (G^dag)[row][c] = conj(G[c][row]).
+    const cf v = ldm(base, DAG ? c * 4 : c);
+    r.gr[k] = v.x;
+    r.gi[k] = DAG ? -v.y : v.y;
+    r.ngi[k] = -r.gi[k];
+  }
+}
+
+// Group g of slots (SA, SB): the register indices of its four amplitudes.
+template <int SA, int SB>
+__device__ __forceinline__ void group_idx(int g, int (&idx)[4]) {
+  const int i0 = ins0(ins0(g, SA), SB);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) u[r * 4 + c] = DAG ? cconj(ldm(M, c * 4 + r)) : ldm(M, r * 4 + c);
+  for (int s = 0; s < 4; ++s) idx[s] = i0 | ((s & 1) << SA) | ((s >> 1) << SB);
+}
+template <int R, int SA, int SB>
+__device__ __forceinline__ void group_product(const Regs<R>& a, int g, const MfmaRows& m, mf4& dr,
+                                              mf4& di) {
+  int idx[4];
+  group_idx<SA, SB>(g, idx);
+  dr = mf4{0.f, 0.f, 0.f, 0.f};
+  di = mf4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float x = a.get(idx[k]).x;
+    dr = mfma4(m.gr[k], x, dr);
+    di = mfma4(m.gi[k], x, di);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float y = a.get(idx[k]).y;
+    dr = mfma4(m.ngi[k], y, dr);
+    di = mfma4(m.gr[k], y, di);
+  }
+}
+
+// Does register i (slots before the op) satisfy the op's controls?  ok: the
+// thread's part.
+__device__ __forceinline__ bool ctrl_ok(const DevOp& op, bool ok, int i) {
+  return ok && (uint32_t(i) & op.q[2]) == op.q[3];
+}
+
+// out <- M in (or M^dagger in) on slots (SA, SB); out's slots are SA, SB, then the
+// others in order.
+template <int R, int SA, int SB>
+__device__ __forceinline__ void reg_dense(const Regs<R>& in, Regs<R>& out, const MfmaRows& m,
+                                          const DevOp& op, bool ok) {
+#pragma unroll
+  for (int g = 0; g < (1 << (R - 2)); ++g) group_product<R, SA, SB>(in, g, m, out.re[g], out.im[g]);
+  if (op.cmask) {
+#pragma unroll
+    for (int g = 0; g < (1 << (R - 2)); ++g) {
+      int idx[4];
+      group_idx<SA, SB>(g, idx);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (!ctrl_ok(op, ok, idx[s])) out.set(g * 4 + s, in.get(idx[s]));
+    }
+  }
+}
+
+// Derivative d of a parameterised op: this thread's <dG u | lam> with u after the
+// op (out's slots) and lam before it (in's slots).
+template <int R, int SA, int SB>
+__device__ __forceinline__ void reg_deriv(const Regs<R>& u, const Regs<R>& lam, const MfmaRows& m,
+                                          const DevOp& op, bool ok, float& part, float& part_im) {
+  part = part_im = 0.f;
 #pragma unroll
   for (int g = 0; g < (1 << (R - 2)); ++g) {
-    const int i0 = ins0(ins0(g, J0), J1);
-    if (CTRL && (((m.tbase | rdep(m, i0)) & cmask) != cval)) continue;
+    mf4 dr, di;
+    group_product<R, 0, 1>(u, g, m, dr, di);
     int idx[4];
+    group_idx<SA, SB>(g, idx);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) idx[s] = i0 | ((s & 1) << J0) | ((s >> 1) << J1);
-    cf v[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) v[s] = a[idx[s]];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      cf acc = cmulr(u[r * 4], v[0]);
-#pragma unroll
-      for (int c = 1; c < 4; ++c) acc = cmac(acc, u[r * 4 + c], v[c]);
-      a[idx[r]] = acc;
-    }
-    if (BOTH) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) v[s] = b[idx[s]];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        cf acc = cmulr(u[r * 4], v[0]);
-#pragma unroll
-        for (int c = 1; c < 4; ++c) acc = cmac(acc, u[r * 4 + c], v[c]);
-        b[idx[r]] = acc;
-      }
+    for (int s = 0; s < 4; ++s) {
+      const cf l = lam.get(idx[s]);
+      if (op.cmask && !ctrl_ok(op, ok, idx[s])) dr[s] = di[s] = 0.f;
+      part = __builtin_fmaf(dr[s], l.x, part);
+      part = __builtin_fmaf(di[s], l.y, part);
+      part_im = __builtin_fmaf(dr[s], l.y, part_im);
+      part_im = __builtin_fmaf(-di[s], l.x, part_im);
     }
   }
 }
 
-// Gates without control qubits (the common case) run a check-free loop: a
-// per-group predicate makes the compiler copy every output register first.
-template <int R, int J, bool DAG, bool BOTH>
-__device__ __forceinline__ void reg_dense1(cf (&a)[1 << R], cf (&b)[1 << R],
-                                           const float2* __restrict__ M, const RegMap<R>& m,
-                                           uint32_t cmask, uint32_t cval) {
-  if (cmask) reg_dense1_c<R, J, DAG, BOTH, true>(a, b, M, m, cmask, cval);
-  else reg_dense1_c<R, J, DAG, BOTH, false>(a, b, M, m, cmask, cval);
-}
-
-template <int R, int J0, int J1, bool DAG, bool BOTH>
-__device__ __forceinline__ void reg_dense2(cf (&a)[1 << R], cf (&b)[1 << R],
-                                           const float2* __restrict__ M, const RegMap<R>& m,
-                                           uint32_t cmask, uint32_t cval) {
-  if (cmask) reg_dense2_c<R, J0, J1, DAG, BOTH, true>(a, b, M, m, cmask, cval);
-  else reg_dense2_c<R, J0, J1, DAG, BOTH, false>(a, b, M, m, cmask, cval);
-}
-
-template <int R, bool DAG, bool BOTH, int J = 0>
-__device__ __forceinline__ void dispatch1(int j, cf (&a)[1 << R], cf (&b)[1 << R], const float2* M,
-                                          const RegMap<R>& m, uint32_t cmask, uint32_t cval) {
-  if constexpr (J < R) {
-    if (j == J) reg_dense1<R, J, DAG, BOTH>(a, b, M, m, cmask, cval);
-    else dispatch1<R, DAG, BOTH, J + 1>(j, a, b, M, m, cmask, cval);
-  }
-}
-
-template <int R, bool DAG, bool BOTH, int J0 = 0, int J1 = 1>
-__device__ __forceinline__ void dispatch2(int j0, int j1, cf (&a)[1 << R], cf (&b)[1 << R],
-                                          const float2* M, const RegMap<R>& m, uint32_t cmask,
-                                          uint32_t cval) {
-  if constexpr (J1 < R) {
-    if (j0 == J0 && j1 == J1) {
-      reg_dense2<R, J0, J1, DAG, BOTH>(a, b, M, m, cmask, cval);
-    } else if constexpr (J1 + 1 < R) {
-      dispatch2<R, DAG, BOTH, J0, J1 + 1>(j0, j1, a, b, M, m, cmask, cval);
-    } else if constexpr (J0 + 2 < R) {
-      dispatch2<R, DAG, BOTH, J0 + 1, J0 + 2>(j0, j1, a, b, M, m, cmask, cval);
-    }
-  }
-}
-
-// Tile positions of the wavefront-index bits of the thread index (bits
-// 6..8) under register mask `mask`: make_map gives thread bit k the k-th
-// lowest non-register position, so they are the non-register positions left
-// after the six lowest (the lane bits).
-__device__ __forceinline__ uint32_t wave_positions(uint32_t mask, int L) {
-  uint32_t rest = ((1u << L) - 1u) & ~mask;
-#pragma unroll
-  for (int k = 0; k < 6; ++k) rest &= rest - 1u;
-  return rest;
-}
-
-template <int R>
-__device__ __forceinline__ int reg_slot(const RegMap<R>& m, uint32_t q) {
-  return __builtin_popcount(m.mask & ((1u << q) - 1u));
-}
-
-// Dense op on a (and, BOTH, on b with the same matrix).
-template <int R, bool DAG, bool BOTH>
-__device__ __forceinline__ void reg_dense(cf (&a)[1 << R], cf (&b)[1 << R], const DevOp& op,
-                                          const float2* M, const RegMap<R>& m) {
-  if (op.k == 1) {
-    dispatch1<R, DAG, BOTH>(reg_slot(m, op.q[0]), a, b, M, m, op.cmask, op.cval);
+// f(SA, SB as constants) for slot pair number `pair` ((0,1), (0,2), .. in order).
+// The last one is not compared: a path on which nothing ran would keep the
+// result registers' old values alive through the op.
+template <int V>
+using IntC = std::integral_constant<int, V>;
+template <int R, int SA = 0, int SB = 1, typename F>
+__device__ __forceinline__ void for_pair(int pair, F&& f) {
+  constexpr int kThis = SA * (2 * R - SA - 1) / 2 + (SB - SA - 1);
+  if constexpr (kThis == R * (R - 1) / 2 - 1) {
+    f(IntC<SA>(), IntC<SB>());
   } else {
-    dispatch2<R, DAG, BOTH>(reg_slot(m, op.q[0]), reg_slot(m, op.q[1]), a, b, M, m, op.cmask,
-                            op.cval);
+    if (pair == kThis) {
+      f(IntC<SA>(), IntC<SB>());
+    } else if constexpr (SB + 1 < R) {
+      for_pair<R, SA, SB + 1>(pair, f);
+    } else {
+      for_pair<R, SA + 1, SA + 2>(pair, f);
+    }
+  }
+}
+template <int R, int S = 0, typename F>
+__device__ __forceinline__ void for_slot(int slot, F&& f) {
+  if constexpr (S + 1 == R) {
+    f(IntC<S>());
+  } else {
+    if (slot == S) f(IntC<S>());
+    else for_slot<R, S + 1>(slot, f);
   }
 }
 
 // ------------------------------------------------------------------ diagonal ops
-// Targets and controls may be any tile qubits; k <= 2.
-template <int R, bool DAG, bool BOTH>
-__device__ __forceinline__ void reg_diag(cf (&a)[1 << R], cf (&b)[1 << R], const DevOp& op,
-                                         const float2* __restrict__ Dg, const RegMap<R>& m) {
-  const bool two = op.k == 2;
-  cf d0 = ldm(Dg, 0), d1 = ldm(Dg, 1);
-  cf d2 = two ? ldm(Dg, 2) : d0, d3 = two ? ldm(Dg, 3) : d1;
-  if (DAG) {
-    d0 = cconj(d0);
-    d1 = cconj(d1);
-    d2 = cconj(d2);
-    d3 = cconj(d3);
-  }
-  const uint32_t q0 = op.q[0], q1 = two ? op.q[1] : op.q[0];
-  const bool ctrl = op.cmask != 0;
-#pragma unroll
-  for (int i = 0; i < (1 << R); ++i) {
-    const uint32_t x = m.tbase | rdep(m, i);
-    if (ctrl && (x & op.cmask) != op.cval) continue;
-    const uint32_t b0 = (x >> q0) & 1u, b1 = two ? ((x >> q1) & 1u) : 0u;
-    const cf d = b1 ? (b0 ? d3 : d2) : (b0 ? d1 : d0);
-    a[i] = cmulr(d, a[i]);
-    if (BOTH) b[i] = cmulr(d, b[i]);
-  }
+// out = D in (and lam in the reverse sweep), slots unchanged.  The op's code says where
+// its targets are: no register slot (one factor per thread), one (a factor per
+// value of that slot), or two.
+template <int R, bool BOTH>
+__device__ __forceinline__ void scale_reg(const Regs<R>& a, const Regs<R>& b, Regs<R>& oa,
+                                          Regs<R>& ob, int i, cf e) {
+  oa.set(i, cmulr(e, a.get(i)));
+  if (BOTH) ob.set(i, cmulr(e, b.get(i)));
 }
+__device__ __forceinline__ cf pick(bool c, cf x, cf y) { return cf{c ? x.x : y.x, c ? x.y : y.y}; }
 
-// Uncontrolled diagonal ops with the position of each target resolved at
-// compile time: P0 / P1 is the register slot of q[0] / q[1], or R when that
-// target is a thread bit (fixed for the whole thread).  The phase of every
-// register is then a compile-time choice among at most two per-thread values,
-// so each amplitude costs one complex multiply.
-template <int R, bool DAG, bool BOTH, bool TWO, int P0, int P1>
-__device__ __forceinline__ void reg_diag_p(cf (&a)[1 << R], cf (&b)[1 << R], const DevOp& op,
-                                           const float2* __restrict__ Dg, const RegMap<R>& m) {
+template <int R, bool DAG, bool BOTH>
+__device__ __forceinline__ void reg_diag(const Regs<R>& a, const Regs<R>& b, Regs<R>& oa,
+                                         Regs<R>& ob, const DevOp& op,
+                                         const float2* __restrict__ Dg, uint32_t tbase, bool ok) {
+  const bool two = op.k == 2;
   cf d[4];
   d[0] = ldm(Dg, 0);
   d[1] = ldm(Dg, 1);
-  d[2] = TWO ? ldm(Dg, 2) : d[0];
-  d[3] = TWO ? ldm(Dg, 3) : d[1];
+  d[2] = two ? ldm(Dg, 2) : d[0];
+  d[3] = two ? ldm(Dg, 3) : d[1];
   if (DAG) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) d[k] = cconj(d[k]);
   }
-  // Fold the thread-bit targets in: e[c] is the phase for register-bit
-  // pattern c (bit 0: q0, bit 1: q1) of this thread.
-  const bool t0 = P0 == R && ((m.tbase >> op.q[0]) & 1u);
-  const bool t1 = TWO && P1 == R && ((m.tbase >> op.q[1]) & 1u);
-  cf e[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int b0 = P0 == R ? -1 : (c & 1);
-    const int b1 = (!TWO) ? 0 : (P1 == R ? -1 : (c >> 1));
-    // Candidates for the thread bits, chosen per thread.
-    const cf x0 = d[(b1 < 0 ? 0 : b1) * 2 + (b0 < 0 ? 0 : b0)];
-    const cf x1 = d[(b1 < 0 ? 0 : b1) * 2 + (b0 < 0 ? 1 : b0)];
-    const cf y0 = d[(b1 < 0 ? 1 : b1) * 2 + (b0 < 0 ? 0 : b0)];
-    const cf y1 = d[(b1 < 0 ? 1 : b1) * 2 + (b0 < 0 ? 1 : b0)];
-    const cf lo = (b0 < 0 && t0) ? x1 : x0;
-    const cf hi = (b0 < 0 && t0) ? y1 : y0;
-    e[c] = (b1 < 0 && t1) ? hi : lo;
-  }
-#pragma unroll
-  for (int i = 0; i < (1 << R); ++i) {
-    const int c = (P0 == R ? 0 : ((i >> P0) & 1)) | (TWO && P1 != R ? (((i >> P1) & 1) << 1) : 0);
-    a[i] = cmulr(e[c], a[i]);
-    if (BOTH) b[i] = cmulr(e[c], b[i]);
-  }
-}
-
-template <int R, bool DAG, bool BOTH, int P0 = 0, int P1 = 0>
-__device__ __forceinline__ void diag_dispatch2(int p0, int p1, cf (&a)[1 << R], cf (&b)[1 << R],
-                                               const DevOp& op, const float2* Dg,
-                                               const RegMap<R>& m) {
-  if constexpr (P0 <= R) {
-    if constexpr (P1 <= R) {
-      // Two register targets sit in ascending slots (q[0] < q[1]); other
-      // pairs cannot occur and get no code.
-      if constexpr (P0 == R || P1 == R || P0 < P1) {
-        if (p0 == P0 && p1 == P1) {
-          reg_diag_p<R, DAG, BOTH, true, P0, P1>(a, b, op, Dg, m);
-          return;
-        }
-      }
-      diag_dispatch2<R, DAG, BOTH, P0, P1 + 1>(p0, p1, a, b, op, Dg, m);
-    } else {
-      diag_dispatch2<R, DAG, BOTH, P0 + 1, 0>(p0, p1, a, b, op, Dg, m);
-    }
-  }
-}
-
-template <int R, bool DAG, bool BOTH, int P0 = 0>
-__device__ __forceinline__ void diag_dispatch1(int p0, cf (&a)[1 << R], cf (&b)[1 << R],
-                                               const DevOp& op, const float2* Dg,
-                                               const RegMap<R>& m) {
-  if constexpr (P0 <= R) {
-    if (p0 == P0) reg_diag_p<R, DAG, BOTH, false, P0, R>(a, b, op, Dg, m);
-    else diag_dispatch1<R, DAG, BOTH, P0 + 1>(p0, a, b, op, Dg, m);
-  }
-}
-
-// Diagonal op: position-resolved variants without controls, the generic
-// per-amplitude selection with them.
-template <int R, bool DAG, bool BOTH>
-__device__ __forceinline__ void reg_diag_any(cf (&a)[1 << R], cf (&b)[1 << R], const DevOp& op,
-                                             const float2* __restrict__ Dg, const RegMap<R>& m) {
+  // Thread bits of the targets (a register slot's bit of tbase is zero).
+  const bool t0 = (tbase >> op.q[0]) & 1u, t1 = two && ((tbase >> op.q[1]) & 1u);
+  const uint32_t s0 = op.code & 7u, s1 = (op.code >> 3) & 7u;  // slots, or R: thread bit
+  const bool r0 = s0 < uint32_t(R), r1 = two && s1 < uint32_t(R);
   if (op.cmask) {
-    reg_diag<R, DAG, BOTH>(a, b, op, Dg, m);
-    return;
-  }
-  const int p0 = ((m.mask >> op.q[0]) & 1u) ? reg_slot(m, op.q[0]) : R;
-  if (op.k == 2) {
-    const int p1 = ((m.mask >> op.q[1]) & 1u) ? reg_slot(m, op.q[1]) : R;
-    diag_dispatch2<R, DAG, BOTH>(p0, p1, a, b, op, Dg, m);
+#pragma unroll
+    for (int i = 0; i < (1 << R); ++i) {
+      const bool b0 = r0 ? ((uint32_t(i) >> s0) & 1u) != 0u : t0;
+      const bool b1 = r1 ? ((uint32_t(i) >> s1) & 1u) != 0u : t1;
+      const cf e = pick(b1, pick(b0, d[3], d[2]), pick(b0, d[1], d[0]));
+      scale_reg<R, BOTH>(a, b, oa, ob, i, pick(ctrl_ok(op, ok, i), e, cf{1.f, 0.f}));
+    }
+  } else if (!r0 && !r1) {
+    const cf e = pick(t1, pick(t0, d[3], d[2]), pick(t0, d[1], d[0]));
+#pragma unroll
+    for (int i = 0; i < (1 << R); ++i) scale_reg<R, BOTH>(a, b, oa, ob, i, e);
+  } else if (r0 != r1) {
+    // e[v]: the factor for value v of the register slot.
+    cf e[2];
+#pragma unroll
+    for (int v = 0; v < 2; ++v) e[v] = r0 ? pick(t1, d[2 + v], d[v]) : pick(t0, d[2 * v + 1], d[2 * v]);
+    for_slot<R>(int(r0 ? s0 : s1), [&](auto S) {
+#pragma unroll
+      for (int i = 0; i < (1 << R); ++i) scale_reg<R, BOTH>(a, b, oa, ob, i, e[(i >> S.value) & 1]);
+    });
   } else {
-    diag_dispatch1<R, DAG, BOTH>(p0, a, b, op, Dg, m);
-  }
-}
-
-// ------------------------------------------------------------------ parameterised ops
-// psi <- G^dag psi;  acc_d += <dG_d psi | lam> (real part in acc[d], imaginary
-// part in acc[kMaxDeriv + d]);  lam <- G^dag lam  (see apply_param).
-// Three sweeps over the registers so that only one matrix is live at a time.
-template <int R, int K, int J0, int J1>
-__device__ __forceinline__ int param_idx(int g, int s) {
-  const int i0 = K == 1 ? ins0(g, J0) : ins0(ins0(g, J0), J1);
-  return K == 1 ? (i0 | (s << J0)) : (i0 | ((s & 1) << J0) | ((s >> 1) << J1));
-}
-
-template <int R, int K, int J0, int J1, bool CTRL>
-__device__ __forceinline__ void reg_dag_apply(cf (&a)[1 << R], const float2* __restrict__ G,
-                                              const DevOp& op, const RegMap<R>& m) {
-  constexpr int D = 1 << K;
-  if constexpr (K == 2 && !CTRL) {
-    MfmaRows rows;
-    mfma_rows<true>(G, rows);
+    // Slots in ascending order; d's index bits follow.
+    const bool sw = s0 > s1;
+    const cf e1 = pick(sw, d[2], d[1]), e2 = pick(sw, d[1], d[2]);
+    const int lo = int(sw ? s1 : s0), hi = int(sw ? s0 : s1);
+    for_pair<R>(lo * (2 * R - lo - 1) / 2 + (hi - lo - 1), [&](auto SA, auto SB) {
 #pragma unroll
-    for (int g = 0; g < (1 << (R - 2)); ++g) {
-      int idx[4];
-      group_idx<R, J0, J1>(g, idx);
-      mf4 dr, di;
-      mfma_apply(a, idx, rows, dr, di);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) a[idx[r]] = cf{dr[r], di[r]};
-    }
-    return;
-  }
-  cf gd[D * D];
-#pragma unroll
-  for (int r = 0; r < D; ++r)
-#pragma unroll
-    for (int c = 0; c < D; ++c) gd[r * D + c] = cconj(ldm(G, c * D + r));
-#pragma unroll
-  for (int g = 0; g < (1 << (R - K)); ++g) {
-    const int i0 = param_idx<R, K, J0, J1>(g, 0);
-    if (CTRL && (((m.tbase | rdep(m, i0)) & op.cmask) != op.cval)) continue;
-    cf v[D];
-#pragma unroll
-    for (int c = 0; c < D; ++c) v[c] = a[param_idx<R, K, J0, J1>(g, c)];
-#pragma unroll
-    for (int r = 0; r < D; ++r) {
-      cf s = cmulr(gd[r * D], v[0]);
-#pragma unroll
-      for (int c = 1; c < D; ++c) s = cmac(s, gd[r * D + c], v[c]);
-      a[param_idx<R, K, J0, J1>(g, r)] = s;
-    }
-  }
-}
-
-template <int R, int K, int J0, int J1, bool CTRL>
-__device__ __forceinline__ void reg_param_kc(cf (&a)[1 << R], cf (&b)[1 << R], const DevOp& op,
-                                             const float2* __restrict__ mats, const RegMap<R>& m,
-                                             double* acc) {
-  constexpr int D = 1 << K;
-  reg_dag_apply<R, K, J0, J1, CTRL>(a, mats + op.mat, op, m);
-  for (int d = 0; d < op.nderiv; ++d) {
-    const float2* dG = mats + (d == 0 ? op.dmat[0] : op.dmat[1]);  // static field access
-    if constexpr (K == 2 && !CTRL) {
-      MfmaRows rows;
-      mfma_rows<false>(dG, rows);
-      float part = 0.f, part_im = 0.f;
-#pragma unroll
-      for (int g = 0; g < (1 << (R - 2)); ++g) {
-        int idx[4];
-        group_idx<R, J0, J1>(g, idx);
-        mf4 dr, di;
-        mfma_apply(a, idx, rows, dr, di);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const cf l = b[idx[r]];
-          part = __builtin_fmaf(dr[r], l.x, part);
-          part = __builtin_fmaf(di[r], l.y, part);
-          part_im = __builtin_fmaf(dr[r], l.y, part_im);
-          part_im = __builtin_fmaf(-di[r], l.x, part_im);
-        }
+      for (int i = 0; i < (1 << R); ++i) {
+        const int c = ((i >> SA.value) & 1) | (((i >> SB.value) & 1) << 1);
+        scale_reg<R, BOTH>(a, b, oa, ob, i, c == 0 ? d[0] : c == 1 ? e1 : c == 2 ? e2 : d[3]);
       }
-      if (d == 0) {
-        acc[0] += double(part);
-        acc[kMaxDeriv] += double(part_im);
-      } else {
-        acc[1] += double(part);
-        acc[kMaxDeriv + 1] += double(part_im);
-      }
-      continue;
-    }
-    cf dg[D * D];
-#pragma unroll
-    for (int i = 0; i < D * D; ++i) dg[i] = ldm(dG, i);
-    float part = 0.f, part_im = 0.f;
-#pragma unroll
-    for (int g = 0; g < (1 << (R - K)); ++g) {
-      const int i0 = param_idx<R, K, J0, J1>(g, 0);
-      if (CTRL && (((m.tbase | rdep(m, i0)) & op.cmask) != op.cval)) continue;
-#pragma unroll
-      for (int r = 0; r < D; ++r) {
-        cf s = cmulr(dg[r * D], a[param_idx<R, K, J0, J1>(g, 0)]);
-#pragma unroll
-        for (int c = 1; c < D; ++c) s = cmac(s, dg[r * D + c], a[param_idx<R, K, J0, J1>(g, c)]);
-        const cf l = b[param_idx<R, K, J0, J1>(g, r)];
-        part += s.x * l.x + s.y * l.y;
-        part_im += s.x * l.y - s.y * l.x;
-      }
-    }
-    if (d == 0) {
-      acc[0] += double(part);
-      acc[kMaxDeriv] += double(part_im);
-    } else {
-      acc[1] += double(part);
-      acc[kMaxDeriv + 1] += double(part_im);
-    }
-  }
-  reg_dag_apply<R, K, J0, J1, CTRL>(b, mats + op.mat, op, m);
-}
-
-template <int R, int K, int J0, int J1>
-__device__ __forceinline__ void reg_param_k(cf (&a)[1 << R], cf (&b)[1 << R], const DevOp& op,
-                                            const float2* __restrict__ mats, const RegMap<R>& m,
-                                            double* acc) {
-  if (op.cmask) reg_param_kc<R, K, J0, J1, true>(a, b, op, mats, m, acc);
-  else reg_param_kc<R, K, J0, J1, false>(a, b, op, mats, m, acc);
-}
-
-template <int R, int J0 = 0>
-__device__ __forceinline__ void param_dispatch1(int j, cf (&a)[1 << R], cf (&b)[1 << R],
-                                                const DevOp& op, const float2* mats,
-                                                const RegMap<R>& m, double* acc) {
-  if constexpr (J0 < R) {
-    if (j == J0) reg_param_k<R, 1, J0, 0>(a, b, op, mats, m, acc);
-    else param_dispatch1<R, J0 + 1>(j, a, b, op, mats, m, acc);
+    });
   }
 }
-
-template <int R, int J0 = 0, int J1 = 1>
-__device__ __forceinline__ void param_dispatch2(int j0, int j1, cf (&a)[1 << R],
-                                                cf (&b)[1 << R], const DevOp& op,
-                                                const float2* mats, const RegMap<R>& m,
-                                                double* acc) {
-  if constexpr (J1 < R) {
-    if (j0 == J0 && j1 == J1) {
-      reg_param_k<R, 2, J0, J1>(a, b, op, mats, m, acc);
-    } else if constexpr (J1 + 1 < R) {
-      param_dispatch2<R, J0, J1 + 1>(j0, j1, a, b, op, mats, m, acc);
-    } else if constexpr (J0 + 2 < R) {
-      param_dispatch2<R, J0 + 1, J0 + 2>(j0, j1, a, b, op, mats, m, acc);
-    }
-  }
-}
-
 
 // ------------------------------------------------------------------ noise channels
 // Trajectory context of a noisy forward run, passed as the run's acc_fn:
@@ -666,92 +446,139 @@ struct IsNoise : std::false_type {};
 template <>
 struct IsNoise<NoiseDraw> : std::true_type {};
 
-// Sum over the 2^gbits lanes of this lane's trajectory group (all of them
+// Sums over the 2^gbits lanes of this lane's trajectory group (all of them
 // end with the same bits: each butterfly step adds the same two values).
 // The DPP steps pair each lane with one that holds the same partial as its
 // butterfly partner (lane ^ 4, lane ^ 8), so the sums are the butterfly's.
+template <int N>
+__device__ __forceinline__ void group_sums(double (&v)[N], int gbits) {
+  auto step = [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = f(v[i]);
+  };
+  if (gbits > 0) step([](double x) { return dpp_add<0xB1>(x); });
+  if (gbits > 1) step([](double x) { return dpp_add<0x4E>(x); });
+  if (gbits > 2) step([](double x) { return dpp_add<0x141>(x); });
+  if (gbits > 3) step([](double x) { return dpp_add<0x140>(x); });
+  if (gbits > 4) step([](double x) { return x + __shfl_xor(x, 16, 64); });
+  if (gbits > 5) step([](double x) { return x + __shfl_xor(x, 32, 64); });
+}
 __device__ __forceinline__ double group_sum(double v, int gbits) {
-  if (gbits > 0) v = dpp_add<0xB1>(v);
-  if (gbits > 1) v = dpp_add<0x4E>(v);
-  if (gbits > 2) v = dpp_add<0x141>(v);
-  if (gbits > 3) v = dpp_add<0x140>(v);
-  if (gbits > 4) v += __shfl_xor(v, 16, 64);
-  if (gbits > 5) v += __shfl_xor(v, 32, 64);
-  return v;
+  double s[1] = {v};
+  group_sums(s, gbits);
+  return s[0];
 }
 
-// One channel on register slot J of this lane's trajectory.  Unitary
-// mixtures pick unitary k with the first u < cum[k]; other channels take
-// p_k = <psi|K_k^dag K_k|psi> from the qubit's reduced density matrix
-// (group sums), pick the first k with u < p_0 + ... + p_k (the last k with
-// p_k > 0 when none) and apply K_k / sqrt(p_k).  Lanes of different
-// trajectories may pick different operators: the matrix is read per lane.
-template <int R, int J>
-__device__ __forceinline__ void reg_channel_j(cf (&a)[1 << R], const DevOp& op,
-                                              const float2* __restrict__ mats,
-                                              NoiseDraw& nd) {
-  constexpr int G = 1 << (R - 1);
+// The operator that a channel applies to this lane's trajectory, times scale.
+struct ChannelPick {
+  int k;
+  float scale;
+};
+
+// This lane's part of the reduced density matrix of register slot J's qubit: |x0|^2,
+// |x1|^2 and (FULL) conj(x0) x1.  Every product is added to a sum that starts from a
+// value the compiler does not know: it would compute the sums of all slots before
+// looking at the op, for every op (2.2x this kernel's FP32 instructions).
+template <int R, int J, bool FULL>
+__device__ __forceinline__ void reg_density(const Regs<R>& a, float (&d)[FULL ? 4 : 2]) {
+#pragma unroll
+  for (int i = 0; i < (FULL ? 4 : 2); ++i) {
+    d[i] = 0.f;
+    asm volatile("" : "+v"(d[i]));
+  }
+#pragma unroll
+  for (int g = 0; g < (1 << (R - 1)); ++g) {
+    const int i0 = ins0(g, J);
+    const cf x0 = a.get(i0), x1 = a.get(i0 | (1 << J));
+    d[0] = __builtin_fmaf(x0.y, x0.y, __builtin_fmaf(x0.x, x0.x, d[0]));
+    d[1] = __builtin_fmaf(x1.y, x1.y, __builtin_fmaf(x1.x, x1.x, d[1]));
+    if constexpr (FULL) {
+      d[2] = __builtin_fmaf(x0.y, x1.y, __builtin_fmaf(x0.x, x1.x, d[2]));
+      d[3] = __builtin_fmaf(-x0.y, x1.x, __builtin_fmaf(x0.x, x1.y, d[3]));
+    }
+  }
+}
+// The first k with u < p_0 + ... + p_k, the last k with p_k > 0 when none.
+template <typename Prob>
+__device__ __forceinline__ ChannelPick pick_kraus(int nk, double u, Prob&& prob) {
+  double cum = 0.0, pp = 1.0;
+  int last = 0, pick = -1;
+  for (int k = 0; k < nk; ++k) {
+    const double pk = prob(k);
+    if (pk > 0.0) last = k;
+    cum += pk;
+    if (pick < 0 && u < cum) {
+      pick = k;
+      pp = pk;
+    }
+  }
+  if (pick < 0) {
+    pick = last;
+    pp = prob(last);
+  }
+  return ChannelPick{pick, float(1.0 / sqrt(pp))};
+}
+
+// Unitary mixtures pick unitary k with the first u < cum[k]; other channels take
+// p_k = <psi|K_k^dag K_k|psi> from the qubit's reduced density matrix, pick the
+// first k with u < p_0 + ... + p_k (the last k with p_k > 0 when none) and apply
+// K_k / sqrt(p_k).  Lanes of different trajectories may pick different operators.
+template <int R>
+__device__ __forceinline__ ChannelPick channel_pick(const Regs<R>& a, const DevOp& op,
+                                                    const float2* __restrict__ mats,
+                                                    NoiseDraw& nd) {
   const int nk = ChanKraus(op.cval);
   const double u = nd(op.col[0]);
   const float2* X = mats + op.dmat[0];
-  int pick = nk - 1;
-  double pp = 1.0;
   if (op.cval & kChanMixture) {
+    int pick = nk - 1;
     for (int k = nk - 2; k >= 0; --k)
       if (u < double(X[k].x)) pick = k;
-    if ((op.cval & kChanFirstIdentity) && pick == 0) return;
-  } else {
-    float s00 = 0.f, s11 = 0.f, sr = 0.f, si = 0.f;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int i0 = ((g >> J) << (J + 1)) | (g & ((1 << J) - 1));
-      const cf x0 = a[i0], x1 = a[i0 | (1 << J)];
-      s00 += x0.x * x0.x + x0.y * x0.y;
-      s11 += x1.x * x1.x + x1.y * x1.y;
-      sr += x0.x * x1.x + x0.y * x1.y;  // conj(x0) * x1
-      si += x0.x * x1.y - x0.y * x1.x;
-    }
-    const double d00 = group_sum(double(s00), nd.gbits), d11 = group_sum(double(s11), nd.gbits);
-    const double dr = group_sum(double(sr), nd.gbits), di = group_sum(double(si), nd.gbits);
-    double cum = 0.0;
-    int last = 0;
-    pick = -1;
-    for (int k = 0; k < nk; ++k) {
-      const float2 e00 = X[4 * k], e01 = X[4 * k + 1], e11 = X[4 * k + 3];
-      const double pk = double(e00.x) * d00 + double(e11.x) * d11 +
-                        2.0 * (double(e01.x) * dr - double(e01.y) * di);
-      if (pk > 0.0) last = k;
-      cum += pk;
-      if (pick < 0 && u < cum) {
-        pick = k;
-        pp = pk;
-      }
-    }
-    if (pick < 0) {
-      pick = last;
-      const float2 e00 = X[4 * last], e01 = X[4 * last + 1], e11 = X[4 * last + 3];
-      pp = double(e00.x) * d00 + double(e11.x) * d11 + 2.0 * (double(e01.x) * dr - double(e01.y) * di);
-    }
+    return ChannelPick{pick, 1.0f};
   }
-  const float2* M = mats + op.mat + 4 * pick;
-  const float sc = (op.cval & kChanMixture) ? 1.0f : float(1.0 / sqrt(pp));
+  if (op.cval & kChanDiagonal) {
+    float s[2];
+    for_slot<R>(int(op.code), [&](auto J) { reg_density<R, J.value, false>(a, s); });
+    double d[2] = {double(s[0]), double(s[1])};
+    group_sums(d, nd.gbits);
+    return pick_kraus(nk, u, [&](int k) {
+      return double(X[4 * k].x) * d[0] + double(X[4 * k + 3].x) * d[1];
+    });
+  }
+  float s[4];
+  for_slot<R>(int(op.code), [&](auto J) { reg_density<R, J.value, true>(a, s); });
+  double d[4] = {double(s[0]), double(s[1]), double(s[2]), double(s[3])};
+  group_sums(d, nd.gbits);
+  return pick_kraus(nk, u, [&](int k) {
+    const float2 e01 = X[4 * k + 1];
+    return double(X[4 * k].x) * d[0] + double(X[4 * k + 3].x) * d[1] +
+           2.0 * (double(e01.x) * d[2] - double(e01.y) * d[3]);
+  });
+}
+
+// out = the picked operator on register slot J of in; the matrix is read per lane.
+// Bound by the number of VALU instructions: with real matrices half the products
+// go, and with diagonal K^dag K half of the density's and of its lane sums (every
+// channel here that is no unitary mixture is both): 717 us (965 us) for 32 rows of
+// 1000 8-qubit trajectories with 128 channels.
+template <int R, int J, bool REAL>
+__device__ __forceinline__ void reg_channel(const Regs<R>& in, Regs<R>& out,
+                                            const float2* __restrict__ M, float sc) {
   const cf m00{M[0].x * sc, M[0].y * sc}, m01{M[1].x * sc, M[1].y * sc};
   const cf m10{M[2].x * sc, M[2].y * sc}, m11{M[3].x * sc, M[3].y * sc};
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int i0 = ((g >> J) << (J + 1)) | (g & ((1 << J) - 1));
-    const cf x0 = a[i0], x1 = a[i0 | (1 << J)];
-    a[i0] = cmac(cmulr(m00, x0), m01, x1);
-    a[i0 | (1 << J)] = cmac(cmulr(m10, x0), m11, x1);
-  }
-}
-
-template <int R, int J = 0>
-__device__ __forceinline__ void reg_channel(int j, cf (&a)[1 << R], const DevOp& op,
-                                            const float2* mats, NoiseDraw& nd) {
-  if constexpr (J < R) {
-    if (j == J) reg_channel_j<R, J>(a, op, mats, nd);
-    else reg_channel<R, J + 1>(j, a, op, mats, nd);
+  for (int g = 0; g < (1 << (R - 1)); ++g) {
+    const int i0 = ins0(g, J);
+    const cf x0 = in.get(i0), x1 = in.get(i0 | (1 << J));
+    if constexpr (REAL) {
+      out.set(i0, cf{__builtin_fmaf(m01.x, x1.x, m00.x * x0.x),
+                     __builtin_fmaf(m01.x, x1.y, m00.x * x0.y)});
+      out.set(i0 | (1 << J), cf{__builtin_fmaf(m11.x, x1.x, m10.x * x0.x),
+                                __builtin_fmaf(m11.x, x1.y, m10.x * x0.y)});
+    } else {
+      out.set(i0, cmac(cmulr(m00, x0), m01, x1));
+      out.set(i0 | (1 << J), cmac(cmulr(m10, x0), m11, x1));
+    }
   }
 }
 
@@ -821,15 +648,14 @@ __device__ __forceinline__ void esync() {
 // Tile I/O of the engine.  LdsIO: the tile enters and leaves in LDS buffers A
 // (and B) in the natural layout; the caller synchronises before the run and
 // the engine synchronises before returning.  TileIO: the first remap loads the
-// registers straight from memory with load(x, a, b) and the run ends by
-// storing them with store(x, a, b), x the tile index of each register (b only
-// in the reverse sweep); LDS is then used only by the remaps in between, and
-// no barrier surrounds the run (a remap's own barriers order its LDS use).
-// With an index function (tile_io_indexed), load and store receive index(x)
-// instead of x.  The index must be OR-linear over disjoint bits of x (a
-// tile's bits deposited into the global index, plus the tile's base), so the
-// engine computes it once per thread (its own bits) and once per register
-// qubit, and each register's index is one OR of those.
+// registers straight from memory with load(thread, reg, set) and the run ends with
+// store(thread, reg, get): register r's amplitude has index thread | reg[r] and
+// goes through set(r, a, b) or get_a(r) and get_b(r) (b only in the reverse sweep).
+// LDS is then used only by the remaps in between, and no barrier surrounds the run
+// (a remap's own barriers order its LDS use).  `thread` is index(x) of this
+// thread's own tile bits x, and `reg`, which is wave-uniform, index of the
+// register's; index must be OR-linear over disjoint bits (a tile's bits
+// deposited into the global index).
 struct LdsIO {};
 struct IdentityIndex {
   __device__ __forceinline__ uint64_t operator()(uint32_t x) const { return x; }
@@ -849,22 +675,31 @@ __device__ __forceinline__ TileIO<LoadFn, StoreFn, IndexFn> tile_io_indexed(Inde
                                                                             StoreFn s) {
   return TileIO<LoadFn, StoreFn, IndexFn>{l, s, i};
 }
-
-// index(tbase | rdep(m, r)) for every register r: the thread's part once, one
-// term per register qubit, then one OR per register (f(r, index)).
-template <int R, typename IO, typename F>
-__device__ __forceinline__ void for_reg_index(const RegMap<R>& m, IO& io, F&& f) {
-  uint64_t g[1 << R];
-  g[0] = io.index(m.tbase);
-#pragma unroll
-  for (int j = 0; j < R; ++j) {
-    const uint64_t gj = io.index(1u << m.rpos[j]);
-#pragma unroll
-    for (int r = 0; r < (1 << j); ++r) g[r | (1 << j)] = g[r] | gj;
-  }
-#pragma unroll
-  for (int r = 0; r < (1 << R); ++r) f(r, g[r]);
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  return uint64_t(uint32_t(uniform(int(uint32_t(x))))) |
+         (uint64_t(uint32_t(uniform(int(uint32_t(x >> 32))))) << 32);
 }
+// f(r) for every register r of g.
+template <size_t N, typename F>
+__device__ __forceinline__ void each_reg(const uint64_t (&)[N], F&& f) {
+#pragma unroll
+  for (int r = 0; r < int(N); ++r) f(r);
+}
+// Global index parts of the 2^R registers (wave-uniform).
+template <int R>
+struct RegIndex {
+  uint64_t g[1 << R];
+  template <typename IO>
+  __device__ __forceinline__ RegIndex(uint32_t slots, IO& io) {
+    g[0] = 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const uint64_t gj = uniform64(io.index(slot_bit(slots, j)));
+#pragma unroll
+      for (int r = 0; r < (1 << j); ++r) g[r | (1 << j)] = g[r] | gj;
+    }
+  }
+};
 template <typename IO>
 struct IsLdsIO {
   static constexpr bool value = false;
@@ -873,6 +708,116 @@ template <>
 struct IsLdsIO<LdsIO> {
   static constexpr bool value = true;
 };
+
+// The part of a run that the op loop carries besides the registers.
+struct RunState {
+  uint32_t tbase;  // this thread's tile bits
+  uint32_t mask;   // register qubits (wave-uniform)
+  int slot;        // derivative matrices of earlier parameterised ops
+  bool first_store;
+  // The thread's part of an op's controls.
+  __device__ __forceinline__ bool ok(const DevOp& op) const {
+    return ((tbase ^ op.cval) & op.cmask & ~mask) == 0u;
+  }
+};
+
+template <typename AccFn>
+struct HasChannels {
+  static constexpr bool value = IsNoise<std::decay_t<AccFn>>::value;
+};
+
+// A remap that leaves the wavefront-index qubits where they are moves
+// every amplitude within its own wavefront: wavefront w stores and
+// reloads exactly the (swizzled) LDS entries it read at the previous
+// remap, so it needs no workgroup barrier.  The first store of a run
+// still waits for the whole workgroup (entries last read in another
+// layout, or by other wavefronts on the previous tile).
+template <int R, bool REV, bool WAVE>
+__device__ __forceinline__ void run_remap(const Regs<R>& ra, const Regs<R>& rb, Regs<R>& oa,
+                                          Regs<R>& ob, const DevOp& op, float2* __restrict__ A,
+                                          float2* __restrict__ B, int L, RunState& st) {
+  const bool local = !WAVE && !st.first_store && (op.code & kCodeLocal);
+  uint32_t off[1 << R];
+  reg_offsets<R>(st.tbase, op.cval, true, off);
+  if (!local) esync<WAVE>();
+  reg_store<R>(ra, A, off);
+  if (REV) reg_store<R>(rb, B, off);
+  st.first_store = false;
+  if (local) esync<true>();
+  else esync<WAVE>();
+  st.mask = op.cmask;
+  st.tbase = thread_base<R, WAVE>(op.dmat[0], L);
+  reg_offsets<R>(st.tbase, op.dmat[0], true, off);
+  reg_load<R>(oa, A, off);
+  if (REV) reg_load<R>(ob, B, off);
+}
+
+// One op, from (ra, rb) to (oa, ob).
+template <int R, bool REV, bool WAVE, typename MS, typename AccFn>
+__device__ __forceinline__ void run_op(const Regs<R>& ra, const Regs<R>& rb, Regs<R>& oa,
+                                       Regs<R>& ob, DevOp& op, float2* __restrict__ A,
+                                       float2* __restrict__ B, int L, MS& mc, AccFn&& acc_fn,
+                                       RunState& st, const ChannelPick& cp) {
+  if (op.type == kOpRemap) {
+    run_remap<R, REV, WAVE>(ra, rb, oa, ob, op, A, B, L, st);
+    return;
+  }
+  const float2* mats = mats_for(mc, op);
+  const bool ok = st.ok(op);
+  if (op.type == kOpDiag) {
+    reg_diag<R, REV, REV>(ra, rb, oa, ob, op, mats + op.mat, st.tbase, ok);
+    return;
+  }
+  if constexpr (!REV && HasChannels<AccFn>::value) {
+    if (op.type == kOpChannel) {
+      const float2* M = mats + op.mat + 4 * cp.k;
+      for_slot<R>(int(op.code), [&](auto J) {
+        if (op.cval & kChanReal) reg_channel<R, J.value, true>(ra, oa, M, cp.scale);
+        else reg_channel<R, J.value, false>(ra, oa, M, cp.scale);
+      });
+      return;
+    }
+  }
+  MfmaRows m;
+  engine_rows<REV>(mats + op.mat, op, m);
+  const int pair = int(op.code & kCodePair);
+  const int nd = REV && op.type == kOpParam ? op.nderiv : 0;
+  float part[2 * kMaxDeriv] = {0.f, 0.f, 0.f, 0.f};
+  for_pair<R>(pair, [&](auto SA, auto SB) {
+    reg_dense<R, SA.value, SB.value>(ra, oa, m, op, ok);
+    if (REV) {
+      reg_dense<R, SA.value, SB.value>(rb, ob, m, op, ok);
+#pragma unroll 1
+      for (int d = 0; d < nd; ++d) {
+        MfmaRows dm;
+        engine_rows<false>(mats + (d == 0 ? op.dmat[0] : op.dmat[1]), op, dm);
+        float re, im;
+        reg_deriv<R, SA.value, SB.value>(oa, rb, dm, op, ok, re, im);
+        if (d == 0) {
+          part[0] = re;
+          part[kMaxDeriv] = im;
+        } else {
+          part[1] = re;
+          part[kMaxDeriv + 1] = im;
+        }
+      }
+    }
+  });
+  if (nd > 0) {
+    // Wave mode: gradient partials count each amplitude once (replica lanes 0).
+    if (WAVE && ((threadIdx.x & 63u) >> (L - R)) != 0u)
+      part[0] = part[1] = part[2] = part[3] = 0.f;
+    // The imaginary parts reach only the callers that use them (the
+    // compiler drops them elsewhere).
+    const double w0 = wave_sum(double(part[0])), v0 = wave_sum(double(part[kMaxDeriv]));
+    if ((threadIdx.x & 63) == 0) acc_fn(st.slot, op.col[0], w0, v0);
+    if (nd > 1) {
+      const double w1 = wave_sum(double(part[1])), v1 = wave_sum(double(part[kMaxDeriv + 1]));
+      if ((threadIdx.x & 63) == 0) acc_fn(st.slot + 1, op.col[1], w1, v1);
+    }
+    st.slot += nd;
+  }
+}
 
 // Apply ops [b, e) to a tile of 2^L amplitudes (A, and B in the reverse sweep).
 // REV = false: apply each op's matrix to A.  REV = true: un-apply (M^dagger)
@@ -887,81 +832,71 @@ template <int R, bool REV, bool WAVE, typename MS, typename AccFn, typename IO>
 __device__ __forceinline__ void reg_run(float2* __restrict__ A, float2* __restrict__ B, int L,
                         const DevOp* __restrict__ ops, int b, int e,
                         MS& mc, AccFn&& acc_fn, IO& io) {
-  // Wave mode: gradient partials count each amplitude once (replica lanes 0).
-  const bool canon = !WAVE || ((threadIdx.x & 63u) >> (L - R)) == 0u;
   constexpr bool kLds = IsLdsIO<IO>::value;
-  cf ra[1 << R];
-  cf rb[1 << R];  // unused when !REV
-  RegMap<R> m;
-  bool have = false, swizzled = false, first_store = true;
-  int slot = 0;
-  for (int i = b; i < e; ++i) {
-    DevOp op = load_op(ops + i);
-    const float2* mats = op.type != kOpRemap ? mats_for(mc, op) : nullptr;
-    if (op.type == kOpRemap) {
-      if constexpr (!kLds) {
-        if (!have) {
-          make_map<R, WAVE>(m, op.cmask, L);
-          for_reg_index<R>(m, io, [&](int r, uint64_t g) { io.load(g, ra[r], rb[r]); });
-          have = true;
-          continue;
+  Regs<R> xa, xb, ya, yb;  // two register sets; the b's unused when !REV
+  const DevOp first = load_op(ops + b);
+  RunState st{thread_base<R, WAVE>(first.dmat[0], L), first.cmask, 0, true};
+  if constexpr (kLds) {
+    uint32_t off[1 << R];
+    reg_offsets<R>(st.tbase, first.dmat[0], false, off);
+    esync<WAVE>();
+    reg_load<R>(xa, A, off);
+    if (REV) reg_load<R>(xb, B, off);
+  } else {
+    const RegIndex<R> reg(first.dmat[0], io);
+    io.load(io.index(st.tbase), reg.g, [&](int r, cf va, cf vb) {
+      xa.set(r, va);
+      if (REV) xb.set(r, vb);
+    });
+  }
+  auto finish = [&](Regs<R>& ra, Regs<R>& rb) {
+    if constexpr (kLds) {
+      uint32_t off[1 << R];
+      reg_offsets<R>(st.tbase, first.dmat[1], false, off);
+      esync<WAVE>();
+      reg_store<R>(ra, A, off);
+      if (REV) reg_store<R>(rb, B, off);
+      esync<WAVE>();
+    } else {
+      const RegIndex<R> reg(first.dmat[1], io);
+      io.store(io.index(st.tbase), reg.g, [&](int r) { return ra.get(r); },
+               [&](int r) { return rb.get(r); });
+    }
+  };
+  // The next op to run on registers r; false at the end.  Channels that leave every
+  // lane's trajectory as it is (unitary 0, the identity) are passed over.
+  int i = b + 1;
+  DevOp op;
+  ChannelPick cp{0, 1.0f};
+  auto next = [&](const Regs<R>& r) -> bool {
+    while (i < e) {
+      op = load_op(ops + i);
+      ++i;
+      if constexpr (!REV && HasChannels<AccFn>::value) {
+        if (op.type == kOpChannel) {
+          DevOp ch = op;
+          const float2* mats = mats_for(mc, ch);
+          cp = channel_pick<R>(r, ch, mats, acc_fn);
+          if ((ch.cval & kChanFirstIdentity) && __ballot(cp.k != 0) == 0) continue;
         }
       }
-      // A remap that leaves the wavefront-index qubits where they are moves
-      // every amplitude within its own wavefront: wavefront w stores and
-      // reloads exactly the (swizzled) LDS entries it read at the previous
-      // remap, so it needs no workgroup barrier.  The first store of a run
-      // still waits for the whole workgroup (entries last read in another
-      // layout, or by other wavefronts on the previous tile).
-      const uint32_t nmask = uint32_t(uniform(int(op.cmask)));
-      const bool local = !WAVE && have && !first_store &&
-                         wave_positions(m.mask, L) == wave_positions(nmask, L);
-      if (have) {
-        if (!local) esync<WAVE>();
-        reg_store<R>(ra, A, m, true);
-        if (REV) reg_store<R>(rb, B, m, true);
-        swizzled = true;
-        first_store = false;
-      }
-      if (local) esync<true>();
-      else esync<WAVE>();
-      make_map<R, WAVE>(m, nmask, L);
-      reg_load<R>(ra, A, m, swizzled);
-      if (REV) reg_load<R>(rb, B, m, swizzled);
-      have = true;
-      continue;
+      return true;
     }
-    if (op.type == kOpDiag) {
-      reg_diag_any<R, REV, REV>(ra, rb, op, mats + op.mat, m);
-    } else if (REV && op.type == kOpParam) {
-      double acc[2 * kMaxDeriv] = {0.0, 0.0, 0.0, 0.0};
-      if (op.k == 1) param_dispatch1<R>(reg_slot(m, op.q[0]), ra, rb, op, mats, m, acc);
-      else param_dispatch2<R>(reg_slot(m, op.q[0]), reg_slot(m, op.q[1]), ra, rb, op, mats, m, acc);
-      if (!canon) acc[0] = acc[1] = acc[2] = acc[3] = 0.0;
-      // The imaginary parts reach only the callers that use them (the
-      // compiler drops them elsewhere).
-      const double w0 = wave_sum(acc[0]), v0 = wave_sum(acc[kMaxDeriv]);
-      if ((threadIdx.x & 63) == 0) acc_fn(slot, op.col[0], w0, v0);
-      if (op.nderiv > 1) {
-        const double w1 = wave_sum(acc[1]), v1 = wave_sum(acc[kMaxDeriv + 1]);
-        if ((threadIdx.x & 63) == 0) acc_fn(slot + 1, op.col[1], w1, v1);
-      }
-      slot += op.nderiv;
-    } else if (op.type == kOpChannel) {
-      if constexpr (!REV && IsNoise<std::decay_t<AccFn>>::value)
-        reg_channel<R>(reg_slot(m, op.q[0]), ra, op, mats, acc_fn);
-    } else {
-      reg_dense<R, REV, REV>(ra, rb, op, mats + op.mat, m);
+    return false;
+  };
+  // One half of the loop per register set; every op goes from one to the other, so
+  // that only one is live between ops.
+  while (true) {
+    if (!next(xa)) {
+      finish(xa, xb);
+      return;
     }
-  }
-  if (!have) return;
-  if constexpr (kLds) {
-    esync<WAVE>();
-    reg_store<R>(ra, A, m, false);
-    if (REV) reg_store<R>(rb, B, m, false);
-    esync<WAVE>();
-  } else {
-    for_reg_index<R>(m, io, [&](int r, uint64_t g) { io.store(g, ra[r], rb[r]); });
+    run_op<R, REV, WAVE>(xa, xb, ya, yb, op, A, B, L, mc, acc_fn, st, cp);
+    if (!next(ya)) {
+      finish(ya, yb);
+      return;
+    }
+    run_op<R, REV, WAVE>(ya, yb, xa, xb, op, A, B, L, mc, acc_fn, st, cp);
   }
 }
 

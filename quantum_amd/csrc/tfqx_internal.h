@@ -36,6 +36,8 @@ enum OpType : uint8_t {
 // (its random stream).
 constexpr uint32_t kChanMixture = 1u << 8;    // unitary mixture
 constexpr uint32_t kChanFirstIdentity = 1u << 9;  // unitary 0 is the identity
+constexpr uint32_t kChanDiagonal = 1u << 10;  // every K_k^dag K_k is diagonal
+constexpr uint32_t kChanReal = 1u << 11;      // every K_k is real
 constexpr int ChanKraus(uint32_t cval) { return int(cval & 15u); }
 
 // Register engine (reg_engine.h): 2^9 threads per workgroup, each holding
@@ -66,13 +68,18 @@ constexpr int kWaveMaxQubits = 10;
 // Batches with fewer wave-eligible circuits than this run them as workgroups.
 constexpr int kWaveMinCircuits = 1024;
 
+// DevOp::code bits (register engine).
+constexpr int kCodePair = 15;   // slot pair of the group
+constexpr int kCodeSwap = 16;   // two qubits: index bits exchanged; one: group bit 1
+constexpr int kCodeLocal = 1;   // remap within wavefronts
+
 // One op on a tile.  Qubit positions are tile-local bit indices (ascending).
 // Matrix layout: row-major 2^k x 2^k complex64, index bit j <-> q[j].
 struct alignas(8) DevOp {
   uint8_t type;
   uint8_t k;
   uint8_t nderiv;
-  uint8_t pad0;
+  uint8_t code;  // register engine: see AnnotateEngine (plan.h)
   uint8_t q[kMaxFuse];
   uint32_t cmask;    // tile-local control bits
   uint32_t cval;     // required values of the control bits

@@ -305,13 +305,13 @@ __device__ __forceinline__ void wave_circuit(const BatchArgs& a, int ci, float2*
   const uint32_t lane = threadIdx.x & 63u;
   // Forward from |0>, final state to P in the natural layout.
   auto fio = tile_io(
-      [](uint64_t t, const auto& g, auto&& set) {
-        each_reg(g, [&](int r) { set(r, cf{(t | g[r]) == 0 ? 1.f : 0.f, 0.f}, cf{}); });
+      [](uint64_t t, const auto& slot, auto&& set_a, auto&&) {
+        each_reg(slot, uint32_t(t), [&](int r, uint32_t x) { set_a(r, cf{x == 0 ? 1.f : 0.f, 0.f}); });
       },
-      [P](uint64_t t, const auto& g, auto&& get_a, auto&&) {
-        each_reg(g, [&](int r) {
-          const cf va = get_a(r);
-          P[uint32_t(t | g[r])] = make_float2(va.x, va.y);
+      [P](uint64_t t, const auto& slot, auto&& get_a, auto&&) {
+        each_reg(slot, uint32_t(t), [&](int r, uint32_t x) {
+          const cf v = get_a(r);
+          P[x] = make_float2(v.x, v.y);
         });
       });
   reg_run_wave<false>(P, P, n, a.ops, uniform(c.fwd_begin), uniform(c.fwd_end), a.mats, NoAcc(),
@@ -325,11 +325,11 @@ __device__ __forceinline__ void wave_circuit(const BatchArgs& a, int ci, float2*
     __threadfence();
     wave_lambda(P, Q, N, a, uniform(c.lam_begin), uniform(c.lam_end));
     auto rio = tile_io(
-        [P, Q](uint64_t t, const auto& g, auto&& set) {
-          each_reg(g, [&](int r) {
-            const uint32_t x = uint32_t(t | g[r]);
+        [P, Q](uint64_t t, const auto& slot, auto&& set_a, auto&& set_b) {
+          each_reg(slot, uint32_t(t), [&](int r, uint32_t x) {
             const float2 u = P[x], v = Q[x];
-            set(r, cf{u.x, u.y}, cf{v.x, v.y});
+            set_a(r, cf{u.x, u.y});
+            set_b(r, cf{v.x, v.y});
           });
         },
         [](uint64_t, const auto&, auto&&, auto&&) {});
@@ -367,22 +367,17 @@ __device__ __forceinline__ void tiled_forward(float2* G, int n, const BatchArgs&
           [&](uint32_t j) -> uint64_t {
             return use_tab ? tile_index_tab(0, j, ps.nlow, tab) : tile_index(0, j, ps);
           },
-          [&](uint64_t th, const auto& g, auto&& set) {
+          [&](uint64_t th, const auto& slot, auto&& set_a, auto&&) {
             const uint64_t x = base | th;
-            if (first) {
-              each_reg(g, [&](int r) { set(r, cf{(x | g[r]) == 0 ? 1.f : 0.f, 0.f}, cf{}); });
-            } else {
-              each_reg(g, [&](int r) {
-                const float2 v = G[x + g[r]];
-                set(r, cf{v.x, v.y}, cf{});
-              });
-            }
+            if (first)
+              each_reg(slot, x, [&](int r, uint64_t y) { set_a(r, cf{y == 0 ? 1.f : 0.f, 0.f}); });
+            else
+              each_reg(slot, G + x, [&](int r, const float2* p) { set_a(r, cf{p->x, p->y}); });
           },
-          [&](uint64_t th, const auto& g, auto&& get_a, auto&&) {
-            const uint64_t x = base | th;
-            each_reg(g, [&](int r) {
-              const cf va = get_a(r);
-              G[x + g[r]] = make_float2(va.x, va.y);
+          [&](uint64_t th, const auto& slot, auto&& get_a, auto&&) {
+            each_reg(slot, G + (base | th), [&](int r, float2* p) {
+              const cf v = get_a(r);
+              *p = make_float2(v.x, v.y);
             });
           });
       if (reg_run_any<false, RMAX>(A, A, ps.L, a.ops, ps.op_begin, ps.op_end, mc, NoAcc(), io))
@@ -430,19 +425,20 @@ __device__ __forceinline__ void tiled_reverse(float2* G, float2* Lg, int n, cons
           [&](uint32_t j) -> uint64_t {
             return use_tab ? tile_index_tab(0, j, ps.nlow, tab) : tile_index(0, j, ps);
           },
-          [&](uint64_t th, const auto& g, auto&& set) {
+          [&](uint64_t th, const auto& slot, auto&& set_a, auto&& set_b) {
             const uint64_t x = base | th;
-            each_reg(g, [&](int r) {
-              const float2 u = G[x + g[r]], v = Lg[x + g[r]];
-              set(r, cf{u.x, u.y}, cf{v.x, v.y});
-            });
+            each_reg(slot, G + x, [&](int r, const float2* p) { set_a(r, cf{p->x, p->y}); });
+            each_reg(slot, Lg + x, [&](int r, const float2* p) { set_b(r, cf{p->x, p->y}); });
           },
-          [&](uint64_t th, const auto& g, auto&& get_a, auto&& get_b) {
+          [&](uint64_t th, const auto& slot, auto&& get_a, auto&& get_b) {
             const uint64_t x = base | th;
-            each_reg(g, [&](int r) {
-              const cf va = get_a(r), vb = get_b(r);
-              G[x + g[r]] = make_float2(va.x, va.y);
-              Lg[x + g[r]] = make_float2(vb.x, vb.y);
+            each_reg(slot, G + x, [&](int r, float2* p) {
+              const cf v = get_a(r);
+              *p = make_float2(v.x, v.y);
+            });
+            each_reg(slot, Lg + x, [&](int r, float2* p) {
+              const cf v = get_b(r);
+              *p = make_float2(v.x, v.y);
             });
           });
       auto acc = [gacc](int, int col, double w, double) { atomicAdd(&gacc[col], 2.0 * w); };

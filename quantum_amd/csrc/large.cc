@@ -306,7 +306,8 @@ void AddDensePass(LargePlan* lp, const FusedOp& f, int n, PassPlan* pp) {
   pp->passes.push_back(p);
 }
 
-void AddPasses(LargePlan* lp, const std::vector<FusedOp>& ops, int n, int L, PassPlan* pp) {
+void AddPasses(LargePlan* lp, const std::vector<FusedOp>& ops, int n, int L, PassPlan* pp,
+               int max_r = 5) {
   for (const auto& f : ops)
     if (Popc(OpMask(f)) > std::min(L, n)) lp->too_wide = true;
   if (lp->too_wide) return;
@@ -314,7 +315,7 @@ void AddPasses(LargePlan* lp, const std::vector<FusedOp>& ops, int n, int L, Pas
   // The streaming passes keep the LDS path unless tuning level 2 asks for the
   // register engine there too; one-state 14-qubit tiles get five register
   // qubits (pass_kernel's wide instantiation).
-  SchedulePasses(ops, n, L, &passes, &lp->ops, &lp->mats, GetTuning().reg_engine >= 2 ? 5 : 0);
+  SchedulePasses(ops, n, L, &passes, &lp->ops, &lp->mats, GetTuning().reg_engine >= 2 ? max_r : 0);
   pp->passes.insert(pp->passes.end(), passes.begin(), passes.end());
 }
 
@@ -435,7 +436,7 @@ Status BuildLargePlan(int mode, const std::vector<Circuit>& circuits,
       std::vector<FusedOp> rev;
       BuildReverseOps(c, fo, tfq_fd, &rev);
       const size_t op0 = lp->ops.size();
-      AddPasses(lp.get(), rev, lc.n, lc.L, &lc.rev);
+      AddPasses(lp.get(), rev, lc.n, lc.L, &lc.rev, kTwoStatePass);
       // Number gradient partial slots in pass order so each pass owns a
       // contiguous slot range; param_cols maps slot -> accumulator index.
       // Inner-product gradients take two slots per derivative (real part,

@@ -99,7 +99,8 @@ constexpr int kDenseTile = 12;
 
 // Group fused ops into tile passes (exposed for tests of the scheduler).
 // max_r: largest register-engine register count for the passes (0: LDS path
-// only; 4: tiles of 12-13 qubits; 5: also 14-qubit one-state tiles).
+// only; 4: tiles of 12-13 qubits; 5: also 14-qubit one-state tiles;
+// kTwoStatePass: two-state streaming passes).
 // With `rec` (and the circuit `c` the ops come from), each op's matrix recipe
 // is recorded for rebinding.
 void SchedulePasses(const std::vector<FusedOp>& ops, int n, int L, std::vector<DevPass>* passes,

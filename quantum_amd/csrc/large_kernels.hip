@@ -69,7 +69,8 @@ struct PassArgs {
 // on 14-qubit tiles (128 KiB of LDS, one workgroup per CU) with the VGPR budget of
 // two waves per SIMD.
 template <bool TWO, bool CPLX, int ENG>
-__global__ __launch_bounds__(kThreads, (TWO || ENG == 5) ? 2 : 4) void pass_kernel(PassArgs a) {
+__global__ __launch_bounds__(TWO && ENG == 3 ? 2 * kThreads : kThreads,
+                             (TWO && ENG != 3) || ENG == 5 ? 2 : 4) void pass_kernel(PassArgs a) {
   constexpr int kPacc = TWO ? (CPLX ? 2 : 1) * kMaxPassDerivs : 1;
   extern __shared__ float2 lds[];
   __shared__ double red[kWaves];
@@ -91,6 +92,16 @@ __global__ __launch_bounds__(kThreads, (TWO || ENG == 5) ? 2 : 4) void pass_kern
   if (TWO)
     for (int k = tid; k < kPacc; k += kThreads) pacc[k] = 0.0;
   __syncthreads();
+  // The tile's first and last register layouts are those of every tile.
+  TileIndex<ENG ? ENG : 1> first, last;
+  if constexpr (ENG > 0) {
+    auto index = [&](uint32_t j) -> uint64_t {
+      return use_tab ? tile_index_tab(0, j, nlow, tab) : tile_index(0, j, ps);
+    };
+    const DevOp op = load_op(a.ops + ps.op_begin);
+    first = tile_index_of<ENG, false>(op.dmat[0], L, index);
+    last = tile_index_of<ENG, false>(op.dmat[1], L, index);
+  }
   for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const uint64_t base = tile_base_of(t, ps);
     auto gidx = [&](uint32_t j) -> uint64_t {
@@ -103,36 +114,30 @@ __global__ __launch_bounds__(kThreads, (TWO || ENG == 5) ? 2 : 4) void pass_kern
     };
     if constexpr (ENG > 0) {
       // The tile goes straight between memory and registers.
-      auto io = tile_io_indexed(
-          [&](uint32_t j) -> uint64_t {
-            return use_tab ? tile_index_tab(0, j, nlow, tab) : tile_index(0, j, ps);
-          },
-          [&](uint64_t th, const auto& g, auto&& set) {
+      auto io = tile_io_fixed(
+          first, last,
+          [&](uint64_t th, const auto& slot, auto&& set_a, auto&& set_b) {
             const uint64_t x = base | th;
             if (TWO) {
-              each_reg(g, [&](int r) {
-                const float2 u = a.psi[x + g[r]], v = a.lam[x + g[r]];
-                set(r, cf{u.x, u.y}, cf{v.x, v.y});
-              });
+              each_reg(slot, a.psi + x, [&](int r, const float2* p) { set_a(r, cf{p->x, p->y}); });
+              each_reg(slot, a.lam + x, [&](int r, const float2* p) { set_b(r, cf{p->x, p->y}); });
             } else if (a.init) {
-              each_reg(g, [&](int r) { set(r, cf{(x | g[r]) == 0 ? 1.f : 0.f, 0.f}, cf{}); });
+              each_reg(slot, x, [&](int r, uint64_t y) { set_a(r, cf{y == 0 ? 1.f : 0.f, 0.f}); });
             } else {
-              each_reg(g, [&](int r) {
-                const float2 u = a.src[x + g[r]];
-                set(r, cf{u.x, u.y}, cf{});
-              });
+              each_reg(slot, a.src + x, [&](int r, const float2* p) { set_a(r, cf{p->x, p->y}); });
             }
           },
-          [&](uint64_t th, const auto& g, auto&& get_a, auto&& get_b) {
+          [&](uint64_t th, const auto& slot, auto&& get_a, auto&& get_b) {
             const uint64_t x = base | th;
-            each_reg(g, [&](int r) {
-              const cf va = get_a(r);
-              (TWO ? a.psi : a.dst)[x + g[r]] = make_float2(va.x, va.y);
-              if (TWO) {
-                const cf vb = get_b(r);
-                a.lam[x + g[r]] = make_float2(vb.x, vb.y);
-              }
+            each_reg(slot, (TWO ? a.psi : a.dst) + x, [&](int r, float2* p) {
+              const cf v = get_a(r);
+              *p = make_float2(v.x, v.y);
             });
+            if (TWO)
+              each_reg(slot, a.lam + x, [&](int r, float2* p) {
+                const cf v = get_b(r);
+                *p = make_float2(v.x, v.y);
+              });
           });
       reg_run<ENG, TWO, false>(A, Bf, L, a.ops, ps.op_begin, ps.op_end, mc, acc, io);
       continue;
@@ -196,9 +201,9 @@ __global__ __launch_bounds__(kThreads, (TWO || ENG == 5) ? 2 : 4) void pass_kern
 }
 
 // The engine a pass was planned for (its op list starts with a remap, or not).
-int pass_engine(const LargePlan& p, const DevPass& ps) {
+int pass_engine(const LargePlan& p, const DevPass& ps, bool two) {
   if (ps.op_begin >= ps.op_end || p.ops[ps.op_begin].type != kOpRemap) return 0;
-  return RegBitsForTile(ps.L, 5);
+  return PassRegBits(ps.L, two ? kTwoStatePass : 5);
 }
 template <bool TWO, bool CPLX>
 void launch_pass(const PassArgs& a, int eng, int grid, size_t lds, hipStream_t stream) {
@@ -208,7 +213,8 @@ void launch_pass(const PassArgs& a, int eng, int grid, size_t lds, hipStream_t s
   } else if (eng == 4) {
     hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 4>), dim3(grid), dim3(kThreads), lds, stream, a);
   } else if (eng == 3) {
-    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 3>), dim3(grid), dim3(kThreads), lds, stream, a);
+    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 3>), dim3(grid), dim3(1 << (a.pass.L - 3)), lds,
+                       stream, a);
   } else {
     hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 0>), dim3(grid), dim3(kThreads), lds, stream, a);
   }
@@ -938,7 +944,7 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
       const uint64_t ntiles = uint64_t(1) << (n - ps.L);
       const int g = int(std::min<uint64_t>(ntiles, uint64_t(grid)));
       const size_t lds = (size_t(1) << ps.L) * sizeof(float2);
-      launch_pass<false, false>(a, pass_engine(*p, ps), g, lds, stream);
+      launch_pass<false, false>(a, pass_engine(*p, ps, false), g, lds, stream);
       first = false;
     }
     if (first) {  // no ops at all: still need |0>
@@ -1083,8 +1089,8 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
         const uint64_t ntiles = uint64_t(1) << (n - ps.L);
         const int g = int(std::min<uint64_t>(ntiles, uint64_t(grid)));
         const size_t lds = 2 * (size_t(1) << ps.L) * sizeof(float2);
-        if (cplx) launch_pass<true, true>(a, pass_engine(*p, ps), g, lds, stream);
-        else launch_pass<true, false>(a, pass_engine(*p, ps), g, lds, stream);
+        if (cplx) launch_pass<true, true>(a, pass_engine(*p, ps, true), g, lds, stream);
+        else launch_pass<true, false>(a, pass_engine(*p, ps, true), g, lds, stream);
         // Partial slots of a pass are contiguous [s0, s0 + nd) (numbered at planning).
         int s0 = -1, nd = 0;
         for (int i = ps.op_begin; i < ps.op_end; ++i) {

@@ -308,7 +308,7 @@ __device__ __forceinline__ void lds_run(float2* A, float2* B, int n, const DevOp
     cache_span(mc, op0.mat, op_mat_len(op0));
     if (threadIdx.x < 64u)
       lds_ops_run<REV, KMAX, true, CPLX>(A, B, n, ops, b, e, mc, win, ring, acc_fn);
-    mc.lo = mc.hi = 0;  // the others do not know where the window is now
+    mc.lo = mc.hi = kNoWindow;  // the others do not know where the window is now
     __syncthreads();
     return;
   }

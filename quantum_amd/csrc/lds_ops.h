@@ -115,11 +115,12 @@ __device__ __forceinline__ void for_ops(const DevOp* ops, int b, int e, const fl
   }
 }
 
-// v + (v of the lane that DPP control CTRL selects within the lane's row of 16).
+// v + (v of the lane that DPP control CTRL selects within the lane's row of 16; every
+// lane selects one, so no old value is set up first).
 template <int CTRL>
 __device__ __forceinline__ double dpp_add(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
   return v + __hiloint2double(hi, lo);
 }
 __device__ __forceinline__ double lane_value(double v, int lane) {

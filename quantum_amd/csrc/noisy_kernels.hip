@@ -268,15 +268,15 @@ __device__ __forceinline__ void wave_chunk(const NoisyArgs& a, const DevChunk& c
   const int fb = uniform(c.fwd_begin), fe = uniform(c.fwd_end);
   if (fb < fe) {
     auto fio = tile_io(
-        [N](uint64_t t, const auto& g, auto&& set) {
-          each_reg(g, [&](int r) {
-            set(r, cf{(uint32_t(t | g[r]) & (N - 1u)) == 0u ? 1.f : 0.f, 0.f}, cf{});
+        [N](uint64_t t, const auto& slot, auto&& set_a, auto&&) {
+          each_reg(slot, uint32_t(t), [&](int r, uint32_t x) {
+            set_a(r, cf{(x & (N - 1u)) == 0u ? 1.f : 0.f, 0.f});
           });
         },
-        [P](uint64_t t, const auto& g, auto&& get_a, auto&&) {
-          each_reg(g, [&](int r) {
-            const cf va = get_a(r);
-            P[uint32_t(t | g[r])] = make_float2(va.x, va.y);
+        [P](uint64_t t, const auto& slot, auto&& get_a, auto&&) {
+          each_reg(slot, uint32_t(t), [&](int r, uint32_t x) {
+            const cf v = get_a(r);
+            P[x] = make_float2(v.x, v.y);
           });
         });
     GlobalMats gm{a.mats};

@@ -225,7 +225,7 @@ void SetTuning(const Tuning& t) {
 
 void InsertRemaps(std::vector<DevOp>* ops, size_t begin, int L, int max_r) {
   if (!g_reg_engine.load()) return;
-  InsertRemapsR(ops, begin, L, RegBitsForTile(L, max_r));
+  InsertRemapsR(ops, begin, L, PassRegBits(L, max_r));
 }
 
 void InsertRemapsR(std::vector<DevOp>* ops, size_t begin, int L, int R) {

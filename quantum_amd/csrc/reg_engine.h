@@ -23,9 +23,9 @@
 // code path it takes (AnnotateEngine), so the device decodes nothing.
 //
 // Bound by instruction issue: per tile of a 28-qubit pass (13 qubits, 8.4 two-qubit
-// ops and 2.8 remaps) a wavefront issues 1226 VALU instructions, 535 of them MFMA,
-// and 939 SALU (in place, and with slots and layouts decoded on the device: 2062 and
-// 1954), and the pass takes 1.41 ms (1.83 ms); copying the state takes 0.89 ms.
+// ops and 2.8 remaps) a wavefront issues 1173 VALU instructions, 535 of them MFMA,
+// and 738 SALU (in place, and with slots and layouts decoded on the device: 2062 and
+// 1954), and the pass takes 1.35 ms (1.83 ms); copying the state takes 0.89 ms.
 //
 // Op matrices are read from an LDS window over the plan's matrix array,
 // refilled when an op's matrices fall outside it.  Parameterised ops (reverse
@@ -148,6 +148,20 @@ __device__ __forceinline__ uint32_t thread_base(uint32_t slots, int L) {
 #pragma unroll
   for (int j = 0; j < R; ++j) x = insert_zero(x, (slots >> (4 * j)) & 15u);
   return x;
+}
+
+// A slot map's tile bits in ascending order.
+template <int R>
+__device__ __forceinline__ uint32_t ascending_slots(uint32_t slots) {
+  uint32_t mask = 0, out = 0;
+#pragma unroll
+  for (int j = 0; j < R; ++j) mask |= slot_bit(slots, j);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    out |= uint32_t(__builtin_ctz(mask)) << (4 * j);
+    mask &= mask - 1u;
+  }
+  return out;
 }
 
 // Byte offsets in LDS of the 2^R registers: register i's index is tbase XOR
@@ -290,8 +304,9 @@ __device__ __forceinline__ void reg_dense(const Regs<R>& in, Regs<R>& out, const
 }
 
 // Derivative d of a parameterised op: this thread's <dG u | lam> with u after the
-// op (out's slots) and lam before it (in's slots).
-template <int R, int SA, int SB>
+// op (out's slots) and lam before it (in's slots).  CTRL: the op has controls (a
+// kernel-uniform test inside would become selects on every op).
+template <int R, int SA, int SB, bool CTRL>
 __device__ __forceinline__ void reg_deriv(const Regs<R>& u, const Regs<R>& lam, const MfmaRows& m,
                                           const DevOp& op, bool ok, float& part, float& part_im) {
   part = part_im = 0.f;
@@ -304,7 +319,7 @@ __device__ __forceinline__ void reg_deriv(const Regs<R>& u, const Regs<R>& lam, 
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const cf l = lam.get(idx[s]);
-      if (op.cmask && !ctrl_ok(op, ok, idx[s])) dr[s] = di[s] = 0.f;
+      if (CTRL && !ctrl_ok(op, ok, idx[s])) dr[s] = di[s] = 0.f;
       part = __builtin_fmaf(dr[s], l.x, part);
       part = __builtin_fmaf(di[s], l.y, part);
       part_im = __builtin_fmaf(dr[s], l.y, part_im);
@@ -590,12 +605,13 @@ __device__ __forceinline__ void reg_channel(const Regs<R>& in, Regs<R>& out,
 struct MatCache {
   float2* lds;  // n entries
   const float2* g;
-  uint32_t lo, hi;
+  uint32_t lo, hi;  // kNoWindow: nothing there yet
   uint32_t n;
 };
+constexpr uint32_t kNoWindow = 1u << 31;  // past every offset
 __device__ __forceinline__ MatCache mat_cache(float2* lds, const float2* g,
                                               uint32_t n = kMatCache) {
-  return MatCache{lds, g, 0u, 0u, n};
+  return MatCache{lds, g, kNoWindow, kNoWindow, n};
 }
 // Make entries [off, off + len) resident in the window (every plan pads its
 // matrix array by at least its kernel's window, so a refill stays inside).
@@ -623,7 +639,10 @@ struct GlobalMats {
 // Make an op's matrices readable and return the array its offsets index
 // (offsets rebased to the LDS window when cached).
 __device__ __forceinline__ const float2* mats_for(MatCache& c, DevOp& op) {
-  cache_span(c, op.mat, op_mat_len(op));
+  // Room for the longest op (one compare against the window's start, where the
+  // op's own length takes a dozen scalar instructions per op).
+  constexpr uint32_t kLongest = 16u * (1u + kMaxDeriv);
+  if (op.mat - c.lo > c.n - kLongest) cache_span(c, op.mat, c.n);
   op.mat -= c.lo;
   op.dmat[0] -= c.lo;
   op.dmat[1] -= c.lo;
@@ -648,23 +667,66 @@ __device__ __forceinline__ void esync() {
 // Tile I/O of the engine.  LdsIO: the tile enters and leaves in LDS buffers A
 // (and B) in the natural layout; the caller synchronises before the run and
 // the engine synchronises before returning.  TileIO: the first remap loads the
-// registers straight from memory with load(thread, reg, set) and the run ends with
-// store(thread, reg, get): register r's amplitude has index thread | reg[r] and
-// goes through set(r, a, b) or get_a(r) and get_b(r) (b only in the reverse sweep).
+// registers straight from memory with load(thread, slot, set_a, set_b) and the run ends with
+// store(thread, slot, get_a, get_b): register r's amplitude has index thread + the
+// sum of slot[j] over the set bits j of r, and goes through set_a(r, v) or get_a(r)
+// (set_b, get_b: the second state of the reverse sweep).
 // LDS is then used only by the remaps in between, and no barrier surrounds the run
 // (a remap's own barriers order its LDS use).  `thread` is index(x) of this
-// thread's own tile bits x, and `reg`, which is wave-uniform, index of the
-// register's; index must be OR-linear over disjoint bits (a tile's bits
+// thread's own tile bits x, and slot[j], which is wave-uniform, index of slot j's
+// bit; index must be OR-linear over disjoint bits (a tile's bits
 // deposited into the global index).
 struct LdsIO {};
 struct IdentityIndex {
   __device__ __forceinline__ uint64_t operator()(uint32_t x) const { return x; }
 };
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  return uint64_t(uint32_t(uniform(int(uint32_t(x))))) |
+         (uint64_t(uint32_t(uniform(int(uint32_t(x >> 32))))) << 32);
+}
+// Global index parts of this thread's tile bits and of each register slot.
+template <int R>
+struct TileIndex {
+  uint64_t thread;
+  uint64_t slot[R];
+};
+template <int R, bool WAVE, typename IndexFn>
+__device__ __forceinline__ TileIndex<R> tile_index_of(uint32_t slots, int L, IndexFn&& index) {
+  TileIndex<R> t;
+  t.thread = index(thread_base<R, WAVE>(ascending_slots<R>(slots), L));
+#pragma unroll
+  for (int j = 0; j < R; ++j) t.slot[j] = uniform64(index(slot_bit(slots, j)));
+  return t;
+}
 template <typename LoadFn, typename StoreFn, typename IndexFn = IdentityIndex>
 struct TileIO {
   LoadFn load;
   StoreFn store;
   IndexFn index;
+  template <int R, bool WAVE>
+  __device__ __forceinline__ TileIndex<R> in(uint32_t slots, int L) const {
+    return tile_index_of<R, WAVE>(slots, L, index);
+  }
+  template <int R, bool WAVE>
+  __device__ __forceinline__ TileIndex<R> out(uint32_t slots, int L) const {
+    return tile_index_of<R, WAVE>(slots, L, index);
+  }
+};
+// The same with the index parts of the first and last layout worked out by the caller
+// (they are those of every tile of a pass).
+template <int N, typename LoadFn, typename StoreFn>
+struct FixedTileIO {
+  LoadFn load;
+  StoreFn store;
+  TileIndex<N> first, last;
+  template <int R, bool WAVE>
+  __device__ __forceinline__ TileIndex<R> in(uint32_t, int) const {
+    return first;
+  }
+  template <int R, bool WAVE>
+  __device__ __forceinline__ TileIndex<R> out(uint32_t, int) const {
+    return last;
+  }
 };
 template <typename LoadFn, typename StoreFn>
 __device__ __forceinline__ TileIO<LoadFn, StoreFn> tile_io(LoadFn l, StoreFn s) {
@@ -675,31 +737,27 @@ __device__ __forceinline__ TileIO<LoadFn, StoreFn, IndexFn> tile_io_indexed(Inde
                                                                             StoreFn s) {
   return TileIO<LoadFn, StoreFn, IndexFn>{l, s, i};
 }
-__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
-  return uint64_t(uint32_t(uniform(int(uint32_t(x))))) |
-         (uint64_t(uint32_t(uniform(int(uint32_t(x >> 32))))) << 32);
+template <int R, typename LoadFn, typename StoreFn>
+__device__ __forceinline__ FixedTileIO<R, LoadFn, StoreFn> tile_io_fixed(const TileIndex<R>& first,
+                                                                         const TileIndex<R>& last,
+                                                                         LoadFn l, StoreFn s) {
+  return FixedTileIO<R, LoadFn, StoreFn>{l, s, first, last};
 }
-// f(r) for every register r of g.
-template <size_t N, typename F>
-__device__ __forceinline__ void each_reg(const uint64_t (&)[N], F&& f) {
+// f(r, x + register r's part) for every register; x: an index or a pointer.  Each is
+// one add from the one without its highest slot (sums of the parts kept in scalar
+// registers: two scalar instructions a register more, and 32 registers).
+template <size_t R, typename T, typename F>
+__device__ __forceinline__ void each_reg(const uint64_t (&slot)[R], T x, F&& f) {
+  T p[1 << R];
+  p[0] = x;
 #pragma unroll
-  for (int r = 0; r < int(N); ++r) f(r);
-}
-// Global index parts of the 2^R registers (wave-uniform).
-template <int R>
-struct RegIndex {
-  uint64_t g[1 << R];
-  template <typename IO>
-  __device__ __forceinline__ RegIndex(uint32_t slots, IO& io) {
-    g[0] = 0;
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const uint64_t gj = uniform64(io.index(slot_bit(slots, j)));
-#pragma unroll
-      for (int r = 0; r < (1 << j); ++r) g[r | (1 << j)] = g[r] | gj;
-    }
+  for (int r = 1; r < (1 << R); ++r) {
+    const int h = 31 - __builtin_clz(uint32_t(r));
+    p[r] = p[r ^ (1 << h)] + slot[h];
   }
-};
+#pragma unroll
+  for (int r = 0; r < (1 << R); ++r) f(r, p[r]);
+}
 template <typename IO>
 struct IsLdsIO {
   static constexpr bool value = false;
@@ -792,7 +850,8 @@ __device__ __forceinline__ void run_op(const Regs<R>& ra, const Regs<R>& rb, Reg
         MfmaRows dm;
         engine_rows<false>(mats + (d == 0 ? op.dmat[0] : op.dmat[1]), op, dm);
         float re, im;
-        reg_deriv<R, SA.value, SB.value>(oa, rb, dm, op, ok, re, im);
+        if (op.cmask) reg_deriv<R, SA.value, SB.value, true>(oa, rb, dm, op, ok, re, im);
+        else reg_deriv<R, SA.value, SB.value, false>(oa, rb, dm, op, ok, re, im);
         if (d == 0) {
           part[0] = re;
           part[kMaxDeriv] = im;
@@ -843,11 +902,9 @@ __device__ __forceinline__ void reg_run(float2* __restrict__ A, float2* __restri
     reg_load<R>(xa, A, off);
     if (REV) reg_load<R>(xb, B, off);
   } else {
-    const RegIndex<R> reg(first.dmat[0], io);
-    io.load(io.index(st.tbase), reg.g, [&](int r, cf va, cf vb) {
-      xa.set(r, va);
-      if (REV) xb.set(r, vb);
-    });
+    const TileIndex<R> t = io.template in<R, WAVE>(first.dmat[0], L);
+    io.load(t.thread, t.slot, [&](int r, cf v) { xa.set(r, v); },
+            [&](int r, cf v) { xb.set(r, v); });
   }
   auto finish = [&](Regs<R>& ra, Regs<R>& rb) {
     if constexpr (kLds) {
@@ -858,8 +915,8 @@ __device__ __forceinline__ void reg_run(float2* __restrict__ A, float2* __restri
       if (REV) reg_store<R>(rb, B, off);
       esync<WAVE>();
     } else {
-      const RegIndex<R> reg(first.dmat[1], io);
-      io.store(io.index(st.tbase), reg.g, [&](int r) { return ra.get(r); },
+      const TileIndex<R> t = io.template out<R, WAVE>(first.dmat[1], L);
+      io.store(t.thread, t.slot, [&](int r) { return ra.get(r); },
                [&](int r) { return rb.get(r); });
     }
   };

@@ -60,6 +60,15 @@ constexpr int RegBitsForTile(int L, int max_r = 4) {
   return (L >= 12 && L - kRegThreadBits <= max_r) ? L - kRegThreadBits : 0;
 }
 
+// Register qubits of a pass: two-state streaming passes (max_r = kTwoStatePass) on
+// 13-qubit tiles take three, the tile's other ten qubits on 1024 threads.  Their
+// LDS lets one workgroup on a CU, and sixteen wavefronts hide more latency there than
+// eight: 518 us a pass of 24 qubits (533 us with four register qubits).
+constexpr int kTwoStatePass = -1;
+constexpr int PassRegBits(int L, int max_r) {
+  return max_r != kTwoStatePass ? RegBitsForTile(L, max_r) : L == 13 ? 3 : RegBitsForTile(L);
+}
+
 // Wave mode of the batched kernel: after the workgroup-sized circuits, each
 // wavefront runs one small circuit (kWaveRegBits..kWaveMaxQubits qubits) in
 // registers, kWaveRegBits register qubits per lane and the rest on lane bits.

@@ -458,7 +458,8 @@ __device__ __forceinline__ void tiled_reverse(float2* G, float2* Lg, int n, cons
 // Modes that keep one state in LDS (at most 64 KiB up to 13 qubits) cap their
 // VGPRs at 128 so two workgroups share a CU (four wavefronts per SIMD): on
 // 11-13-qubit expectation batches that runs 1.4-1.5x faster than 190 VGPRs
-// at one workgroup per CU, the spills it costs included.
+// at one workgroup per CU, the general kernels' spills included (the register-engine
+// kernels need 100-107).
 // The LDS engine needs few registers in every mode.
 constexpr int BatchMinWaves(int mode, int var) {
   return (var == kVariantLds || mode == kModeExpectation || mode == kModeState ||

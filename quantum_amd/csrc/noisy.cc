@@ -45,11 +45,6 @@ DevOp ChannelOp(const Channel& ch, int ordinal, std::vector<cfloat>* mats) {
           mats->push_back(cfloat(float(e.real()), float(e.imag())));
         }
     }
-    bool diag = true;
-    for (int k = 0; k < ch.nk; ++k)
-      diag = diag && (*mats)[d.dmat[0] + 4 * k + 1] == cfloat(0) &&
-             (*mats)[d.dmat[0] + 4 * k + 2] == cfloat(0);
-    if (diag) d.cval |= kChanDiagonal;
   }
   bool real = true;
   for (int i = 0; i < 4 * ch.nk; ++i) real = real && (*mats)[d.mat + size_t(i)].imag() == 0.0f;

@@ -490,14 +490,14 @@ struct ChannelPick {
   float scale;
 };
 
-// This lane's part of the reduced density matrix of register slot J's qubit: |x0|^2,
-// |x1|^2 and (FULL) conj(x0) x1.  Every product is added to a sum that starts from a
-// value the compiler does not know: it would compute the sums of all slots before
-// looking at the op, for every op (2.2x this kernel's FP32 instructions).
-template <int R, int J, bool FULL>
-__device__ __forceinline__ void reg_density(const Regs<R>& a, float (&d)[FULL ? 4 : 2]) {
+// This lane's part of |x0|^2 and |x1|^2 summed over register slot J's qubit.  Every
+// product is added to a sum that starts from a value the compiler does not know: it
+// would compute the sums of all slots before looking at the op, for every op (2.2x
+// this kernel's FP32 instructions).
+template <int R, int J>
+__device__ __forceinline__ void reg_density(const Regs<R>& a, float (&d)[2]) {
 #pragma unroll
-  for (int i = 0; i < (FULL ? 4 : 2); ++i) {
+  for (int i = 0; i < 2; ++i) {
     d[i] = 0.f;
     asm volatile("" : "+v"(d[i]));
   }
@@ -507,10 +507,6 @@ __device__ __forceinline__ void reg_density(const Regs<R>& a, float (&d)[FULL ? 
     const cf x0 = a.get(i0), x1 = a.get(i0 | (1 << J));
     d[0] = __builtin_fmaf(x0.y, x0.y, __builtin_fmaf(x0.x, x0.x, d[0]));
     d[1] = __builtin_fmaf(x1.y, x1.y, __builtin_fmaf(x1.x, x1.x, d[1]));
-    if constexpr (FULL) {
-      d[2] = __builtin_fmaf(x0.y, x1.y, __builtin_fmaf(x0.x, x1.x, d[2]));
-      d[3] = __builtin_fmaf(-x0.y, x1.x, __builtin_fmaf(x0.x, x1.y, d[3]));
-    }
   }
 }
 // The first k with u < p_0 + ... + p_k, the last k with p_k > 0 when none.
@@ -535,7 +531,8 @@ __device__ __forceinline__ ChannelPick pick_kraus(int nk, double u, Prob&& prob)
 }
 
 // Unitary mixtures pick unitary k with the first u < cum[k]; other channels take
-// p_k = <psi|K_k^dag K_k|psi> from the qubit's reduced density matrix, pick the
+// p_k = <psi|K_k^dag K_k|psi> from the qubit's populations (K_k^dag K_k is diagonal
+// for every channel kind: its K_k have at most one entry in a row and column), pick the
 // first k with u < p_0 + ... + p_k (the last k with p_k > 0 when none) and apply
 // K_k / sqrt(p_k).  Lanes of different trajectories may pick different operators.
 template <int R>
@@ -551,30 +548,18 @@ __device__ __forceinline__ ChannelPick channel_pick(const Regs<R>& a, const DevO
       if (u < double(X[k].x)) pick = k;
     return ChannelPick{pick, 1.0f};
   }
-  if (op.cval & kChanDiagonal) {
-    float s[2];
-    for_slot<R>(int(op.code), [&](auto J) { reg_density<R, J.value, false>(a, s); });
-    double d[2] = {double(s[0]), double(s[1])};
-    group_sums(d, nd.gbits);
-    return pick_kraus(nk, u, [&](int k) {
-      return double(X[4 * k].x) * d[0] + double(X[4 * k + 3].x) * d[1];
-    });
-  }
-  float s[4];
-  for_slot<R>(int(op.code), [&](auto J) { reg_density<R, J.value, true>(a, s); });
-  double d[4] = {double(s[0]), double(s[1]), double(s[2]), double(s[3])};
+  float s[2];
+  for_slot<R>(int(op.code), [&](auto J) { reg_density<R, J.value>(a, s); });
+  double d[2] = {double(s[0]), double(s[1])};
   group_sums(d, nd.gbits);
   return pick_kraus(nk, u, [&](int k) {
-    const float2 e01 = X[4 * k + 1];
-    return double(X[4 * k].x) * d[0] + double(X[4 * k + 3].x) * d[1] +
-           2.0 * (double(e01.x) * d[2] - double(e01.y) * d[3]);
+    return double(X[4 * k].x) * d[0] + double(X[4 * k + 3].x) * d[1];
   });
 }
 
 // out = the picked operator on register slot J of in; the matrix is read per lane.
 // Bound by the number of VALU instructions: with real matrices half the products
-// go, and with diagonal K^dag K half of the density's and of its lane sums (every
-// channel here that is no unitary mixture is both): 717 us (965 us) for 32 rows of
+// go (every channel that is no unitary mixture has them): 688 us (965 us) for 32 rows of
 // 1000 8-qubit trajectories with 128 channels.
 template <int R, int J, bool REAL>
 __device__ __forceinline__ void reg_channel(const Regs<R>& in, Regs<R>& out,

@@ -36,8 +36,7 @@ enum OpType : uint8_t {
 // (its random stream).
 constexpr uint32_t kChanMixture = 1u << 8;    // unitary mixture
 constexpr uint32_t kChanFirstIdentity = 1u << 9;  // unitary 0 is the identity
-constexpr uint32_t kChanDiagonal = 1u << 10;  // every K_k^dag K_k is diagonal
-constexpr uint32_t kChanReal = 1u << 11;      // every K_k is real
+constexpr uint32_t kChanReal = 1u << 10;      // every K_k is real
 constexpr int ChanKraus(uint32_t cval) { return int(cval & 15u); }
 
 // Register engine (reg_engine.h): 2^9 threads per workgroup, each holding

@@ -2,11 +2,10 @@
 // tile, fused ops of at most two qubits; the register engine takes the tiles of
 // 12-13 qubits).
 //
-// A lane owns a group of four amplitudes, the four values of two qubits: the
-// op's targets, or a one-qubit op's target and another qubit.  It loads them
-// from LDS, multiplies by the 4x4 matrix on v_mfma_f32_4x4x1f32 (reg_engine.h)
-// and stores them; a barrier separates ops.  Groups whose control qubits do not
-// match run along and are not stored.
+// A lane owns the four amplitudes of a two-qubit op's targets: it loads them from
+// LDS, multiplies by the 4x4 matrix on v_mfma_f32_4x4x1f32 (reg_engine.h) and stores
+// them; a barrier separates ops.  A one-qubit op takes a pair a lane, on FMAs.  Lanes
+// whose control qubits do not match run along and store nothing.
 //
 // What bounds small circuits is the latency of one op, not work: a 10-qubit
 // op is 256 groups.  Hence
@@ -17,12 +16,15 @@
 //    (its LDS accesses are in order) without a barrier per op;
 //  - op descriptors come from an LDS window; the next one is read while an op
 //    runs (a scalar load would share the wait counter of the op's LDS reads).
-//  - gradient partials are reduced eight derivatives at a time (PartRing).
+//  - gradient partials are reduced eight at a time (PartRing).
 // Per op of a circuit that has the chip to itself (64 circuits, two-qubit ops
 // with two derivatives in the reverse sweep): 8 qubits 0.54 us forward and 1.21
 // reverse (FMA sweeps with a barrier each: 0.68 and 1.69), 10 qubits 0.60 and
 // 1.46 (0.80 and 1.87), 11 qubits 0.76 and 1.84 (1.01 and 2.29).  What is left is
 // the issue of a few hundred dependent instructions by one wavefront per SIMD.
+// One-qubit ops as MFMA groups of two pairs, the other half of the matrix zero, took
+// 657 us on 64 circuits of 10 qubits and 600 symbols (half of the symbols in one-qubit
+// ops), with a pair a lane 607.
 #pragma once
 
 #include "reg_engine.h"
@@ -64,31 +66,48 @@ __device__ __forceinline__ DevOp desc_unpack(uint32_t word) {
   return o;
 }
 
-// MFMA rows of a one-qubit matrix on index bit T of the group (identity on the
-// other bit).
+// (dr, di) = G v for a lane's group v of a two-qubit op, its products added in the
+// order of apply_dense (lds_ops.h): column 0 as cmul contracts it (the product that is
+// rounded by itself first; another one in the adjoint, where the imaginary part is a
+// difference), the others as cmacf.  So amplitudes have the bits that the FMA path gives
+// them, and a shot, drawn by comparing a prefix sum with a uniform, the same outcome.
 template <bool DAG>
-__device__ __forceinline__ void mfma_rows1(const float2* __restrict__ M, int T, MfmaRows& r) {
-  const int row = int(threadIdx.x & 3u);
-  const int rt = (row >> T) & 1, ro = (row >> (1 - T)) & 1;
-  cf m[2];
+__device__ __forceinline__ void ordered_apply(const float2 (&v)[4], const MfmaRows& m, mf4& dr,
+                                              mf4& di) {
+  const mf4 zero{0.f, 0.f, 0.f, 0.f};
+  dr = mfma4(m.gr[0], v[0].x, mfma4(m.ngi[0], v[0].y, zero));
+  di = DAG ? mfma4(m.gr[0], v[0].y, mfma4(m.gi[0], v[0].x, zero))
+           : mfma4(m.gi[0], v[0].x, mfma4(m.gr[0], v[0].y, zero));
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    m[c] = ldm(M, DAG ? c * 2 + rt : rt * 2 + c);
-    if (DAG) m[c].y = -m[c].y;
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const bool same = ((k >> (1 - T)) & 1) == ro;
-    const cf v = ((k >> T) & 1) ? m[1] : m[0];
-    r.gr[k] = same ? v.x : 0.f;
-    r.gi[k] = same ? v.y : 0.f;
-    r.ngi[k] = -r.gi[k];
+  for (int k = 1; k < 4; ++k) {
+    dr = mfma4(m.ngi[k], v[k].y, mfma4(m.gr[k], v[k].x, dr));
+    di = mfma4(m.gi[k], v[k].x, mfma4(m.gr[k], v[k].y, di));
   }
 }
-template <bool DAG>
-__device__ __forceinline__ void op_rows(const float2* __restrict__ M, int k, int t, MfmaRows& r) {
-  if (k == 2) mfma_rows<DAG>(M, r);
-  else mfma_rows1<DAG>(M, t, r);
+
+// o = the op's matrix (or its adjoint) times v, the 2^K amplitudes of a lane.  One qubit:
+// FMAs on a pair.  On MFMA a pair would need another one beside it, with zeros between
+// the two: NaN in both where one of them is not finite.
+template <int K, bool DAG>
+__device__ __forceinline__ void lane_apply(const float2* __restrict__ M, const float2 (&v)[1 << K],
+                                           float2 (&o)[1 << K]) {
+  if constexpr (K == 2) {
+    MfmaRows G;
+    mfma_rows<DAG>(M, G);
+    mf4 dr, di;
+    ordered_apply<DAG>(v, G, dr, di);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) o[s] = make_float2(dr[s], di[s]);
+  } else {
+    float2 m[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      m[i] = M[DAG ? (i & 1) * 2 + (i >> 1) : i];
+      if (DAG) m[i].y = -m[i].y;
+    }
+    o[0] = cmacf(cmul(m[0], v[0]), m[1], v[1]);
+    o[1] = cmacf(cmul(m[2], v[0]), m[3], v[1]);
+  }
 }
 
 // As cache_span, by one wavefront.
@@ -130,11 +149,101 @@ __device__ __forceinline__ void flush_parts(const PartRing<CPLX>* r, int count, 
   if (s == 0 && d < count) acc_fn(r->col[d], re, im);
 }
 
+// One dense or parameterised op of K qubits on the states A and (REV) B: 2^K amplitudes
+// a lane and round.  A derivative's partials are summed over a lane's 2^K amplitudes in
+// FP32, over everything else in FP64.
+template <int K, bool REV, bool SOLO, bool CPLX, typename AccFn>
+__device__ __forceinline__ void lds_dense(float2* __restrict__ A, float2* __restrict__ B, int n,
+                                          const DevOp& op, const float2* __restrict__ M,
+                                          PartRing<CPLX>* ring, int& parts, AccFn&& acc_fn) {
+  constexpr int D = 1 << K;
+  constexpr uint32_t kStep = SOLO ? 64u : uint32_t(kThreads);
+  const uint32_t lane = threadIdx.x & 63u, first = SOLO ? 0u : threadIdx.x & ~63u;
+  const uint32_t count = 1u << (n - K);
+  const int nd = REV && op.type == kOpParam ? op.nderiv : 0;
+  uint32_t dep[D];
+#pragma unroll
+  for (int s = 0; s < D; ++s)
+    dep[s] = (uint32_t(s & 1) << op.q[0]) | (K == 2 ? uint32_t(s >> 1) << op.q[1] : 0u);
+  double acc[2 * kMaxDeriv] = {0.0, 0.0, 0.0, 0.0};
+  if (ring && first < count) {
+    // Room for this op's partials: one per derivative and round.
+    const int need = nd * (count > kStep ? int(count / kStep) : 1);
+    if (parts + need > kPartDerivs) {
+      esync<true>();
+      flush_parts<CPLX>(ring, parts, acc_fn);
+      esync<true>();
+      parts = 0;
+    }
+    if (lane < uint32_t(need)) ring->col[parts + int(lane)] = nd > 1 && (lane & 1u) ? op.col[1] : op.col[0];
+  }
+  // Every lane runs every round: MFMA takes its operands from all lanes.
+  // Lanes past the last repeat one (and store the same values).
+  for (uint32_t g0 = first; g0 < count; g0 += kStep) {
+    const uint32_t g = g0 + lane;
+    uint32_t x0 = insert_zero(g & (count - 1u), op.q[0]);
+    if (K == 2) x0 = insert_zero(x0, op.q[1]);
+    const bool ok = (x0 & op.cmask) == op.cval;
+    float2 a[D], l[D], u[D], w[D];
+#pragma unroll
+    for (int s = 0; s < D; ++s) a[s] = A[x0 | dep[s]];
+    if constexpr (REV) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) l[s] = B[x0 | dep[s]];
+    }
+    lane_apply<K, REV>(M, a, u);
+    if constexpr (REV) lane_apply<K, REV>(M, l, w);
+    if (ok) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) A[x0 | dep[s]] = u[s];
+      if constexpr (REV) {
+#pragma unroll
+        for (int s = 0; s < D; ++s) B[x0 | dep[s]] = w[s];
+      }
+    }
+    if constexpr (REV) {
+      if (nd > 0) {
+#pragma unroll
+        for (int d = 0; d < kMaxDeriv; ++d) {
+          if (d >= nd) break;
+          float2 t[D];
+          lane_apply<K, false>(M + D * D * (1 + d), u, t);
+          float part = 0.f, part_im = 0.f;
+#pragma unroll
+          for (int s = 0; s < D; ++s) {
+            part = __builtin_fmaf(t[s].x, l[s].x, part);
+            part = __builtin_fmaf(t[s].y, l[s].y, part);
+            part_im = __builtin_fmaf(t[s].x, l[s].y, part_im);
+            part_im = __builtin_fmaf(-t[s].y, l[s].x, part_im);
+          }
+          if (g >= count || !ok) part = part_im = 0.f;
+          if (ring) {
+            ring->part[parts + d][lane] = part;
+            if constexpr (CPLX) ring->part_im[parts + d][lane] = part_im;
+          } else {
+            acc[d] += double(part);
+            acc[kMaxDeriv + d] += double(part_im);
+          }
+        }
+        if (ring) parts += nd;
+      }
+    }
+  }
+  if (REV && nd > 0 && !ring && first < count) {
+    const double w0 = wave_sum(acc[0]), v0 = wave_sum(acc[kMaxDeriv]);
+    const double w1 = wave_sum(acc[1]), v1 = wave_sum(acc[kMaxDeriv + 1]);
+    if (lane == 0u) {
+      acc_fn(op.col[0], w0, v0);
+      if (nd > 1) acc_fn(op.col[1], w1, v1);
+    }
+  }
+}
+
 // Ops [b, e) on the states A and (REV) B of n >= 2 qubits; SOLO: by this
 // wavefront alone.  acc_fn(column, re, im) gets a wavefront's <dG psi | lambda>
 // partials, from one lane each.  ring: room for this wavefront's partials, or
-// null (a lane then holds several groups' sums, or LDS is full): every
-// derivative is reduced at once.
+// null (LDS is full, or the state takes more rounds than the ring has entries):
+// every derivative is then reduced at once.
 template <bool REV, int KMAX, bool SOLO, bool CPLX, typename AccFn>
 __device__ __forceinline__ void lds_ops_run(float2* __restrict__ A, float2* __restrict__ B, int n,
                                             const DevOp* __restrict__ ops, int b, int e,
@@ -142,8 +251,7 @@ __device__ __forceinline__ void lds_ops_run(float2* __restrict__ A, float2* __re
                                             AccFn&& acc_fn) {
   constexpr uint32_t kStep = SOLO ? 64u : uint32_t(kThreads);
   const uint32_t tid = SOLO ? (threadIdx.x & 63u) : threadIdx.x;
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t N = 1u << n, ngroups = N >> 2;
+  const uint32_t N = 1u << n;
   int parts = 0;  // derivatives in the ring
   DevOp op;
   for (int i = b, at = 0; i < e; ++i, ++at) {
@@ -178,110 +286,10 @@ __device__ __forceinline__ void lds_ops_run(float2* __restrict__ A, float2* __re
     } else if (KMAX > 2 && op.k > 2) {
       apply_op<REV, KMAX>(A, n, op, M);
       if (REV) apply_op<REV, KMAX>(B, n, op, M);
+    } else if (op.k == 2) {
+      lds_dense<2, REV, SOLO, CPLX>(A, B, n, op, M, ring, parts, acc_fn);
     } else {
-      // The group's two qubits, and which of them a one-qubit op acts on.
-      const uint32_t q0 = op.k == 2 ? op.q[0] : 0u;
-      const uint32_t q1 = op.k == 2 ? op.q[1] : (op.q[0] == 0 ? 1u : op.q[0]);
-      const int t = op.k == 2 || op.q[0] == 0 ? 0 : 1;
-      const uint32_t d1 = 1u << q0, d2 = 1u << q1;
-      const int DD = 1 << (2 * op.k);
-      const int nd = REV && op.type == kOpParam ? op.nderiv : 0;
-      double acc[2 * kMaxDeriv] = {0.0, 0.0, 0.0, 0.0};
-      // Every lane runs every round: MFMA takes its operands from all lanes.
-      // Lanes past the last group repeat one (and store the same values).
-      for (uint32_t g0 = SOLO ? 0u : (tid & ~63u); g0 < ngroups; g0 += kStep) {
-        const uint32_t g = g0 + lane;
-        const uint32_t x0 = insert_zero(insert_zero(g & (ngroups - 1u), q0), q1);
-        const uint32_t x[4] = {x0, x0 | d1, x0 | d2, x0 | d1 | d2};
-        cf a[4], l[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const float2 v = A[x[s]];
-          a[s] = cf{v.x, v.y};
-        }
-        if (REV) {
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            const float2 v = B[x[s]];
-            l[s] = cf{v.x, v.y};
-          }
-        }
-        constexpr int idx[4] = {0, 1, 2, 3};
-        MfmaRows G;
-        op_rows<REV>(M, op.k, t, G);
-        mf4 ar, ai, br, bi;
-        mfma_apply(a, idx, G, ar, ai);
-        if constexpr (REV) mfma_apply(l, idx, G, br, bi);
-        if (op.cmask == 0u) {
-#pragma unroll
-          for (int s = 0; s < 4; ++s) A[x[s]] = make_float2(ar[s], ai[s]);
-          if constexpr (REV) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) B[x[s]] = make_float2(br[s], bi[s]);
-          }
-        } else {
-          // Per amplitude: a one-qubit op's other qubit may be one of its controls.
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            if ((x[s] & op.cmask) == op.cval) {
-              A[x[s]] = make_float2(ar[s], ai[s]);
-              if constexpr (REV) B[x[s]] = make_float2(br[s], bi[s]);
-            } else {
-              l[s] = cf{0.f, 0.f};  // contributes nothing below
-            }
-          }
-        }
-        if constexpr (REV) {
-          if (nd > 0) {
-            cf u[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) u[s] = cf{ar[s], ai[s]};
-#pragma unroll
-            for (int d = 0; d < kMaxDeriv; ++d) {
-              if (d >= nd) break;
-              MfmaRows D;
-              op_rows<false>(M + DD * (1 + d), op.k, t, D);
-              mf4 sr, si;
-              mfma_apply(u, idx, D, sr, si);
-              float part = 0.f, part_im = 0.f;
-#pragma unroll
-              for (int s = 0; s < 4; ++s) {
-                part = __builtin_fmaf(sr[s], l[s].x, part);
-                part = __builtin_fmaf(si[s], l[s].y, part);
-                part_im = __builtin_fmaf(sr[s], l[s].y, part_im);
-                part_im = __builtin_fmaf(-si[s], l[s].x, part_im);
-              }
-              if (g >= ngroups) part = part_im = 0.f;
-              if (ring) {  // one group per lane
-                ring->part[parts + d][lane] = part;
-                if constexpr (CPLX) ring->part_im[parts + d][lane] = part_im;
-              } else {
-                acc[d] += double(part);
-                acc[kMaxDeriv + d] += double(part_im);
-              }
-            }
-          }
-        }
-      }
-      if (REV && nd > 0 && (SOLO || (tid & ~63u) < ngroups)) {
-        if (ring) {
-          if (lane < uint32_t(nd)) ring->col[parts + int(lane)] = lane == 0u ? op.col[0] : op.col[1];
-          parts += nd;
-          if (parts > kPartDerivs - kMaxDeriv) {
-            esync<true>();
-            flush_parts<CPLX>(ring, parts, acc_fn);
-            esync<true>();
-            parts = 0;
-          }
-        } else {
-          const double w0 = wave_sum(acc[0]), v0 = wave_sum(acc[kMaxDeriv]);
-          const double w1 = wave_sum(acc[1]), v1 = wave_sum(acc[kMaxDeriv + 1]);
-          if (lane == 0u) {
-            acc_fn(op.col[0], w0, v0);
-            if (nd > 1) acc_fn(op.col[1], w1, v1);
-          }
-        }
-      }
+      lds_dense<1, REV, SOLO, CPLX>(A, B, n, op, M, ring, parts, acc_fn);
     }
     op = desc_unpack(next);
     if (SOLO) esync<true>();
@@ -299,7 +307,7 @@ __device__ __forceinline__ void lds_run(float2* A, float2* B, int n, const DevOp
                                         AccFn&& acc_fn) {
   if (b >= e) return;
   __syncthreads();
-  // One group per lane: rounds of kThreads groups.
+  // At most two rounds, so that an op's partials fit the ring.
   PartRing<CPLX>* ring =
       REV && rings && (1u << n) <= 4u * kThreads ? rings + (threadIdx.x >> 6) : nullptr;
   if (KMAX <= 2 && n <= kSoloMaxQubits) {

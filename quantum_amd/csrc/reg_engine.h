@@ -100,23 +100,6 @@ __device__ __forceinline__ void mfma_rows(const float2* __restrict__ M, MfmaRows
 __device__ __forceinline__ mf4 mfma4(float a, float b, mf4 c) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 }
-// (dr, di) = G v for the four amplitudes v_k = a[idx[k]] of every lane.
-template <int N>
-__device__ __forceinline__ void mfma_apply(const cf (&a)[N], const int (&idx)[4],
-                                           const MfmaRows& m, mf4& dr, mf4& di) {
-  dr = mf4{0.f, 0.f, 0.f, 0.f};
-  di = mf4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    dr = mfma4(m.gr[k], a[idx[k]].x, dr);
-    di = mfma4(m.gi[k], a[idx[k]].x, di);
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    dr = mfma4(m.ngi[k], a[idx[k]].y, dr);
-    di = mfma4(m.gr[k], a[idx[k]].y, di);
-  }
-}
 
 __host__ __device__ constexpr int ins0(int g, int j) {
   return ((g >> j) << (j + 1)) | (g & ((1 << j) - 1));

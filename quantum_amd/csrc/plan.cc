@@ -695,7 +695,7 @@ void AppendRecipe(const FusedOp& f, const Circuit& c, const DevOp& d, SharedReci
   r.nderiv = f.param ? f.nderiv : 0;
   for (int i = 0; i < r.nderiv; ++i) {
     r.dmat[i] = d.dmat[i];
-    r.dgate[i] = int8_t(f.dgate[i]);
+    r.dgate[i] = f.dgate[i];
     r.dsym[i] = int8_t(f.dsym[i]);
   }
   rec->ops.push_back(r);

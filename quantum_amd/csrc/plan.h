@@ -64,8 +64,8 @@ struct OpRecipe {
   uint32_t mat = 0;                  // offsets into the row's matrices
   uint32_t dmat[kMaxDeriv];
   int nderiv = 0;
-  int8_t dgate[kMaxDeriv] = {0, 0};  // kind 3: block position of each derivative's gate
-  int8_t dsym[kMaxDeriv] = {0, 1};   // ... and which of its symbols
+  int dgate[kMaxDeriv] = {0, 0};    // kind 3: block position of each derivative's gate
+  int8_t dsym[kMaxDeriv] = {0, 1};  // ... and which of its symbols
 };
 
 struct SharedRecipe {

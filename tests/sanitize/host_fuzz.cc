@@ -296,6 +296,47 @@ void ExerciseRebind(const Circuit& c, const float* vals) {
   }
 }
 
+// One block of `count` gates on two qubits with symbolic gates at `at`: the host
+// re-evaluation for the values that the plan was built with writes the plan's own
+// matrices, for per-row and for shared recipes.
+void LongBlock(int count, const std::vector<int>& at) {
+  Program p;
+  for (int i = 0; i < count; ++i) {
+    Arg e = Value(0.01f * float(i % 50) - 0.2f);
+    for (size_t s = 0; s < at.size(); ++s)
+      if (at[s] == i) e = Sym(s ? "b" : "a");
+    p.moments.push_back({i % 3 == 2 ? Op("ISP", {"0", "1"}, Eigen(e))
+                                    : Op("YP", {i % 2 ? "1" : "0"}, Eigen(e))});
+  }
+  std::unordered_map<std::string, int> cols{{"a", 0}, {"b", 1}};
+  const float vals[3] = {0.25f, -1.5f, 3.0f};
+  SymbolMap sm;
+  sm.columns = &cols;
+  sm.values = vals;
+  Circuit c;
+  if (!BuildCircuit(p, sm, &c).ok()) abort();
+  ExerciseRebind(c, vals);
+  PlanOptions opt;
+  opt.mode = kModeAdjoint;
+  opt.adjoint = opt.keep_all_lambda = true;
+  opt.fuse.max_fuse = 2;
+  opt.fuse.structural_diag = true;
+  std::vector<CircuitJob> jobs{CircuitJob{&c, nullptr, nullptr, nullptr, 0}};
+  BatchProgram prog, sprog;
+  std::vector<SharedRecipe> recipes;
+  SharedRecipe shared;
+  BuildBatchProgram(jobs, 1, 3, opt, 1, &prog, &recipes);
+  std::vector<RowRebind> rows{CompactRecipe(c, recipes[0])};
+  std::vector<cfloat> mats(prog.mats.size());
+  for (size_t i = 0; i < mats.size(); ++i) mats[i] = prog.mats[i];
+  RebindBatchProgram(rows, vals, 3, opt.tfq_fd, 1, prog, mats.data());
+  BuildSharedBatchProgram(c, jobs, vals, 3, 1, opt, 1, &sprog, &shared);
+  if (mats != prog.mats || sprog.mats != prog.mats) {
+    fprintf(stderr, "host_fuzz: a block of %d gates is re-evaluated to other matrices\n", count);
+    abort();
+  }
+}
+
 void OneProgram(const std::string& bytes, const std::vector<std::string>& sums, uint64_t* ok) {
   Program prog;
   if (!DecodeProgram(reinterpret_cast<const uint8_t*>(bytes.data()), bytes.size(), &prog)) return;
@@ -335,6 +376,11 @@ void OneProgram(const std::string& bytes, const std::vector<std::string>& sums, 
 
 int main(int argc, char** argv) {
   const long iters = argc > 1 ? atol(argv[1]) : 20000;
+  LongBlock(30, {3, 27});
+  LongBlock(128, {127});
+  LongBlock(129, {128});
+  LongBlock(300, {0, 299});
+  LongBlock(40000, {33000});
   std::mt19937_64 rng(argc > 2 ? strtoull(argv[2], nullptr, 10) : 1);
   std::vector<std::string> progs, sums = SeedSums(), texts;
   for (const auto& p : SeedPrograms()) progs.push_back(EncodeProgram(p));

@@ -311,3 +311,35 @@ def test_device_values_of_long_blocks(mode, gates, at):
     dev.stage_values(v2)
     _say(f"long block, {gates} gates, mode={mode}")
     np.testing.assert_allclose(_launch(dev, shape), _launch(host, shape), atol=MATCH)
+
+
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("gates,at", [(128, (127,)), (129, (128,)), (300, (0, 299))])
+def test_derivatives_behind_many_gates(shared, gates, at):
+    """Gradient gates at position 128 and beyond of one block: a plan rebound on the
+    device or on the host equals a plan built with the new values, within MATCH of the
+    largest output as above, and the oracle within the suite's bound."""
+    rng = np.random.default_rng(gates)
+    q = C.LineQubit.range(2)
+    names = ["a", "b"]
+    ops = []
+    for i in range(gates):
+        e = C.Symbol(names[at.index(i)]) if i in at else float(rng.uniform(-1, 1))
+        ops.append(C.ISwapPowGate(exponent=e).on(q[1], q[0]) if i % 3 == 2 else
+                   C.YPowGate(exponent=e).on(q[i % 2]))
+    circuits = [C.Circuit(ops)] * 2 + [C.Circuit(ops + [C.Z(q[0])] * (not shared))]
+    progs = S.convert_to_tensor(circuits)
+    ps = S.convert_to_tensor([[W.random_pauli_sum(rng, q, 3), W.random_pauli_sum(rng, q, 2)]] * 3)
+    v1, v2 = _values(rng, 3, 2), _values(rng, 3, 2)
+    g = rng.uniform(-1, 1, size=(3, 2)).astype(np.float32)
+    host, shape = _adjoint_plan(progs, names, v1, ps, g)
+    dev, _ = _adjoint_plan(progs, names, v1, ps, g)
+    fresh, _ = _adjoint_plan(progs, names, v2, ps, g)
+    host.rebind(v2)
+    dev.stage_values(v2)
+    _say(f"derivatives behind {gates} gates, shared={shared}")
+    want = _launch(fresh, shape)
+    tol = MATCH * max(1.0, np.abs(want).max())
+    np.testing.assert_allclose(_launch(host, shape), want, atol=tol)
+    np.testing.assert_allclose(_launch(dev, shape), want, atol=tol)
+    _check_oracle(want, progs, names, v2, ps, g, "analytic")

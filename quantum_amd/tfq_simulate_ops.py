@@ -119,10 +119,16 @@ def _run(plan, out_shape, dtype):
     return out
 
 
-def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None):
+def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None,
+                stage_new=True):
     """``launch(plan)`` with the plan of a recent call of ``op`` whose string
     tensors, names and ``extra`` arguments were the same, rebound to ``values``
-    and ``seed``, or with ``build()``'s (see ``plan_cache``)."""
+    and ``seed``, or with ``build()``'s (see ``plan_cache``).
+
+    ``stage_new``: a new plan's symbolic matrices are evaluated on the device as a
+    reused one's are.  The host's differ from those in the last bit of a sine or
+    cosine, enough to move a draw: a seeded call would return other shots the
+    second time, or once its plan has left the cache."""
     from . import plan_cache
     if not _torch().cuda.is_available():
         return launch(build())  # the inputs' own errors before the missing device
@@ -130,12 +136,18 @@ def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None):
     key = (op, plan_cache.digest(*strings), tuple(names), tuple(x.shape for x in strings),
            dev.index, stream, *extra)
 
+    def new_plan():
+        plan = build()
+        if stage_new and values.size and not plan.stats()["streaming"]:
+            plan.stage_values(values)
+        return plan
+
     def rebind(plan):
         plan.stage_values(values)
         if seed is not None:
             plan.set_seed(seed)
 
-    return plan_cache.run(key, build, rebind, launch)
+    return plan_cache.run(key, new_plan, rebind, launch)
 
 
 def _plan_args(programs, names, values):
@@ -169,7 +181,7 @@ def tfq_simulate_expectation(programs, symbol_names, symbol_values, pauli_sums):
     shape = (programs.shape[0], pauli_sums.shape[1])
     return _run_cached("expectation", (programs, pauli_sums), names, values,
                        lambda: plan_expectation(programs, names, values, pauli_sums)[0],
-                       lambda plan: _run(plan, shape, _torch().float32))
+                       lambda plan: _run(plan, shape, _torch().float32), stage_new=False)
 
 
 def tfq_simulate_state(programs, symbol_names, symbol_values):

@@ -78,3 +78,27 @@ def test_other_counts_and_shapes_are_other_plans():
     assert a.shape == (1, 10, 3) and b.shape == (1, 20, 3)
     np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy()[:, :10])
     assert len(plan_cache._CACHE) == 2
+
+
+@pytest.mark.parametrize("op", ["state", "samples", "sampled", "inner"])
+def test_equal_calls_give_equal_results(op):
+    """The same arguments as the first call, with other values in between, after the
+    plan has left the cache, and without a cache: the same bits.  A gate and its inverse
+    leave matrix entries in which the last bit of a sine or cosine shows."""
+    B = 64
+    q = C.LineQubit.range(2)
+    a = C.Symbol("a")
+    circuit = C.Circuit([C.XPowGate(exponent=e).on(x) for e in (a, a * -1.0) for x in q])
+    progs = S.convert_to_tensor([circuit] * B)
+    sums = S.convert_to_tensor([[C.PauliSum([C.PauliString({q[0]: "X"}, 0.7)])] * 2] * B)
+    other = S.convert_to_tensor([[C.Circuit([C.I(x) for x in q])] * 2] * B)
+    fn, _ = _ops(progs, ["a"], sums, other)[op]
+    v = np.random.default_rng(8).uniform(-3, 3, (B, 1)).astype(np.float32)
+    print(f"[gpu-case] equal calls, {op}", flush=True)
+    first = fn(v, 3).cpu().numpy()
+    fn(np.zeros_like(v), 4)
+    np.testing.assert_array_equal(fn(v, 3).cpu().numpy(), first)
+    plan_cache.clear()
+    np.testing.assert_array_equal(fn(v, 3).cpu().numpy(), first)
+    plan_cache.set_capacity(0)
+    np.testing.assert_array_equal(fn(v, 3).cpu().numpy(), first)

@@ -3,12 +3,12 @@
 The reference parses, resolves and fuses every program on every call
 (``core/ops/parse_context.cc:60-92``).  Here an op call whose programs, symbol
 names and Pauli sums (or paired programs) are byte-identical to a recent call's
-reuses that call's plan, and a sampling op's new seed is set in it: only the symbolic gate matrices are re-evaluated for the new symbol
-values (on the device, ``tfqx_plan_stage_values``), and for the adjoint the
-lambda weights for the new downstream gradients
-(``tfqx_plan_rebind_downstream``); the upload then carries only what changed
-(``tfqx_plan_upload_changed``).  A training loop therefore pays the host
-planner once.
+reuses that call's plan, and a sampling op's new seed is set in it: only the
+symbolic gate matrices are re-evaluated for the new symbol values (on the
+device, ``tfqx_plan_stage_values``), and for the adjoint the lambda weights for
+the new downstream gradients (``tfqx_plan_rebind_downstream``); the upload then
+carries only what changed (``tfqx_plan_upload_changed``).  A training loop
+therefore pays the host planner once.
 
 Keys hold a 128-bit xxh3 digest of the string tensors' bytes and offsets, the
 symbol names, the shapes, the op's other arguments, the caller's stream and
@@ -16,8 +16,13 @@ the planner's settings generation (bumped by every fusion/tuning setter), so a
 changed setting never reuses a plan built under the old one.  Plans on the
 HBM-streaming path and noisy plans cannot be rebound and are not cached.
 
-Entries are least-recently-used, at most ``set_capacity(n)`` of them (default
-8; 0 disables the cache).  A per-entry lock serialises rebind + upload + launch
+Entries are least-recently-used, at most ``set_capacity(n)`` of a group (default
+8; 0 disables the cache).  The ops of a training loop (expectations and
+gradients) are one group, the others (states, draws, overlaps) another, so that
+calls of one kind do not push out plans of the other.  The second group's plans
+can hold large states and were built for one call as often as not: together
+they keep at most ``HELD_BYTES`` of device workspace, and a plan above that is
+dropped after its call.  A per-entry lock serialises rebind + upload + launch
 of one plan; launches of one plan stay ordered because the stream is part of
 the key.
 """
@@ -35,15 +40,26 @@ _LOCK = threading.Lock()
 _CACHE = collections.OrderedDict()
 _CAPACITY = 8
 _GENERATION = [0]
+HELD_BYTES = 1 << 30
 
 
 def set_capacity(n):
-    """Keep at most ``n`` plans (0 disables reuse and empties the cache)."""
+    """Keep at most ``n`` plans of each group (0 disables reuse and empties the cache)."""
     global _CAPACITY
     with _LOCK:
         _CAPACITY = max(0, int(n))
-        while len(_CACHE) > _CAPACITY:
-            _CACHE.popitem(last=False)
+        _evict(False)
+        _evict(True)
+
+
+def _evict(bounded):
+    """Drop a group's oldest entries until it is within its limits (under _LOCK)."""
+    mine = [k for k, e in _CACHE.items() if e.bounded == bounded]
+    held = sum(_CACHE[k].nbytes for k in mine)
+    for count, k in zip(range(len(mine), 0, -1), mine):
+        if count <= _CAPACITY and held <= HELD_BYTES:
+            break
+        held -= _CACHE.pop(k).nbytes
 
 
 def clear():
@@ -124,16 +140,19 @@ def digest(*string_tensors):
 
 
 class _Entry:
-    __slots__ = ("plan", "lock")
+    __slots__ = ("plan", "lock", "bounded", "nbytes")
 
-    def __init__(self, plan):
+    def __init__(self, plan, bounded):
         self.plan = plan
         self.lock = threading.Lock()
+        self.bounded = bounded
+        self.nbytes = plan.workspace_bytes if bounded else 0
 
 
-def run(key, build, rebind, launch):
+def run(key, build, rebind, launch, bounded=False):
     """``launch(plan)`` with a cached plan for ``key`` (rebound by
-    ``rebind(plan)``) or a fresh one from ``build()``; returns launch's result."""
+    ``rebind(plan)``) or a fresh one from ``build()``; returns launch's result.
+    ``bounded``: the plan belongs to the group that ``HELD_BYTES`` limits."""
     if _CAPACITY == 0:
         return launch(build())
     key = key + (_GENERATION[0],)
@@ -149,12 +168,13 @@ def run(key, build, rebind, launch):
     st = plan.stats()
     if st["streaming"] or getattr(plan, "noisy", False):
         return launch(plan)
-    entry = _Entry(plan)
+    entry = _Entry(plan, bounded)
+    if entry.nbytes > HELD_BYTES:
+        return launch(plan)
     with entry.lock:
         out = launch(plan)
     with _LOCK:
         _CACHE[key] = entry
         _CACHE.move_to_end(key)
-        while len(_CACHE) > _CAPACITY:
-            _CACHE.popitem(last=False)
+        _evict(bounded)
     return out

@@ -120,15 +120,16 @@ def _run(plan, out_shape, dtype):
 
 
 def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None,
-                stage_new=True):
+                training=False):
     """``launch(plan)`` with the plan of a recent call of ``op`` whose string
     tensors, names and ``extra`` arguments were the same, rebound to ``values``
     and ``seed``, or with ``build()``'s (see ``plan_cache``).
 
-    ``stage_new``: a new plan's symbolic matrices are evaluated on the device as a
-    reused one's are.  The host's differ from those in the last bit of a sine or
-    cosine, enough to move a draw: a seeded call would return other shots the
-    second time, or once its plan has left the cache."""
+    ``training``: an op of a training loop, whose plans are a group of their own
+    in the cache.  A new plan of the others has its symbolic matrices evaluated on
+    the device as a reused one's are.  The host's differ from those in the last bit
+    of a sine or cosine, enough to move a draw: a seeded call would return other
+    shots the second time, or once its plan has left the cache."""
     from . import plan_cache
     if not _torch().cuda.is_available():
         return launch(build())  # the inputs' own errors before the missing device
@@ -138,7 +139,7 @@ def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None,
 
     def new_plan():
         plan = build()
-        if stage_new and values.size and not plan.stats()["streaming"]:
+        if not training and values.size and not plan.stats()["streaming"]:
             plan.stage_values(values)
         return plan
 
@@ -147,7 +148,7 @@ def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None,
         if seed is not None:
             plan.set_seed(seed)
 
-    return plan_cache.run(key, new_plan, rebind, launch)
+    return plan_cache.run(key, new_plan, rebind, launch, bounded=not training)
 
 
 def _plan_args(programs, names, values):
@@ -181,7 +182,7 @@ def tfq_simulate_expectation(programs, symbol_names, symbol_values, pauli_sums):
     shape = (programs.shape[0], pauli_sums.shape[1])
     return _run_cached("expectation", (programs, pauli_sums), names, values,
                        lambda: plan_expectation(programs, names, values, pauli_sums)[0],
-                       lambda plan: _run(plan, shape, _torch().float32), stage_new=False)
+                       lambda plan: _run(plan, shape, _torch().float32), training=True)
 
 
 def tfq_simulate_state(programs, symbol_names, symbol_values):

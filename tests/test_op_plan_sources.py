@@ -12,6 +12,8 @@ from quantum_amd import tfq_simulate_ops as sim
 
 
 class _Plan:
+    workspace_bytes = 256
+
     def __init__(self, streaming=0):
         self.streaming = streaming
         self.staged = []

@@ -97,3 +97,69 @@ def test_streaming_plans_are_not_cached_and_capacity_zero_disables():
         assert n[0] == 4 and len(plan_cache._CACHE) == 0
     finally:
         plan_cache.set_capacity(8)
+
+
+class _Sized(_FakePlan):
+    def __init__(self, nbytes):
+        super().__init__()
+        self.workspace_bytes = nbytes
+
+
+def _runner(built):
+    def run(key, bounded, nbytes=256):
+        def build():
+            built.append(key)
+            return _Sized(nbytes)
+
+        def rebind(p):
+            p.rebinds += 1
+
+        return plan_cache.run((key,), build, rebind, lambda p: p, bounded=bounded)
+
+    return run
+
+
+def test_one_off_calls_leave_a_training_plan_in_place():
+    """Eight sampling calls between two steps, and a loop over five circuits that calls
+    a gradient and a sampling op on each: every gradient plan is built once."""
+    plan_cache.clear()
+    built = []
+    run = _runner(built)
+    try:
+        run("gradient", False)
+        for i in range(8):
+            run(f"one-off {i}", True)
+        run("gradient", False)
+        assert built.count("gradient") == 1
+        plan_cache.clear()
+        del built[:]
+        for _ in range(3):
+            for c in range(5):
+                run(f"gradient {c}", False)
+                run(f"samples {c}", True)
+        assert len(built) == 10
+    finally:
+        plan_cache.clear()
+
+
+def test_held_workspaces_are_bounded():
+    plan_cache.clear()
+    built = []
+    run = _runner(built)
+    limit = plan_cache.HELD_BYTES
+    try:
+        for _ in range(2):
+            run("too large", True, limit + 1)
+        assert built.count("too large") == 2 and len(plan_cache._CACHE) == 0
+        for i in range(3):
+            run(f"state {i}", True, limit // 2)
+        assert sum(e.nbytes for e in plan_cache._CACHE.values()) <= limit
+        assert [k[0] for k in plan_cache._CACHE] == ["state 1", "state 2"]
+        run("state 2", True)
+        run("large gradient", False, 4 * limit)  # not under the limit
+        assert [k[0] for k in plan_cache._CACHE] == ["state 1", "state 2", "large gradient"]
+        plan_cache.set_capacity(1)
+        assert [k[0] for k in plan_cache._CACHE] == ["state 2", "large gradient"]
+    finally:
+        plan_cache.set_capacity(8)
+        plan_cache.clear()

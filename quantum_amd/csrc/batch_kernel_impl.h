@@ -475,7 +475,8 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE, VAR)) void batch_kern
   __shared__ int s_ci;
   constexpr bool kGeneral = VAR == kVariantAny || VAR == kVariantWide;
   __shared__ uint64_t tab[kGeneral ? kTileTable : 1];
-  __shared__ uint32_t win[kDescWindow * kDescWords];
+  alignas(16) __shared__ uint32_t win[kDescWindow * kDescWords];
+  static_assert(__alignof__(win) >= alignof(DevTerm), "the window is read as terms too");
   // The general kernels have no LDS left for partials (two 13-qubit tiles).
   constexpr bool kGradMode = MODE == kModeAdjoint || MODE == kModeInnerProductGrad;
   constexpr bool kRings = VAR == kVariantLds && kGradMode;

@@ -70,7 +70,7 @@ struct PassArgs {
 // two waves per SIMD.
 template <bool TWO, bool CPLX, int ENG>
 __global__ __launch_bounds__(TWO && ENG == 3 ? 2 * kThreads : kThreads,
-                             (TWO && ENG != 3) || ENG == 5 ? 2 : 4) void pass_kernel(PassArgs a) {
+                             (TWO && ENG == 0) || ENG == 5 ? 2 : 4) void pass_kernel(PassArgs a) {
   constexpr int kPacc = TWO ? (CPLX ? 2 : 1) * kMaxPassDerivs : 1;
   extern __shared__ float2 lds[];
   __shared__ double red[kWaves];
@@ -205,19 +205,27 @@ int pass_engine(const LargePlan& p, const DevPass& ps, bool two) {
   if (ps.op_begin >= ps.op_end || p.ops[ps.op_begin].type != kOpRemap) return 0;
   return PassRegBits(ps.L, two ? kTwoStatePass : 5);
 }
+// Two-state passes have three register qubits or none.
+constexpr bool two_state_engines_ok() {
+  for (int L = 0; L <= kMaxTile; ++L)
+    if (PassRegBits(L, kTwoStatePass) != 0 && PassRegBits(L, kTwoStatePass) != 3) return false;
+  return true;
+}
+static_assert(two_state_engines_ok(), "launch_pass has no kernel for such a two-state pass");
+// false: there is no kernel for that engine.
 template <bool TWO, bool CPLX>
-void launch_pass(const PassArgs& a, int eng, int grid, size_t lds, hipStream_t stream) {
-  if (eng == 5) {
-    if constexpr (!TWO)
-      hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 5>), dim3(grid), dim3(kThreads), lds, stream, a);
-  } else if (eng == 4) {
-    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 4>), dim3(grid), dim3(kThreads), lds, stream, a);
-  } else if (eng == 3) {
-    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 3>), dim3(grid), dim3(1 << (a.pass.L - 3)), lds,
-                       stream, a);
-  } else {
-    hipLaunchKernelGGL((pass_kernel<TWO, CPLX, 0>), dim3(grid), dim3(kThreads), lds, stream, a);
+bool launch_pass(const PassArgs& a, int eng, int grid, size_t lds, hipStream_t stream) {
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, a);
+    return true;
+  };
+  if (eng == 0) return launch(pass_kernel<TWO, CPLX, 0>, kThreads);
+  if (eng == 3) return launch(pass_kernel<TWO, CPLX, 3>, 1 << (a.pass.L - 3));
+  if constexpr (!TWO) {
+    if (eng == 4) return launch(pass_kernel<TWO, CPLX, 4>, kThreads);
+    if (eng == 5) return launch(pass_kernel<TWO, CPLX, 5>, kThreads);
   }
+  return false;
 }
 
 // ------------------------------------------------------------------ dense passes
@@ -554,7 +562,6 @@ __global__ __launch_bounds__(kThreads) void finish_expect(const double* __restri
 }
 
 // Serial finishing steps (one thread): avoids host round trips between kernels.
-
 __global__ void finish_sampled(const double* sums, int count, const float* coefs,
                                const int* shots, float ident, float* out) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
@@ -908,6 +915,7 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
   double* bincl = bsum + std::max<size_t>(1, amps_max >> kCdfBlockLog);
   const int grid = p->grid;
   const int64_t nslots = p->mode == kModeInnerProduct ? p->K : p->O;
+  bool launched = true;  // every pass had a kernel
 
   auto run_passes = [&](const PassPlan& pp, int n, float2* dst, bool init_first) {
     bool first = init_first;
@@ -944,7 +952,7 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
       const uint64_t ntiles = uint64_t(1) << (n - ps.L);
       const int g = int(std::min<uint64_t>(ntiles, uint64_t(grid)));
       const size_t lds = (size_t(1) << ps.L) * sizeof(float2);
-      launch_pass<false, false>(a, pass_engine(*p, ps, false), g, lds, stream);
+      launched &= launch_pass<false, false>(a, pass_engine(*p, ps, false), g, lds, stream);
       first = false;
     }
     if (first) {  // no ops at all: still need |0>
@@ -1089,8 +1097,9 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
         const uint64_t ntiles = uint64_t(1) << (n - ps.L);
         const int g = int(std::min<uint64_t>(ntiles, uint64_t(grid)));
         const size_t lds = 2 * (size_t(1) << ps.L) * sizeof(float2);
-        if (cplx) launch_pass<true, true>(a, pass_engine(*p, ps, true), g, lds, stream);
-        else launch_pass<true, false>(a, pass_engine(*p, ps, true), g, lds, stream);
+        const int eng = pass_engine(*p, ps, true);
+        launched &= cplx ? launch_pass<true, true>(a, eng, g, lds, stream)
+                         : launch_pass<true, false>(a, eng, g, lds, stream);
         // Partial slots of a pass are contiguous [s0, s0 + nd) (numbered at planning).
         int s0 = -1, nd = 0;
         for (int i = ps.op_begin; i < ps.op_end; ++i) {
@@ -1190,6 +1199,7 @@ int LargeLaunch(LargePlan* p, void* ws, void* output, hipStream_t stream, char* 
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return Err(err, len, std::string("large-state kernels: ") + hipGetErrorString(e));
+  if (!launched) return Err(err, len, "large-state kernels: no kernel for one of the plan's passes");
   return 0;
 }
 

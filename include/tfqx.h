@@ -231,9 +231,11 @@ int tfqx_plan_rebind_downstream(tfqx_plan* plan, const float* downstream_grads, 
 int tfqx_plan_stage_values(tfqx_plan* plan, const float* symbol_values, char* err,
                            int64_t err_len);
 
-/* New random seed for the sampling and noisy plans (no upload needed; other
- * plans ignore it).  The reference draws a fresh seed per call
- * (tfq_simulate_samples_op.cc:131-140). */
+/* New random seed for the sampling and noisy plans, on the batch kernel and the
+ * streaming path: the seed of the plan's later launches, which need no new upload
+ * (other plans ignore it).  It is an argument of the kernels, so a graph keeps the
+ * seed that its plan had when it was captured: capture again for another one.  The
+ * reference draws a fresh seed per call (tfq_simulate_samples_op.cc:131-140). */
 int tfqx_plan_set_seed(tfqx_plan* plan, uint64_t seed, char* err, int64_t err_len);
 
 /* Fusion decisions of the planner for one program (host only): the fused ops

@@ -250,7 +250,8 @@ class Plan:
                                                err, 4096), err)
 
     def set_seed(self, seed):
-        """New random seed for a sampling or noisy plan."""
+        """New random seed for later launches of a sampling or noisy plan (graphs
+        captured before keep theirs)."""
         err = ctypes.create_string_buffer(4096)
         check(self._lib.tfqx_plan_set_seed(self.handle, seed, err, 4096), err)
 

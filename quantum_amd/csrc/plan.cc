@@ -367,25 +367,17 @@ void AnnotateEngine(std::vector<DevOp>* ops, size_t begin, int L, int R) {
       o.code = uint8_t(slot_of(o.q[0]) | (o.k > 1 ? slot_of(o.q[1]) : R) << 3);
       continue;
     }
-    int a = slot_of(o.q[0]);
-    if (o.type == kOpChannel) {
+    const int a = slot_of(o.q[0]);
+    if (o.k == 1) {
       o.code = uint8_t(a);
       continue;
     }
-    int b;
-    bool swap;
-    if (o.k > 1) {
-      b = slot_of(o.q[1]);
-      swap = a > b;
-    } else {
-      swap = a != 0;
-      b = a == 0 ? 1 : 0;
-    }
+    const int b = slot_of(o.q[1]);
     const int lo = std::min(a, b), hi = std::max(a, b);
-    o.code = uint8_t((lo * (2 * R - lo - 1) / 2 + (hi - lo - 1)) | (swap ? kCodeSwap : 0));
-    std::vector<int> next{slots[size_t(lo)], slots[size_t(hi)]};
+    o.code = uint8_t((lo * (2 * R - lo - 1) / 2 + (hi - lo - 1)) | (a > b ? kCodeSwap : 0));
+    std::vector<int> next{slots[size_t(a)], slots[size_t(b)]};
     for (int j = 0; j < R; ++j)
-      if (j != lo && j != hi) next.push_back(slots[size_t(j)]);
+      if (j != a && j != b) next.push_back(slots[size_t(j)]);
     slots.swap(next);
   }
   (*ops)[begin].dmat[1] = pack();

@@ -119,10 +119,10 @@ void InsertRemapsR(std::vector<DevOp>* ops, size_t begin, int L, int R);
 //             wavefront index moves.  The first remap's dmat[1]: the slots at the end.
 //   others    q[2], q[3]: controls among the slots and their values
 //   diagonal  code: slot of q[0] | slot of q[1] << 3 (R: a thread bit, or no target)
-//   channel   code: slot of q[0]
-//   dense,    code: number of the slot pair, in order, and kCodeSwap.  A one-qubit
-//   param     op takes slot 0, or slots 0 and its own, along.
-// A dense or parameterised op leaves its pair in slots 0 and 1, the others after it.
+//   channel, one qubit    code: slot of q[0]
+//   dense, param          code: number of the slot pair, in order, and kCodeSwap when
+//                         q[0]'s slot is the second.  It leaves its targets in slots 0 and
+//                         1, the others after it; a one-qubit op leaves all where they are.
 void AnnotateEngine(std::vector<DevOp>* ops, size_t begin, int L, int R);
 
 // Planner tuning (process-wide; 0 = default): register engine on/off and the

@@ -19,6 +19,12 @@
 // permutes the slots instead of moving registers, and goes from one set of
 // registers to another, so the op loop has two halves, one per set.  (In place,
 // with fixed slots, every op ended in 64 register moves beside its 64 MFMAs.)
+// Each ordered pair of slots has a code path of its own: the targets are always
+// taken in the order of the op's matrix, so the rounding of a state (and of the
+// draws from it) does not depend on the slots, and the matrix rows need no
+// rearranging.  (One path per unordered pair, rows exchanged: 5% more for a
+// two-state pass, 0.7% less for a batch of 4-16-qubit gradients, whose kernel
+// holds every engine and feels the code size.)
 // The planner knows the slots at every op and stores in each descriptor which
 // code path it takes (AnnotateEngine), so the device decodes nothing.
 //
@@ -47,10 +53,15 @@ static_assert(kThreads == (1 << kRegThreadBits), "register engine assumes 512 th
 struct cf {
   float x, y;
 };
+// a * b.  FIXED: with the rounding written out.  Which product an fma takes in is up to
+// the compiler otherwise, and may differ from one place to the next, which draws from a
+// forward run's state must not; a reverse sweep is 3% faster with its choice.
+template <bool FIXED>
 __device__ __forceinline__ cf cmulr(cf a, cf b) {
+  if constexpr (FIXED)
+    return cf{__builtin_fmaf(a.x, b.x, -(a.y * b.y)), __builtin_fmaf(a.x, b.y, a.y * b.x)};
   return cf{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
-__device__ __forceinline__ cf caddr(cf a, cf b) { return cf{a.x + b.x, a.y + b.y}; }
 // acc + u * v as four FMAs.
 __device__ __forceinline__ cf cmac(cf acc, cf u, cf v) {
   acc.x = __builtin_fmaf(u.x, v.x, acc.x);
@@ -189,54 +200,27 @@ __device__ __forceinline__ void reg_store(const Regs<R>& a, float2* __restrict__
 }
 
 // ------------------------------------------------------------------ dense ops
-// A operands of an op's matrix.  sw: the group index has the op's two index
-// bits exchanged (the planner gives targets to slots in either order).  A
-// one-qubit matrix acts on group bit t, the identity on the other.
+// A operands of a two-qubit op's matrix (or its adjoint).
 template <bool DAG>
-__device__ __forceinline__ void engine_rows(const float2* __restrict__ M, const DevOp& op,
-                                            MfmaRows& r) {
-  const uint32_t code = op.code;
-  uint32_t l = threadIdx.x & 3u;
-  asm volatile("" : "+v"(l));  // not kept in registers from op to op
-  if (op.k == 1) {
-    const int t = (code & kCodeSwap) ? 1 : 0;
-    const int row = int(l);
-    const int rt = (row >> t) & 1, ro = (row >> (1 - t)) & 1;
-    cf m[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      m[c] = ldm(M, DAG ? c * 2 + rt : rt * 2 + c);
-      if (DAG) m[c].y = -m[c].y;
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const bool same = ((k >> (1 - t)) & 1) == ro;
-      const cf v = ((k >> t) & 1) ? m[1] : m[0];
-      r.gr[k] = same ? v.x : 0.f;
-      r.gi[k] = same ? v.y : 0.f;
-      r.ngi[k] = -r.gi[k];
-    }
-    return;
-  }
-  const bool sw = (code & kCodeSwap) != 0;
-  const uint32_t row = sw ? ((l & 1u) << 1 | l >> 1) : l;
-  const int k1 = sw ? 2 : 1;
+__device__ __forceinline__ void engine_rows(const float2* __restrict__ M, MfmaRows& r) {
+  uint32_t row = threadIdx.x & 3u;
+  asm volatile("" : "+v"(row));  // not kept in registers from op to op
   const float2* base = M + (DAG ? row : row * 4u);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int c = k == 1 ? k1 : k == 2 ? 3 - k1 : k;
-    // (G^dag)[row][c] = conj(G[c][row]).
-    const cf v = ldm(base, DAG ? c * 4 : c);
+    // (G^dag)[row][k] = conj(G[k][row]).
+    const cf v = ldm(base, DAG ? k * 4 : k);
     r.gr[k] = v.x;
     r.gi[k] = DAG ? -v.y : v.y;
     r.ngi[k] = -r.gi[k];
   }
 }
 
-// Group g of slots (SA, SB): the register indices of its four amplitudes.
+// Group g of slots (SA, SB), the op's two targets in its own order: the register
+// indices of its four amplitudes.
 template <int SA, int SB>
 __device__ __forceinline__ void group_idx(int g, int (&idx)[4]) {
-  const int i0 = ins0(ins0(g, SA), SB);
+  const int i0 = ins0(ins0(g, SA < SB ? SA : SB), SA < SB ? SB : SA);
 #pragma unroll
   for (int s = 0; s < 4; ++s) idx[s] = i0 | ((s & 1) << SA) | ((s >> 1) << SB);
 }
@@ -311,6 +295,55 @@ __device__ __forceinline__ void reg_deriv(const Regs<R>& u, const Regs<R>& lam, 
   }
 }
 
+// One-qubit op on slot S: the slots stay.  FMAs on pairs, as many cycles as MFMAs on
+// groups with the identity on another slot, which would take zero times that slot's other
+// amplitudes into each sum (NaN where they are not finite).
+template <int R, int S, bool REV>
+__device__ __forceinline__ void reg_dense1(const Regs<R>& in, Regs<R>& out, const cf (&m)[4],
+                                           const DevOp& op, bool ok) {
+#pragma unroll
+  for (int g = 0; g < (1 << (R - 1)); ++g) {
+    const int i0 = ins0(g, S), i1 = i0 | (1 << S);
+    const cf x0 = in.get(i0), x1 = in.get(i1);
+    out.set(i0, cmac(cmulr<!REV>(m[0], x0), m[1], x1));
+    out.set(i1, cmac(cmulr<!REV>(m[2], x0), m[3], x1));
+  }
+  if (op.cmask) {
+#pragma unroll
+    for (int i = 0; i < (1 << R); ++i)
+      if (!ctrl_ok(op, ok, i)) out.set(i, in.get(i));
+  }
+}
+template <int R, int S, bool CTRL>
+__device__ __forceinline__ void reg_deriv1(const Regs<R>& u, const Regs<R>& lam, const cf (&m)[4],
+                                           const DevOp& op, bool ok, float& part, float& part_im) {
+  part = part_im = 0.f;
+#pragma unroll
+  for (int g = 0; g < (1 << (R - 1)); ++g) {
+    const int i0 = ins0(g, S), i1 = i0 | (1 << S);
+    const cf u0 = u.get(i0), u1 = u.get(i1);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      cf d = cmac(cmulr<false>(m[2 * r], u0), m[2 * r + 1], u1);
+      const int i = r ? i1 : i0;
+      const cf l = lam.get(i);
+      if (CTRL && !ctrl_ok(op, ok, i)) d = cf{0.f, 0.f};
+      part = __builtin_fmaf(d.x, l.x, part);
+      part = __builtin_fmaf(d.y, l.y, part);
+      part_im = __builtin_fmaf(d.x, l.y, part_im);
+      part_im = __builtin_fmaf(-d.y, l.x, part_im);
+    }
+  }
+}
+template <bool DAG>
+__device__ __forceinline__ void one_qubit_matrix(const float2* __restrict__ M, cf (&m)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m[i] = ldm(M, DAG ? (i & 1) * 2 + (i >> 1) : i);
+    if (DAG) m[i] = cconj(m[i]);
+  }
+}
+
 // f(SA, SB as constants) for slot pair number `pair` ((0,1), (0,2), .. in order).
 // The last one is not compared: a path on which nothing ran would keep the
 // result registers' old values alive through the op.
@@ -331,6 +364,14 @@ __device__ __forceinline__ void for_pair(int pair, F&& f) {
     }
   }
 }
+// The same in the order of a two-qubit op's targets: its products are then summed in the
+// order of its matrix whatever slots they are in.
+template <int R, typename F>
+__device__ __forceinline__ void for_ordered_pair(uint32_t code, F&& f) {
+  const int pair = int(code & kCodePair);
+  if (code & kCodeSwap) for_pair<R>(pair, [&](auto SA, auto SB) { f(SB, SA); });
+  else for_pair<R>(pair, f);
+}
 template <int R, int S = 0, typename F>
 __device__ __forceinline__ void for_slot(int slot, F&& f) {
   if constexpr (S + 1 == R) {
@@ -348,8 +389,8 @@ __device__ __forceinline__ void for_slot(int slot, F&& f) {
 template <int R, bool BOTH>
 __device__ __forceinline__ void scale_reg(const Regs<R>& a, const Regs<R>& b, Regs<R>& oa,
                                           Regs<R>& ob, int i, cf e) {
-  oa.set(i, cmulr(e, a.get(i)));
-  if (BOTH) ob.set(i, cmulr(e, b.get(i)));
+  oa.set(i, cmulr<!BOTH>(e, a.get(i)));
+  if (BOTH) ob.set(i, cmulr<!BOTH>(e, b.get(i)));
 }
 __device__ __forceinline__ cf pick(bool c, cf x, cf y) { return cf{c ? x.x : y.x, c ? x.y : y.y}; }
 
@@ -476,7 +517,7 @@ struct ChannelPick {
 // This lane's part of |x0|^2 and |x1|^2 summed over register slot J's qubit.  Every
 // product is added to a sum that starts from a value the compiler does not know: it
 // would compute the sums of all slots before looking at the op, for every op (2.2x
-// this kernel's FP32 instructions).
+// this kernel's FP32 instructions).  The rounding is written out: draws depend on it.
 template <int R, int J>
 __device__ __forceinline__ void reg_density(const Regs<R>& a, float (&d)[2]) {
 #pragma unroll
@@ -488,8 +529,8 @@ __device__ __forceinline__ void reg_density(const Regs<R>& a, float (&d)[2]) {
   for (int g = 0; g < (1 << (R - 1)); ++g) {
     const int i0 = ins0(g, J);
     const cf x0 = a.get(i0), x1 = a.get(i0 | (1 << J));
-    d[0] = __builtin_fmaf(x0.y, x0.y, __builtin_fmaf(x0.x, x0.x, d[0]));
-    d[1] = __builtin_fmaf(x1.y, x1.y, __builtin_fmaf(x1.x, x1.x, d[1]));
+    d[0] += __builtin_fmaf(x0.x, x0.x, x0.y * x0.y);
+    d[1] += __builtin_fmaf(x1.x, x1.x, x1.y * x1.y);
   }
 }
 // The first k with u < p_0 + ... + p_k, the last k with p_k > 0 when none.
@@ -542,7 +583,7 @@ __device__ __forceinline__ ChannelPick channel_pick(const Regs<R>& a, const DevO
 
 // out = the picked operator on register slot J of in; the matrix is read per lane.
 // Bound by the number of VALU instructions: with real matrices half the products
-// go (every channel that is no unitary mixture has them): 688 us (965 us) for 32 rows of
+// go (every channel that is no unitary mixture has them): 700 us (965 us) for 32 rows of
 // 1000 8-qubit trajectories with 128 channels.
 template <int R, int J, bool REAL>
 __device__ __forceinline__ void reg_channel(const Regs<R>& in, Regs<R>& out,
@@ -559,8 +600,8 @@ __device__ __forceinline__ void reg_channel(const Regs<R>& in, Regs<R>& out,
       out.set(i0 | (1 << J), cf{__builtin_fmaf(m11.x, x1.x, m10.x * x0.x),
                                 __builtin_fmaf(m11.x, x1.y, m10.x * x0.y)});
     } else {
-      out.set(i0, cmac(cmulr(m00, x0), m01, x1));
-      out.set(i0 | (1 << J), cmac(cmulr(m10, x0), m11, x1));
+      out.set(i0, cmac(cmulr<true>(m00, x0), m01, x1));
+      out.set(i0 | (1 << J), cmac(cmulr<true>(m10, x0), m11, x1));
     }
   }
 }
@@ -804,32 +845,54 @@ __device__ __forceinline__ void run_op(const Regs<R>& ra, const Regs<R>& rb, Reg
       return;
     }
   }
-  MfmaRows m;
-  engine_rows<REV>(mats + op.mat, op, m);
-  const int pair = int(op.code & kCodePair);
   const int nd = REV && op.type == kOpParam ? op.nderiv : 0;
   float part[2 * kMaxDeriv] = {0.f, 0.f, 0.f, 0.f};
-  for_pair<R>(pair, [&](auto SA, auto SB) {
-    reg_dense<R, SA.value, SB.value>(ra, oa, m, op, ok);
-    if (REV) {
-      reg_dense<R, SA.value, SB.value>(rb, ob, m, op, ok);
+  auto keep = [&](int d, float re, float im) {
+    if (d == 0) {
+      part[0] = re;
+      part[kMaxDeriv] = im;
+    } else {
+      part[1] = re;
+      part[kMaxDeriv + 1] = im;
+    }
+  };
+  if (op.k == 1) {
+    cf m[4];
+    one_qubit_matrix<REV>(mats + op.mat, m);
+    for_slot<R>(int(op.code), [&](auto S) {
+      reg_dense1<R, S.value, REV>(ra, oa, m, op, ok);
+      if (REV) {
+        reg_dense1<R, S.value, REV>(rb, ob, m, op, ok);
 #pragma unroll 1
-      for (int d = 0; d < nd; ++d) {
-        MfmaRows dm;
-        engine_rows<false>(mats + (d == 0 ? op.dmat[0] : op.dmat[1]), op, dm);
-        float re, im;
-        if (op.cmask) reg_deriv<R, SA.value, SB.value, true>(oa, rb, dm, op, ok, re, im);
-        else reg_deriv<R, SA.value, SB.value, false>(oa, rb, dm, op, ok, re, im);
-        if (d == 0) {
-          part[0] = re;
-          part[kMaxDeriv] = im;
-        } else {
-          part[1] = re;
-          part[kMaxDeriv + 1] = im;
+        for (int d = 0; d < nd; ++d) {
+          cf dm[4];
+          one_qubit_matrix<false>(mats + (d == 0 ? op.dmat[0] : op.dmat[1]), dm);
+          float re, im;
+          if (op.cmask) reg_deriv1<R, S.value, true>(oa, rb, dm, op, ok, re, im);
+          else reg_deriv1<R, S.value, false>(oa, rb, dm, op, ok, re, im);
+          keep(d, re, im);
         }
       }
-    }
-  });
+    });
+  } else {
+    MfmaRows m;
+    engine_rows<REV>(mats + op.mat, m);
+    for_ordered_pair<R>(op.code, [&](auto SA, auto SB) {
+      reg_dense<R, SA.value, SB.value>(ra, oa, m, op, ok);
+      if (REV) {
+        reg_dense<R, SA.value, SB.value>(rb, ob, m, op, ok);
+#pragma unroll 1
+        for (int d = 0; d < nd; ++d) {
+          MfmaRows dm;
+          engine_rows<false>(mats + (d == 0 ? op.dmat[0] : op.dmat[1]), dm);
+          float re, im;
+          if (op.cmask) reg_deriv<R, SA.value, SB.value, true>(oa, rb, dm, op, ok, re, im);
+          else reg_deriv<R, SA.value, SB.value, false>(oa, rb, dm, op, ok, re, im);
+          keep(d, re, im);
+        }
+      }
+    });
+  }
   if (nd > 0) {
     // Wave mode: gradient partials count each amplitude once (replica lanes 0).
     if (WAVE && ((threadIdx.x & 63u) >> (L - R)) != 0u)

@@ -78,7 +78,7 @@ constexpr int kWaveMinCircuits = 1024;
 
 // DevOp::code bits (register engine).
 constexpr int kCodePair = 15;   // slot pair of the group
-constexpr int kCodeSwap = 16;   // two qubits: index bits exchanged; one: group bit 1
+constexpr int kCodeSwap = 16;   // q[0] is in the pair's second slot
 constexpr int kCodeLocal = 1;   // remap within wavefronts
 
 // One op on a tile.  Qubit positions are tile-local bit indices (ascending).

@@ -344,8 +344,9 @@ __device__ __forceinline__ void wave_circuit(const BatchArgs& a, int ci, float2*
 }
 
 // Tiled forward: the state lives in global memory G; each pass streams its
-// tiles through LDS buffer A.  The first pass starts from |0>.
-template <int VAR, int RMAX = 4>
+// tiles through LDS buffer A.  The first pass starts from |0>.  RMAX: largest
+// register count of the register engine's tile I/O (reg_run_any), 0 for none.
+template <int VAR, int RMAX>
 __device__ __forceinline__ void tiled_forward(float2* G, int n, const BatchArgs& a, int pb, int pe, float2* A,
                               uint64_t* tab, MatCache& mc, uint32_t* win) {
   const int tid = threadIdx.x;
@@ -362,26 +363,28 @@ __device__ __forceinline__ void tiled_forward(float2* G, int n, const BatchArgs&
       auto gidx = [&](uint32_t j) -> uint64_t {
         return use_tab ? tile_index_tab(base, j, ps.nlow, tab) : tile_index(base, j, ps);
       };
-      // Register engine: the tile goes straight between G and the registers.
-      auto io = tile_io_indexed(
-          [&](uint32_t j) -> uint64_t {
-            return use_tab ? tile_index_tab(0, j, ps.nlow, tab) : tile_index(0, j, ps);
-          },
-          [&](uint64_t th, const auto& slot, auto&& set_a, auto&&) {
-            const uint64_t x = base | th;
-            if (first)
-              each_reg(slot, x, [&](int r, uint64_t y) { set_a(r, cf{y == 0 ? 1.f : 0.f, 0.f}); });
-            else
-              each_reg(slot, G + x, [&](int r, const float2* p) { set_a(r, cf{p->x, p->y}); });
-          },
-          [&](uint64_t th, const auto& slot, auto&& get_a, auto&&) {
-            each_reg(slot, G + (base | th), [&](int r, float2* p) {
-              const cf v = get_a(r);
-              *p = make_float2(v.x, v.y);
+      if constexpr (RMAX > 0) {
+        // Register engine: the tile goes straight between G and the registers.
+        auto io = tile_io_indexed(
+            [&](uint32_t j) -> uint64_t {
+              return use_tab ? tile_index_tab(0, j, ps.nlow, tab) : tile_index(0, j, ps);
+            },
+            [&](uint64_t th, const auto& slot, auto&& set_a, auto&&) {
+              const uint64_t x = base | th;
+              if (first)
+                each_reg(slot, x, [&](int r, uint64_t y) { set_a(r, cf{y == 0 ? 1.f : 0.f, 0.f}); });
+              else
+                each_reg(slot, G + x, [&](int r, const float2* p) { set_a(r, cf{p->x, p->y}); });
+            },
+            [&](uint64_t th, const auto& slot, auto&& get_a, auto&&) {
+              each_reg(slot, G + (base | th), [&](int r, float2* p) {
+                const cf v = get_a(r);
+                *p = make_float2(v.x, v.y);
+              });
             });
-          });
-      if (reg_run_any<false, RMAX>(A, A, ps.L, a.ops, ps.op_begin, ps.op_end, mc, NoAcc(), io))
-        continue;
+        if (reg_run_any<false, RMAX>(A, A, ps.L, a.ops, ps.op_begin, ps.op_end, mc, NoAcc(), io))
+          continue;
+      }
       if (first) {
         for (uint32_t j = tid; j < T; j += kThreads) A[j] = make_float2(gidx(j) == 0 ? 1.f : 0.f, 0.f);
       } else {
@@ -554,8 +557,9 @@ __global__ __launch_bounds__(kThreads, BatchMinWaves(MODE, VAR)) void batch_kern
     } else if constexpr (kGeneral) {
       // The adjoint's forward carries one state: its passes may use 14-qubit
       // tiles (the LDS of the two 13-qubit reverse tiles) and five register
-      // qubits.
-      tiled_forward<VAR, MODE == kModeAdjoint ? 5 : 4>(gpsi, n, a, uniform(c.fwd_pass_begin),
+      // qubits.  The other modes' tiles have 14 qubits and run on the LDS engine;
+      // without the register engine's tile I/O their kernels spill less.
+      tiled_forward<VAR, MODE == kModeAdjoint ? 5 : 0>(gpsi, n, a, uniform(c.fwd_pass_begin),
                                                        uniform(c.fwd_pass_end), psi, tab, mc, win);
     }
 

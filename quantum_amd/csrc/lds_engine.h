@@ -66,49 +66,56 @@ __device__ __forceinline__ DevOp desc_unpack(uint32_t word) {
   return o;
 }
 
-// (dr, di) = G v for a lane's group v of a two-qubit op, its products added in the
-// order of apply_dense (lds_ops.h): column 0 as cmul contracts it (the product that is
-// rounded by itself first; another one in the adjoint, where the imaginary part is a
-// difference), the others as cmacf.  So amplitudes have the bits that the FMA path gives
-// them, and a shot, drawn by comparing a prefix sum with a uniform, the same outcome.
-template <bool DAG>
-__device__ __forceinline__ void ordered_apply(const float2 (&v)[4], const MfmaRows& m, mf4& dr,
-                                              mf4& di) {
-  const mf4 zero{0.f, 0.f, 0.f, 0.f};
-  dr = mfma4(m.gr[0], v[0].x, mfma4(m.ngi[0], v[0].y, zero));
-  di = DAG ? mfma4(m.gr[0], v[0].y, mfma4(m.gi[0], v[0].x, zero))
-           : mfma4(m.gi[0], v[0].x, mfma4(m.gr[0], v[0].y, zero));
-#pragma unroll
-  for (int k = 1; k < 4; ++k) {
-    dr = mfma4(m.ngi[k], v[k].y, mfma4(m.gr[k], v[k].x, dr));
-    di = mfma4(m.gi[k], v[k].x, mfma4(m.gr[k], v[k].y, di));
-  }
-}
-
-// o = the op's matrix (or its adjoint) times v, the 2^K amplitudes of a lane.  One qubit:
-// FMAs on a pair.  On MFMA a pair would need another one beside it, with zeros between
-// the two: NaN in both where one of them is not finite.
+// A lane's part of an op's matrix (or its adjoint, DAG) and its product with v, the lane's
+// 2^K amplitudes.  Two qubits: MFMA rows.  One qubit: the matrix, for FMAs on a pair; on
+// MFMA a pair would need another one beside it, with zeros between the two: NaN in both
+// where one of them is not finite.
 template <int K, bool DAG>
-__device__ __forceinline__ void lane_apply(const float2* __restrict__ M, const float2 (&v)[1 << K],
-                                           float2 (&o)[1 << K]) {
-  if constexpr (K == 2) {
-    MfmaRows G;
-    mfma_rows<DAG>(M, G);
-    mf4 dr, di;
-    ordered_apply<DAG>(v, G, dr, di);
+struct LaneMatrix;
+
+// The products of a two-qubit op are added in the order of apply_dense (lds_ops.h):
+// column 0 as cmul contracts it (the product that is rounded by itself first; another one
+// in the adjoint, where the imaginary part is a difference), the others as cmacf.  So
+// amplitudes have the bits that the FMA path gives them, and a shot, drawn by comparing a
+// prefix sum with a uniform, the same outcome.
+template <bool DAG>
+struct LaneMatrix<2, DAG> {
+  MfmaRows m;
+  __device__ __forceinline__ explicit LaneMatrix(const float2* __restrict__ M) {
+    mfma_rows<DAG>(M, m);
+  }
+  __device__ __forceinline__ void apply(const float2 (&v)[4], float2 (&o)[4]) const {
+    const mf4 zero{0.f, 0.f, 0.f, 0.f};
+    mf4 dr = mfma4(m.ngi[0], v[0].y, zero);
+    mf4 di = DAG ? mfma4(m.gi[0], v[0].x, zero) : mfma4(m.gr[0], v[0].y, zero);
+    dr = mfma4(m.gr[0], v[0].x, dr);
+    di = DAG ? mfma4(m.gr[0], v[0].y, di) : mfma4(m.gi[0], v[0].x, di);
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+      dr = mfma4(m.gr[k], v[k].x, dr);
+      di = mfma4(m.gr[k], v[k].y, di);
+      dr = mfma4(m.ngi[k], v[k].y, dr);
+      di = mfma4(m.gi[k], v[k].x, di);
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s) o[s] = make_float2(dr[s], di[s]);
-  } else {
-    float2 m[4];
+  }
+};
+template <bool DAG>
+struct LaneMatrix<1, DAG> {
+  float2 m[4];
+  __device__ __forceinline__ explicit LaneMatrix(const float2* __restrict__ M) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       m[i] = M[DAG ? (i & 1) * 2 + (i >> 1) : i];
       if (DAG) m[i].y = -m[i].y;
     }
+  }
+  __device__ __forceinline__ void apply(const float2 (&v)[2], float2 (&o)[2]) const {
     o[0] = cmacf(cmul(m[0], v[0]), m[1], v[1]);
     o[1] = cmacf(cmul(m[2], v[0]), m[3], v[1]);
   }
-}
+};
 
 // As cache_span, by one wavefront.
 __device__ __forceinline__ void cache_span_solo(MatCache& c, uint32_t off, uint32_t len) {
@@ -177,6 +184,7 @@ __device__ __forceinline__ void lds_dense(float2* __restrict__ A, float2* __rest
     }
     if (lane < uint32_t(need)) ring->col[parts + int(lane)] = nd > 1 && (lane & 1u) ? op.col[1] : op.col[0];
   }
+  const LaneMatrix<K, REV> G(M);
   // Every lane runs every round: MFMA takes its operands from all lanes.
   // Lanes past the last repeat one (and store the same values).
   for (uint32_t g0 = first; g0 < count; g0 += kStep) {
@@ -191,23 +199,29 @@ __device__ __forceinline__ void lds_dense(float2* __restrict__ A, float2* __rest
 #pragma unroll
       for (int s = 0; s < D; ++s) l[s] = B[x0 | dep[s]];
     }
-    lane_apply<K, REV>(M, a, u);
-    if constexpr (REV) lane_apply<K, REV>(M, l, w);
-    if (ok) {
+    // All loads are under way before the first product: in the kernels that are short of
+    // registers the compiler loads one amplitude after the other (a 16-qubit state in
+    // 14-qubit tiles: 1357 us, with the barrier 1216).
+    __builtin_amdgcn_sched_barrier(0);
+    G.apply(a, u);
+    if constexpr (REV) G.apply(l, w);
+    auto store = [&]() {
 #pragma unroll
       for (int s = 0; s < D; ++s) A[x0 | dep[s]] = u[s];
       if constexpr (REV) {
 #pragma unroll
         for (int s = 0; s < D; ++s) B[x0 | dep[s]] = w[s];
       }
-    }
+    };
+    if (op.cmask == 0u) store();
+    else if (ok) store();
     if constexpr (REV) {
       if (nd > 0) {
 #pragma unroll
         for (int d = 0; d < kMaxDeriv; ++d) {
           if (d >= nd) break;
           float2 t[D];
-          lane_apply<K, false>(M + D * D * (1 + d), u, t);
+          LaneMatrix<K, false>(M + D * D * (1 + d)).apply(u, t);
           float part = 0.f, part_im = 0.f;
 #pragma unroll
           for (int s = 0; s < D; ++s) {

@@ -130,7 +130,8 @@ __device__ __forceinline__ uint32_t sample_one(const float2* __restrict__ s, uin
 }
 
 // ------------------------------------------------------------------ workgroup trajectories
-// One channel on an LDS state (all threads; selection rule as reg_channel_j).
+// One channel on an LDS state (all threads; selection rule as channel_pick, with the
+// coherences that no channel kind has a use for: E_k is diagonal).
 __device__ __forceinline__ void lds_channel(float2* s, int n, const DevOp& op, const float2* mats,
                                             double u, double* red) {
   const int nk = ChanKraus(op.cval);

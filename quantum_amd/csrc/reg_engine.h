@@ -1,8 +1,8 @@
 // Register-resident gate engine for a 2^L-amplitude state tile held in LDS.
 //
-// A workgroup of 512 threads keeps the tile in VGPRs: each thread holds 2^R
-// amplitudes (R = L - 9, 3..5) whose indices differ only in R "register
-// qubits"; the thread index fills the other L - R bits.  Ops whose targets
+// A workgroup of 512 threads keeps the tile in VGPRs (13-qubit tiles of two states:
+// 1024 threads): each thread holds 2^R amplitudes (R = L - 9, or 10 there; 3..5) whose
+// indices differ only in R "register qubits"; the thread index fills the other L - R bits.  Ops whose targets
 // are register qubits (and diagonal ops on any qubits, with controls on any
 // qubits) are applied in registers with no LDS traffic and no barrier.  The
 // host planner splits the op list into segments whose non-diagonal targets
@@ -46,7 +46,7 @@
 namespace tfqx {
 namespace {
 
-static_assert(kThreads == (1 << kRegThreadBits), "register engine assumes 512 threads");
+static_assert(kThreads == (1 << kRegThreadBits), "RegBitsForTile assumes 512 threads");
 
 // Register-resident complex amplitude.  A plain two-float struct (not the HIP
 // vector type, whose union members turn register arrays into scratch memory).

@@ -41,8 +41,9 @@ constexpr int ChanKraus(uint32_t cval) { return int(cval & 15u); }
 
 // Register engine (reg_engine.h): 2^9 threads per workgroup, each holding
 // 2^R amplitudes of a 2^L tile in registers, R = L - 9 for tiles of 12..13
-// qubits; other tile sizes use the LDS path.  The planner inserts kOpRemap
-// ops exactly when this returns nonzero and every op of the list has k <= 2.
+// qubits (two-state streaming passes: PassRegBits); other tile sizes use the LDS
+// path.  The planner inserts kOpRemap ops exactly when RegBitsForTile or PassRegBits
+// returns nonzero and every op of the list has k <= 2.
 constexpr int kRegThreadBits = 9;
 
 // The register engine reads op matrices from an LDS window of this many
@@ -62,7 +63,8 @@ constexpr int RegBitsForTile(int L, int max_r = 4) {
 // Register qubits of a pass: two-state streaming passes (max_r = kTwoStatePass) on
 // 13-qubit tiles take three, the tile's other ten qubits on 1024 threads.  Their
 // LDS lets one workgroup on a CU, and sixteen wavefronts hide more latency there than
-// eight: 518 us a pass of 24 qubits (533 us with four register qubits).
+// eight: 518 us a pass of 24 qubits against 533 with four register qubits, when that was
+// chosen (465 us now).
 constexpr int kTwoStatePass = -1;
 constexpr int PassRegBits(int L, int max_r) {
   return max_r != kTwoStatePass ? RegBitsForTile(L, max_r) : L == 13 ? 3 : RegBitsForTile(L);

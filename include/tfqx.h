@@ -320,6 +320,10 @@ int tfqx_ps_weights_from_symbols(const uint8_t* programs, const int64_t* program
  * expected algorithmic real flops of one launch.  No reference counterpart. */
 int tfqx_plan_stats(const tfqx_plan* plan, int64_t* out, int64_t n);
 
+/* 1 for a plan on the HBM-streaming path (tfqx_plan_stats' [6], without the
+ * counting). */
+int tfqx_plan_streaming(const tfqx_plan* plan);
+
 /* Largest qubit count in the batch (sizes the samples / state outputs). */
 int64_t tfqx_plan_max_num_qubits(const tfqx_plan* plan);
 /* Device workspace the plan needs (bytes). */

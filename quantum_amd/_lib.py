@@ -84,6 +84,8 @@ def _declare(lib):
     lib.tfqx_plan_set_seed.restype = c.c_int
     lib.tfqx_plan_upload_changed.argtypes = [P, P, P, c.c_char_p, i64]
     lib.tfqx_plan_upload_changed.restype = c.c_int
+    lib.tfqx_plan_streaming.argtypes = [P]
+    lib.tfqx_plan_streaming.restype = c.c_int
     lib.tfqx_plan_stats.argtypes = [P, P, i64]
     lib.tfqx_plan_stats.restype = c.c_int
     for name in ("tfqx_plan_simulate_expectation", "tfqx_plan_simulate_sampled_expectation",
@@ -156,7 +158,7 @@ EXPORTED_SYMBOLS = (
     "tfqx_plan_rebind_downstream", "tfqx_plan_stage_values", "tfqx_plan_set_seed",
     "tfqx_plan_upload_changed",
     "tfqx_debug_fuse", "tfqx_debug_philox_uniform",
-    "tfqx_plan_stats",
+    "tfqx_plan_stats", "tfqx_plan_streaming",
     "tfqx_plan_max_num_qubits", "tfqx_plan_workspace_bytes",
     "tfqx_plan_output_bytes", "tfqx_plan_upload", "tfqx_plan_launch", "tfqx_plan_launch_plain",
     "tfqx_plan_launch_noalloc",
@@ -214,6 +216,10 @@ class Plan:
     @property
     def max_num_qubits(self):
         return int(self._lib.tfqx_plan_max_num_qubits(self.handle))
+
+    @property
+    def streaming(self):
+        return bool(self._lib.tfqx_plan_streaming(self.handle))
 
     def stats(self):
         out = (ctypes.c_int64 * 10)()

@@ -1015,6 +1015,8 @@ int tfqx_plan_rebind_downstream(tfqx_plan* p, const float* downstream, char* err
   return TFQX_OK;
 }
 
+int tfqx_plan_streaming(const tfqx_plan* p) { return p && p->large ? 1 : 0; }
+
 int tfqx_plan_stats(const tfqx_plan* p, int64_t* out, int64_t n) {
   if (!p || !out) return TFQX_INVALID_ARGUMENT;
   int64_t v[24] = {0};

@@ -44,7 +44,7 @@ def _inner_product_raw(programs, names, values, other):
         return Plan(_lib.lib().tfqx_plan_inner_product, *args, Ot.ptr, Ot.off, other.shape[1])
 
     return _run_cached("inner_product", (programs, other), names, values, build,
-                       lambda plan: _run(plan, other.shape, _torch().complex64))
+                       lambda plan, where: _run(plan, other.shape, _torch().complex64, where))
 
 
 def _grad_raw(programs, names, values, other, prev_grad, derivative):

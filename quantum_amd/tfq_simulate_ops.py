@@ -108,9 +108,10 @@ def _common(programs, symbol_names, symbol_values):
     return programs, names, values
 
 
-def _run(plan, out_shape, dtype):
+def _run(plan, out_shape, dtype, where=None):
+    """``where``: the caller's (device, stream), when it has asked for them."""
     torch = _torch()
-    dev, stream = _device_and_stream()
+    dev, stream = where or _device_and_stream()
     out = torch.empty(out_shape, dtype=dtype, device=dev)
     if out.numel() == 0 and plan.workspace_bytes <= 256:
         return out
@@ -121,7 +122,7 @@ def _run(plan, out_shape, dtype):
 
 def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None,
                 training=False):
-    """``launch(plan)`` with the plan of a recent call of ``op`` whose string
+    """``launch(plan, where)`` with the plan of a recent call of ``op`` whose string
     tensors, names and ``extra`` arguments were the same, rebound to ``values``
     and ``seed``, or with ``build()``'s (see ``plan_cache``).
 
@@ -131,15 +132,16 @@ def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None,
     of a sine or cosine, enough to move a draw: a seeded call would return other
     shots the second time, or once its plan has left the cache."""
     from . import plan_cache
-    if not _torch().cuda.is_available():
-        return launch(build())  # the inputs' own errors before the missing device
-    dev, stream = _device_and_stream()
+    try:
+        where = dev, stream = _device_and_stream()
+    except RuntimeError:
+        return launch(build(), None)  # the inputs' own errors before the missing device
     key = (op, plan_cache.digest(*strings), tuple(names), tuple(x.shape for x in strings),
            dev.index, stream, *extra)
 
     def new_plan():
         plan = build()
-        if not training and values.size and not plan.stats()["streaming"]:
+        if not training and values.size and not plan.streaming:
             plan.stage_values(values)
         return plan
 
@@ -148,7 +150,8 @@ def _run_cached(op, strings, names, values, build, launch, extra=(), seed=None,
         if seed is not None:
             plan.set_seed(seed)
 
-    return plan_cache.run(key, new_plan, rebind, launch, bounded=not training)
+    return plan_cache.run(key, new_plan, rebind, lambda plan: launch(plan, where),
+                          bounded=not training)
 
 
 def _plan_args(programs, names, values):
@@ -182,7 +185,7 @@ def tfq_simulate_expectation(programs, symbol_names, symbol_values, pauli_sums):
     shape = (programs.shape[0], pauli_sums.shape[1])
     return _run_cached("expectation", (programs, pauli_sums), names, values,
                        lambda: plan_expectation(programs, names, values, pauli_sums)[0],
-                       lambda plan: _run(plan, shape, _torch().float32), training=True)
+                       lambda plan, where: _run(plan, shape, _torch().float32, where), training=True)
 
 
 def tfq_simulate_state(programs, symbol_names, symbol_values):
@@ -194,8 +197,9 @@ def tfq_simulate_state(programs, symbol_names, symbol_values):
         return Plan(_lib.lib().tfqx_plan_simulate_state, *args)
 
     return _run_cached("state", (programs,), names, values, build,
-                       lambda plan: _run(plan, (programs.shape[0], 2 ** plan.max_num_qubits),
-                                         _torch().complex64))
+                       lambda plan, where: _run(
+                           plan, (programs.shape[0], 2 ** plan.max_num_qubits),
+                           _torch().complex64, where))
 
 
 def _num_samples_scalar(num_samples):
@@ -227,8 +231,9 @@ def tfq_simulate_samples(programs, symbol_names, symbol_values, num_samples, see
         return Plan(_lib.lib().tfqx_plan_simulate_samples, *args, n, seed)
 
     return _run_cached("samples", (programs,), names, values, build,
-                       lambda plan: _run(plan, (programs.shape[0], n, plan.max_num_qubits),
-                                         _torch().int8), extra=(n,), seed=seed)
+                       lambda plan, where: _run(
+                           plan, (programs.shape[0], n, plan.max_num_qubits), _torch().int8, where),
+                       extra=(n,), seed=seed)
 
 
 def tfq_simulate_sampled_expectation(programs, symbol_names, symbol_values, pauli_sums,
@@ -255,7 +260,7 @@ def tfq_simulate_sampled_expectation(programs, symbol_names, symbol_values, paul
                     pauli_sums.shape[1], np_ptr(ns), seed)
 
     return _run_cached("sampled_expectation", (programs, pauli_sums), names, values, build,
-                       lambda plan: _run(plan, pauli_sums.shape, _torch().float32),
+                       lambda plan, where: _run(plan, pauli_sums.shape, _torch().float32, where),
                        extra=(ns.tobytes(),), seed=seed)
 
 

@@ -19,7 +19,7 @@ class _Plan:
         self.staged = []
 
     def stats(self):
-        return {"streaming": self.streaming}
+        raise AssertionError("a call needs one flag, not the counts over all ops")
 
     def stage_values(self, values):
         self.staged.append(values.copy())
@@ -41,7 +41,7 @@ def fake_device(monkeypatch):
 def _call(values, streaming=0, **kw):
     progs = np.array([b"p"] * len(values), dtype=object)
     return sim._run_cached("op", (progs,), ["a"], values, lambda: _Plan(streaming),
-                           lambda plan: plan, **kw)
+                           lambda plan, where: plan, **kw)
 
 
 @pytest.mark.parametrize("capacity", [8, 0])
